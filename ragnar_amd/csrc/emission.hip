@@ -73,25 +73,6 @@ __global__ void __launch_bounds__(64) product_pair_kernel(const double* __restri
   if (static_cast<int>(threadIdx.x) == ks[0]) out[e] = make_float2(best_c, best_s);
 }
 
-// ---------------------------------------------------------------------------
-// Shared inner loop: 64 sources of `src` against the lane's NB bins.
-// ---------------------------------------------------------------------------
-template <int NB>
-__device__ __forceinline__ void eval_sources(const float4* __restrict__ src, int count,
-                                             const float (&c)[NB], const float (&S)[NB],
-                                             const float2* __restrict__ ltab, float (&acc)[NB]) {
-#pragma unroll 4
-  for (int j = 0; j < count; ++j) {
-    const float4 q = src[j];
-#pragma unroll
-    for (int k = 0; k < NB; ++k) {
-      const float u = fmaf(c[k], S[k], q.y) + q.z;
-      const float2 cs = ltab[cvt_sat_u32(u)];
-      acc[k] = fmaf(q.x, fmaf(u, cs.y, cs.x), acc[k]);
-    }
-  }
-}
-
 struct ParticleSourceFn {
   ParticlesDev D;
   using Raw = RawParticle;
@@ -138,6 +119,7 @@ __global__ void __launch_bounds__(kThreads) forward_kernel(SourceFn fn, size_t n
     S[k] = cs.y;
     dacc[k] = 0.0;
   }
+  __syncthreads();  // the table is in LDS; each wave's part of the tile is its own
 
   const size_t stride = static_cast<size_t>(gridDim.x) * kThreads;
   size_t base = static_cast<size_t>(blockIdx.x) * kThreads;
@@ -149,13 +131,15 @@ __global__ void __launch_bounds__(kThreads) forward_kernel(SourceFn fn, size_t n
     if (p < n) s = fn.make(raw, P);
     // the next tile's inputs load while this tile is evaluated
     if (p + stride < n) raw = fn.load(p + stride);
-    __syncthreads();  // the previous tile has been consumed
-    tile[threadIdx.x] = make_float4(s.W, s.vhi, s.vlo, 0.0f);
-    __syncthreads();
+    int count[NB + 1];
+    const int slot = class_slot<NB>(blocks_reached<NB>(s, P), count);
+    wave_lds_fence();  // the wave's previous sources have been read
+    tile[wave * 64 + slot] = make_float4(s.W, s.vhi, s.vlo, 0.0f);
+    wave_lds_fence();
     float acc[NB];
 #pragma unroll
     for (int k = 0; k < NB; ++k) acc[k] = 0.0f;
-    eval_sources<NB>(tile + wave * 64, 64, c, S, ltab, acc);
+    eval_classes<NB, NB>(tile + wave * 64, 0, count, c, S, ltab, acc);
 #pragma unroll
     for (int k = 0; k < NB; ++k) dacc[k] += static_cast<double>(acc[k]);
   }
@@ -228,9 +212,39 @@ __device__ __forceinline__ float group_sum(float v) {
   return v;
 }
 
+// Steps [step, ...) while their first (furthest-reaching) source reaches KB
+// blocks or more: the sums over the KB leading 64-bin blocks, which hold the
+// lane's bins k < KB 64 / LPP.
+template <int LPP, int NBL, int KB, int NBQ>
+__device__ __forceinline__ void adjoint_classes(const float4* __restrict__ src, float2* __restrict__ ac, int step,
+                                                const int (&count)[NBQ + 1], int grp, int li, const float (&c)[NBL],
+                                                const float (&S)[NBL], const float (&g)[NBL],
+                                                const float2* __restrict__ ltab) {
+  constexpr int PPW = 64 / LPP;
+  for (; step * PPW < count[KB]; ++step) {
+    const int j = step * PPW + grp;
+    const float4 q = src[j];
+    float a = 0.0f, cc = 0.0f;
+#pragma unroll
+    for (int k = 0; k < KB * (64 / LPP); ++k) {
+      const float u = fmaf(c[k], S[k], q.y) + q.z;
+      const float2 cs = ltab[cvt_sat_u32(u)];
+      a = fmaf(g[k], fmaf(u, cs.y, cs.x), a);
+      cc = fmaf(g[k], cs.y, cc);
+    }
+    a = group_sum<LPP>(a);
+    cc = group_sum<LPP>(cc);
+    if (li == LPP - 1) ac[j] = make_float2(a, cc);
+  }
+  if constexpr (KB > 1) adjoint_classes<LPP, NBL, KB - 1, NBQ>(src, ac, step, count, grp, li, c, S, g, ltab);
+}
+
 // LPP lanes share one source; a wave evaluates 64 / LPP sources at a time, so
 // the per-source reduction (2 x log2(LPP) DPP adds) is amortised over the
 // group's LPP x NBL bins.  Lane i of a group owns bins e = i + LPP k, k < NBL.
+// The wave's sources are sorted by the 64-bin blocks they reach
+// (blocks_reached); the bins past them have F = s = 0, so they add nothing
+// unless dL/dS is not finite somewhere (then every block is evaluated).
 template <int LPP, int NBL>
 __global__ void __launch_bounds__(kThreads) adjoint_kernel(ParticlesDev D, size_t n, PlanDev P,
                                                            const float* __restrict__ gbar,
@@ -241,12 +255,13 @@ __global__ void __launch_bounds__(kThreads) adjoint_kernel(ParticlesDev D, size_
   float2* ltab = reinterpret_cast<float2*>(smem + kThreads * (sizeof(float4) + sizeof(float2)));
   for (int j = threadIdx.x; j < P.TP; j += kThreads) ltab[j] = P.table[j];
 
-  constexpr int PPW = 64 / LPP;  // sources per wave step
+  constexpr int NBQ = LPP * NBL / 64;  // 64-bin blocks
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int grp = lane / LPP;
   const int li = lane % LPP;
   float c[NBL], S[NBL], g[NBL];
+  bool odd = false;
 #pragma unroll
   for (int k = 0; k < NBL; ++k) {
     const int e = li + LPP * k;
@@ -254,7 +269,10 @@ __global__ void __launch_bounds__(kThreads) adjoint_kernel(ParticlesDev D, size_
     c[k] = cs.x;
     S[k] = cs.y;
     g[k] = (e < P.nbins) ? gbar[e] * P.bine[e] : 0.0f;
+    odd |= !(fabsf(g[k]) < INFINITY);
   }
+  const bool all_blocks = __ballot(odd) != 0;
+  __syncthreads();  // the table is in LDS; each wave's parts of tile and ac are its own
   const double dlnx = -P.K / 0.69314718055994530942;  // dF/dln x = s * du/dln x
 
   const size_t stride = static_cast<size_t>(gridDim.x) * kThreads;
@@ -267,27 +285,17 @@ __global__ void __launch_bounds__(kThreads) adjoint_kernel(ParticlesDev D, size_
     Source s{0.0f, P.v_safe, 0.0f};
     if (p < n) s = particle_source(cur, P);
     if (p + stride < n) raw = load_particle(D, p + stride);  // next tile, in flight
-    __syncthreads();
-    tile[threadIdx.x] = make_float4(s.W, s.vhi, s.vlo, 0.0f);
-    __syncthreads();
-    for (int step = 0; step < 64 / PPW; ++step) {
-      const int j = wave * 64 + step * PPW + grp;
-      const float4 q = tile[j];
-      float a = 0.0f, cc = 0.0f;
-#pragma unroll
-      for (int k = 0; k < NBL; ++k) {
-        const float u = fmaf(c[k], S[k], q.y) + q.z;
-        const float2 cs = ltab[cvt_sat_u32(u)];
-        a = fmaf(g[k], fmaf(u, cs.y, cs.x), a);
-        cc = fmaf(g[k], cs.y, cc);
-      }
-      a = group_sum<LPP>(a);
-      cc = group_sum<LPP>(cc);
-      if (li == LPP - 1) ac[j] = make_float2(a, cc);
-    }
-    __syncthreads();
+    int count[NBQ + 1];
+    const int reach = all_blocks ? (s.W == 0.0f ? 0 : NBQ) : blocks_reached<NBQ>(s, P);
+    const int slot = wave * 64 + class_slot<NBQ>(reach, count);
+    wave_lds_fence();  // the wave's previous sources and sums have been read
+    tile[slot] = make_float4(s.W, s.vhi, s.vlo, 0.0f);
+    ac[slot] = make_float2(0.0f, 0.0f);
+    wave_lds_fence();
+    adjoint_classes<LPP, NBL, NBQ, NBQ>(tile + wave * 64, ac + wave * 64, 0, count, grp, li, c, S, g, ltab);
+    wave_lds_fence();
     if (p >= n) continue;
-    const float2 mine = ac[threadIdx.x];
+    const float2 mine = ac[slot];
     ParticleGrads g{};
     if (s.W != 0.0f) {
       const OmegaTerms o = omega_terms(cur, P.em);
@@ -440,6 +448,12 @@ void build_sync_plan(SyncPlan& plan, const rgn_ftable* table, const float* h_bin
   plan.win_lo = amin - plan.Z;
   plan.win_hi = amax;
   plan.v_safe = static_cast<float>(std::rint(amax));
+  for (int k = 0; k < 8; ++k) {
+    plan.ublk[k] = -1e30f;
+    for (int e = 64 * k; e < std::min(nbins, 64 * (k + 1)); ++e) {
+      if (live[e]) plan.ublk[k] = std::max(plan.ublk[k], static_cast<float>(plan.Z - A[e]));
+    }
+  }
 
   plan.T = T;
   plan.A = A;
@@ -461,6 +475,7 @@ PlanDev device_view(const SyncPlan& plan) {
   P.win_lo = plan.win_lo;
   P.win_hi = plan.win_hi;
   P.v_safe = plan.v_safe;
+  std::copy(std::begin(plan.ublk), std::end(plan.ublk), P.ublk);
   return P;
 }
 

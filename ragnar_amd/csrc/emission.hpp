@@ -21,6 +21,7 @@ struct SyncPlan {
   double Amin = 0.0, Amax = 0.0;
   double win_lo = 0.0, win_hi = 0.0;
   float v_safe = 0.f;
+  float ublk[8] = {};       // largest U_e of the live bins of each 64-bin block
   std::vector<float> bins;  // host copy of the photon bins
   DeviceBuffer table;       // float2[TP]
   DeviceBuffer bincs;       // float2[nbins_pad]

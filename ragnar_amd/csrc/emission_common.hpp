@@ -60,6 +60,7 @@ struct PlanDev {
   double win_lo;    // a particle contributes iff win_lo < B_p < win_hi
   double win_hi;
   float v_safe;     // V_hi for a particle that contributes nowhere
+  float ublk[8];    // largest U_e of the live bins of each 64-bin block (-1e30: none)
 };
 
 // Hardware float -> uint32 conversion: negative inputs and NaN give 0, inputs
@@ -283,6 +284,87 @@ __device__ __forceinline__ Source make_source(float W, float eps, const PlanDev&
     }
   }
   return s;
+}
+
+// Bin reach.  F is exactly zero beyond the table's zero tail (u < 1), so a
+// source adds nothing to the 64-bin blocks k whose largest U_e + B stays below
+// 1; a power-law population puts most sources far below the highest bins (2^24
+// particles, 256 bins over 9 decades: 2.1 of 4 blocks on average).  The
+// pair-by-pair kernels are bound by VALU issue, so they sort the 64 sources of
+// a wave by the number of leading blocks they reach and evaluate each class
+// against its own blocks only: 10^6 particles x 256 bins 53 -> 44 us a call,
+// 27M particles in 4096 cells x 256 bins 1061 -> 819 us.
+// 0.99 leaves room for the float rounding of ublk and B (below 2e-3 at the
+// table's size limit); pairs left out would have added exactly zero.  A
+// non-finite weight reaches every bin (its products with zero are NaN).
+template <int NB>
+__device__ __forceinline__ int blocks_reached(const Source& s, const PlanDev& P) {
+  const float v = s.vhi + s.vlo;
+  int c = 0;
+#pragma unroll
+  for (int k = 0; k < NB; ++k) {
+    if (P.ublk[k] + v >= 0.99f) c = k + 1;
+  }
+  if (s.W == 0.0f) c = 0;
+  return fabsf(s.W) < INFINITY ? c : NB;
+}
+
+// Slot of the lane's source among the wave's 64, classes in descending order;
+// count[k] (1 <= k <= NB): sources of the wave that reach k blocks or more.
+template <int NB>
+__device__ __forceinline__ int class_slot(int c, int (&count)[NB + 1]) {
+  int total = 0, slot = 0;
+#pragma unroll
+  for (int k = NB; k >= 0; --k) {
+    const unsigned long long m = __ballot(c == k);
+    const int before = __builtin_amdgcn_mbcnt_hi(static_cast<unsigned>(m >> 32),
+                                                 __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(m), 0u));
+    if (c == k) slot = total + before;
+    total += __popcll(m);
+    count[k] = total;
+  }
+  return slot;
+}
+
+// LDS written and read by one wave only (its lanes run in lockstep): orders
+// the two without a block barrier.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// acc[k] += W F over sources [j, end) of src for the blocks k < KB.
+template <int KB, int NB>
+__device__ __forceinline__ void eval_blocks(const float4* __restrict__ src, int& j, int end, const float (&c)[NB],
+                                            const float (&S)[NB], const float2* __restrict__ ltab,
+                                            float (&acc)[NB]) {
+  constexpr int kStep = KB <= 2 ? 8 : 4;  // sources in flight
+  for (; j < end; j += kStep) {
+#pragma unroll
+    for (int q = 0; q < kStep; ++q) {
+      const float4 s = src[j + q];
+#pragma unroll
+      for (int k = 0; k < KB; ++k) {
+        const float u = fmaf(c[k], S[k], s.y) + s.z;
+        const float2 cs = ltab[cvt_sat_u32(u)];
+        acc[k] = fmaf(s.x, fmaf(u, cs.y, cs.x), acc[k]);
+      }
+    }
+  }
+}
+
+// A wave's 64 sources (sorted by class_slot) against its lanes' bins, class
+// by class; a step may run past a class's end into sources that reach fewer
+// blocks, whose extra terms are zero.
+template <int KB, int NB>
+__device__ __forceinline__ void eval_classes(const float4* __restrict__ src, int j, const int (&count)[NB + 1],
+                                             const float (&c)[NB], const float (&S)[NB],
+                                             const float2* __restrict__ ltab, float (&acc)[NB]) {
+  // the eight-source steps of KB <= 2 start at a multiple of eight, so no step
+  // reads past the wave's 64 sources
+  eval_blocks<KB, NB>(src, j, KB == 3 ? (count[KB] + 7) & ~7 : count[KB], c, S, ltab, acc);
+  if constexpr (KB > 1) eval_classes<KB - 1, NB>(src, j, count, c, S, ltab, acc);
 }
 
 // One entry of the distribution kernel matrix K[g, e] (KernelFromDist,
