@@ -597,6 +597,8 @@ def roofline(prof, n, nb, plan):
     forward_kernel (direct): 6 FP32 VALU flop per particle x bin eval (the
       inner loop: two FMAs forming u, one table-index conversion, the FMA of
       the interpolant and the accumulating FMA); bound: FP32 VALU.
+    binned_stream: reads u and B (24 B/particle); its list of sources outside
+      the window (10 B for each of those) is left out; bound: HBM.
     binned_bucket: reads u and B (24 B/particle) and writes each contributing
       source's (W, phi) (8 B/particle); its run descriptors (4 B per non-empty
       run, ~40 sources per run here) are left out; bound: HBM.
@@ -611,7 +613,9 @@ def roofline(prof, n, nb, plan):
         return {"bound": "valu", "achieved": achieved / 1e12, "peak": PEAK_FP32 / 1e12,
                 "unit": "TFLOP/s", "frac": achieved / PEAK_FP32, "traffic": read_traffic(name),
                 "kernel": name, "kernel_ms": ms, "flop_per_eval": FLOP_PER_EVAL_FWD}
-    if name == "binned_bucket":
+    if name == "binned_stream":
+        nbytes = 24 * n
+    elif name == "binned_bucket":
         nbytes = 32 * n
     elif name == "binned_subhist":
         items = n // 16384 + info["NK"]

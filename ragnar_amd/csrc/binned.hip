@@ -14,8 +14,13 @@
 // with P = prefix at r_e and T = totals.  This is the same piecewise-linear
 // function the direct kernel evaluates pair by pair, summed in FP64.
 //
-// Forward (a scatter), no global atomics (device-scope FP64 atomics run at
-// ~14 G/s on MI355X):
+// Forward up to 256 bins: one persistent block per CU (binned_stream) reads its
+// particles once and keeps the moments of a window of consecutive buckets in
+// LDS; the sources outside the window go to a list in memory and are reduced at
+// the end, bucket by bucket; the block's FP64 spectrum goes to combine_kernel.
+//
+// Forward beyond (a scatter), no global atomics (device-scope FP64 atomics run
+// at ~14 G/s on MI355X):
 //   bucket    each block of 8192 particles computes (k, W, phi), counting-sorts
 //             its sources by k in LDS and writes the sorted (W, phi) chunk
 //             coalesced, plus one run descriptor per non-empty bucket;
@@ -44,7 +49,7 @@
 namespace rgn {
 
 namespace {
-constexpr int kLutCells = 2048;  // sub-cell lookup cells in a sub-histogram block
+constexpr int kLutCells = 2048;  // sub-cell lookup cells of the forward pass
 constexpr int kLog2Tab = 256;    // entries of the factorised passes' log2 table
 }  // namespace
 
@@ -54,11 +59,12 @@ void build_binned_tables(SyncPlan& plan, const std::vector<float>& xs, const std
   for (int e = 0; e < plan.nbins; ++e) {
     if (plan.live[e]) alphas.push_back(plan.A[e] - std::floor(plan.A[e]));
   }
+  // One sub-cell boundary per live bin, equal offsets kept (the sub-cells
+  // between them stay empty), so that rank r belongs to one bin, ri[r].
   std::sort(alphas.begin(), alphas.end());
-  alphas.erase(std::unique(alphas.begin(), alphas.end()), alphas.end());
   plan.M = static_cast<int>(alphas.size());
-  std::vector<BinInfo> bi(plan.nbins);
-  std::vector<int> rcount(plan.M + 1, 0);
+  std::vector<BinInfo> bi(plan.nbins), ri(std::max(1, plan.M));
+  std::vector<int> used(plan.M + 1, 0);
   for (int e = 0; e < plan.nbins; ++e) {
     if (!plan.live[e]) {
       bi[e] = BinInfo{0.0, 0, -1};
@@ -66,19 +72,10 @@ void build_binned_tables(SyncPlan& plan, const std::vector<float>& xs, const std
     }
     const double a = std::floor(plan.A[e]);
     const double al = plan.A[e] - a;
-    const int r = static_cast<int>(std::lower_bound(alphas.begin(), alphas.end(), al) - alphas.begin());
+    const int r0 = static_cast<int>(std::lower_bound(alphas.begin(), alphas.end(), al) - alphas.begin());
+    const int r = r0 + used[r0]++;
     bi[e] = BinInfo{plan.A[e], static_cast<int>(a), r};
-    ++rcount[r];
-  }
-  // live bins grouped by alpha rank, ascending e within a rank
-  std::vector<int> rptr(plan.M + 1, 0), rlist;
-  for (int r = 0; r < plan.M; ++r) rptr[r + 1] = rptr[r] + rcount[r];
-  rlist.resize(std::max(1, rptr[plan.M]));
-  {
-    std::vector<int> cur(rptr.begin(), rptr.end() - 1);
-    for (int e = 0; e < plan.nbins; ++e) {
-      if (bi[e].r >= 0) rlist[cur[bi[e].r]++] = e;
-    }
+    ri[r] = BinInfo{al, bi[e].a, e};
   }
   std::vector<SegInfo> seg(std::max(T - 1, 1));
   auto tau = [&](int i) { return (std::log2(static_cast<double>(xs[i])) - plan.log2_xmin) * plan.K; };
@@ -86,6 +83,10 @@ void build_binned_tables(SyncPlan& plan, const std::vector<float>& xs, const std
     const double t0 = tau(s), t1 = tau(s + 1);
     seg[s] = SegInfo{t0, ys[s], (static_cast<double>(ys[s + 1]) - ys[s]) / (t1 - t0)};
   }
+  // the same lines as functions of t - s: entry s + 1 holds (value at t = s,
+  // slope); the entries before and after the table's segments are zero
+  std::vector<double2> line(T + 1, make_double2(0.0, 0.0));
+  for (int s = 0; s + 1 < T; ++s) line[s + 1] = make_double2(seg[s].y + (s - seg[s].tau) * seg[s].sigma, seg[s].sigma);
   if (plan.M > 0) {
     // sources can contribute only for B in (A_min - tau_{T-1}, A_max)
     plan.kmin = static_cast<int>(std::floor(plan.Amin - (T - 1))) - 1;
@@ -122,7 +123,7 @@ void build_binned_tables(SyncPlan& plan, const std::vector<float>& xs, const std
   plan.jlut.reset(jlut.size() * sizeof(unsigned short));
   RGN_HIP(hipMemcpy(plan.jlut.ptr, jlut.data(), plan.jlut.bytes, hipMemcpyHostToDevice));
   {
-    // the sub-histogram's lookup cells c of [c / JQ2, (c + 1) / JQ2): the alphas
+    // the forward pass's lookup cells c of [c / JQ2, (c + 1) / JQ2): the alphas
     // below the cell, a flag for cells holding two alphas or more, and the
     // first threshold (as float bits)
     const int JQ2 = std::min(JQ, kLutCells), r = JQ / JQ2;
@@ -138,14 +139,14 @@ void build_binned_tables(SyncPlan& plan, const std::vector<float>& xs, const std
     plan.sublut.reset(lut.size() * sizeof(uint2));
     RGN_HIP(hipMemcpy(plan.sublut.ptr, lut.data(), plan.sublut.bytes, hipMemcpyHostToDevice));
   }
-  plan.rptr.reset(rptr.size() * sizeof(int));
-  RGN_HIP(hipMemcpy(plan.rptr.ptr, rptr.data(), plan.rptr.bytes, hipMemcpyHostToDevice));
-  plan.rlist.reset(rlist.size() * sizeof(int));
-  RGN_HIP(hipMemcpy(plan.rlist.ptr, rlist.data(), plan.rlist.bytes, hipMemcpyHostToDevice));
   plan.binfo.reset(bi.size() * sizeof(BinInfo));
   RGN_HIP(hipMemcpy(plan.binfo.ptr, bi.data(), bi.size() * sizeof(BinInfo), hipMemcpyHostToDevice));
+  plan.rinfo.reset(ri.size() * sizeof(BinInfo));
+  RGN_HIP(hipMemcpy(plan.rinfo.ptr, ri.data(), plan.rinfo.bytes, hipMemcpyHostToDevice));
   plan.seg.reset(seg.size() * sizeof(SegInfo));
   RGN_HIP(hipMemcpy(plan.seg.ptr, seg.data(), seg.size() * sizeof(SegInfo), hipMemcpyHostToDevice));
+  plan.line.reset(line.size() * sizeof(double2));
+  RGN_HIP(hipMemcpy(plan.line.ptr, line.data(), plan.line.bytes, hipMemcpyHostToDevice));
   {
     // log2 table (log2_tab): entry i holds 2 inv_i and -log2 inv_i, inv_i = RN(1 / c_i),
     // c_i = 1 + (i + 1/2) / 256, the logarithm in long double
@@ -177,21 +178,27 @@ struct BinnedDev {
   const float* athr;
   const unsigned short* jlut;
   const uint2* sublut;
-  const int* rptr;
-  const int* rlist;
   const BinInfo* binfo;
+  const BinInfo* rinfo;
   const SegInfo* seg;
+  const double2* line;
   const float* bine;
   const double2* l2tab;
   int M, JQ, T, kmin, NK, nbins;
   EmitConst em;
   double K;
+  double c_peak;  // e_at / (B0 g_syn^2)
 };
 
+double peak_scale(const SyncPlan& p) {
+  const EmitConst c = emit_const(p);
+  return static_cast<double>(p.e_at) * c.rDg * c.rB0;
+}
+
 BinnedDev binned_view(const SyncPlan& p) {
-  return BinnedDev{p.alpha.as<double>(), p.athr.as<float>(), p.jlut.as<unsigned short>(), p.sublut.as<uint2>(), p.rptr.as<int>(), p.rlist.as<int>(),
-                   p.binfo.as<BinInfo>(), p.seg.as<SegInfo>(), p.bine.as<float>(), p.l2tab.as<double2>(),
-                   p.M, p.JQ, p.T, p.kmin, p.NK, p.nbins, emit_const(p), p.K};
+  return BinnedDev{p.alpha.as<double>(), p.athr.as<float>(), p.jlut.as<unsigned short>(), p.sublut.as<uint2>(), 
+                   p.binfo.as<BinInfo>(), p.rinfo.as<BinInfo>(), p.seg.as<SegInfo>(), p.line.as<double2>(), p.bine.as<float>(), p.l2tab.as<double2>(),
+                   p.M, p.JQ, p.T, p.kmin, p.NK, p.nbins, emit_const(p), p.K, peak_scale(p)};
 }
 
 // log2 of a positive finite float to ~1e-11 absolute, from a table (in LDS):
@@ -286,6 +293,547 @@ __global__ void __launch_bounds__(kThreads) fill_zero(unsigned* __restrict__ p, 
   for (size_t i = static_cast<size_t>(blockIdx.x) * kThreads + threadIdx.x; i < n;
        i += static_cast<size_t>(gridDim.x) * kThreads) {
     p[i] = 0u;
+  }
+}
+
+// Start of the window of `len` consecutive buckets holding the most sources
+// of hist (lowest start on ties); hist becomes its inclusive prefix sums.  Every
+// thread of the NT-thread block calls it, after a barrier on hist; s_key:
+// NT / 64 words of LDS, s_part likewise.
+template <int NT>
+__device__ __forceinline__ int densest_window(unsigned* hist, int NK, int len, unsigned long long* s_key,
+                                              unsigned* s_part, int* s_w0) {
+  unsigned before = 0;
+  for (int k0 = 0; k0 < NK; k0 += NT) {
+    const int k = k0 + static_cast<int>(threadIdx.x);
+    const unsigned c = k < NK ? hist[k] : 0u;
+    unsigned all;
+    const unsigned x = block_prefix<unsigned, NT>(c, all, s_part);
+    if (k < NK) hist[k] = before + x + c;
+    before += all;
+  }
+  __syncthreads();
+  const int nw = max(1, NK - len + 1);
+  unsigned best = 0;
+  int bw = 0x7fffffff;
+  for (int w = threadIdx.x; w < nw; w += NT) {
+    const unsigned c = hist[min(NK, w + len) - 1] - (w ? hist[w - 1] : 0u);
+    if (c > best || (c == best && w < bw)) {
+      best = c;
+      bw = w;
+    }
+  }
+  // block arg-max: pack (count, -start) into 64 bits
+  unsigned long long key = (static_cast<unsigned long long>(best) << 32) |
+                           static_cast<unsigned>(0x7fffffff - min(bw, 0x7fffffff));
+#pragma unroll
+  for (int m = 1; m < 64; m <<= 1) {
+    const unsigned long long o = __shfl_xor(key, m);
+    key = o > key ? o : key;
+  }
+  if ((threadIdx.x & 63) == 0) s_key[threadIdx.x >> 6] = key;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    unsigned long long k2 = s_key[0];
+    for (int i = 1; i < NT / 64; ++i) k2 = s_key[i] > k2 ? s_key[i] : k2;
+    *s_w0 = 0x7fffffff - static_cast<int>(k2 & 0xffffffffu);
+  }
+  __syncthreads();
+  return min(*s_w0, nw - 1);
+}
+
+// A value that is the same in every lane of the wave, in a scalar register.
+__device__ __forceinline__ unsigned wave_uniform(unsigned v) { return __builtin_amdgcn_readfirstlane(v); }
+
+// v moved by a DPP control (lanes without a source, and rows outside ROW_MASK,
+// read 0).
+template <int CTRL, int ROW_MASK = 0xf>
+__device__ __forceinline__ double dpp_d(double v) {
+  constexpr bool kBound = ROW_MASK == 0xf;  // bound_ctrl supplies the zero: no register to clear first
+  const unsigned long long b = __double_as_longlong(v);
+  const unsigned lo = __builtin_amdgcn_update_dpp(0, static_cast<int>(b), CTRL, ROW_MASK, 0xf, kBound);
+  const unsigned hi = __builtin_amdgcn_update_dpp(0, static_cast<int>(b >> 32), CTRL, ROW_MASK, 0xf, kBound);
+  return __longlong_as_double(static_cast<unsigned long long>(hi) << 32 | lo);
+}
+
+// Inclusive sum over the lanes of a wave.
+__device__ __forceinline__ double wave_scan(double v) {
+  v += dpp_d<0x111>(v);  // row_shr 1, 2, 4, 8: within rows of 16 lanes
+  v += dpp_d<0x112>(v);
+  v += dpp_d<0x114>(v);
+  v += dpp_d<0x118>(v);
+  v += dpp_d<kDppRowBcast15, 0xa>(v);
+  v += dpp_d<kDppRowBcast31, 0xc>(v);
+  return v;
+}
+
+__device__ __forceinline__ double last_lane(double v) {
+  const unsigned long long b = __double_as_longlong(v);
+  const unsigned lo = __builtin_amdgcn_readlane(static_cast<int>(b), 63);
+  const unsigned hi = __builtin_amdgcn_readlane(static_cast<int>(b >> 32), 63);
+  return __longlong_as_double(static_cast<unsigned long long>(hi) << 32 | lo);
+}
+
+// 1 / sqrt(x) to about one ulp for finite x > 0 (hardware estimate, one
+// third-order step); x = 0 and x = inf give NaN.
+__device__ __forceinline__ double rsqrt_nr(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-x * y, y, 1.0);
+  return fma(y * e, fma(e, 0.375, 0.5), y);
+}
+
+// One particle of the forward pass in FP64: its weight W times B0, and B = k +
+// phi (k counted from kmin); false when it contributes nowhere.  With G = gamma
+// V = gamma E + u x B and Q = |G|^2 - (u.E)^2 = gamma^2 rootQ^2, the emission
+// terms need one reciprocal square root y = (Q gamma^2)^(-1/2):
+//   chi = rootQ / B0 = Q y / B0,   e_peak = e_at gamma^2 chi / g_syn^2 = (Q gamma^2 y) e_at / (B0 g_syn^2).
+// Nothing is rounded to float on the way (the reference rounds the squared
+// momenta, chi and e_peak); half the instructions of omega_terms_approx and
+// log2_tab, in a pass that issues vector instructions most of its time.
+// e_peak outside the float range (0, infinite, negative, NaN) drops the
+// particle, as synchrotron.hpp:162 does.  tab: stage_log2's table.
+struct StreamSource {
+  double W, phi;
+  int k;
+};
+
+template <bool HAS_E>
+__device__ __forceinline__ bool stream_source(const RawParticle& r, const BinnedDev& P,
+                                              const double2* __restrict__ tab, StreamSource& o) {
+  const double ux = r.ux, uy = r.uy, uz = r.uz, bx = r.bx, by = r.by, bz = r.bz;
+  const double g2 = fma(ux, ux, fma(uy, uy, fma(uz, uz, 1.0)));
+  double gx = fma(uy, bz, -uz * by), gy = fma(uz, bx, -ux * bz), gz = fma(ux, by, -uy * bx);
+  double Q;
+  if (HAS_E) {
+    const double ex = r.ex, ey = r.ey, ez = r.ez;
+    const double gamma = g2 * rsqrt_nr(g2);
+    gx = fma(gamma, ex, gx);
+    gy = fma(gamma, ey, gy);
+    gz = fma(gamma, ez, gz);
+    const double ue = fma(ux, ex, fma(uy, ey, uz * ez));
+    Q = fma(gx, gx, fma(gy, gy, fma(gz, gz, -ue * ue)));
+  } else {
+    Q = fma(gx, gx, fma(gy, gy, gz * gz));
+  }
+  const double x = Q * g2;
+  const double y = rsqrt_nr(x);
+  const double e = x * y * P.c_peak;
+  o.W = Q * y * static_cast<double>(r.w);
+  const unsigned long long bits = __double_as_longlong(e);
+  const unsigned hi = static_cast<unsigned>(bits >> 32);
+  constexpr unsigned kLo = (1023u - 149u) << 20, kHi = (1023u + 128u) << 20;  // 2^-149 <= e < 2^128
+  const bool in_range = hi - kLo < kHi - kLo;
+  const double mf = __longlong_as_double(static_cast<long long>(
+    (bits & 0x000fffffffffffffull) | 0x3fe0000000000000ull));  // [0.5, 1)
+  const double2 t = tab[(hi >> 12) & (kLog2Tab - 1)];
+  const double d = fma(mf, t.x, -1.0);
+  const double q = d * fma(d, fma(d, 1.0 / 3.0, -0.5), 1.0);  // ln(1 + d)
+  const double B = fma(static_cast<double>(static_cast<int>(hi >> 20)), P.K, fma(q, 1.4426950408889634 * P.K, t.y));
+  const double fl = floor(B);
+  o.phi = B - fl;
+  o.k = static_cast<int>(fl);
+  return in_range && static_cast<unsigned>(o.k) < static_cast<unsigned>(P.NK);
+}
+
+// The log2 table of log2_tab with the second entries scaled to table units and
+// shifted, so that K log2 x - kmin = (exponent bits) K + q K / ln 2 + entry.
+__device__ __forceinline__ double2 stage_log2(double2 t, const BinnedDev& P) {
+  return make_double2(t.x, (t.y - 1023.0) * P.K - static_cast<double>(P.kmin));
+}
+
+// The photon bins of one lane: ranks lane * Q + q, q < Q (a = INT_MIN: none),
+// and the lane's share of the block's spectrum.
+template <int Q>
+struct LaneBins {
+  double alpha[Q], acc[Q];
+  int a[Q];
+};
+
+// Place of sub-cell j in a row of moments: the Q sub-cells of a lane's bins lie
+// row_width apart, so that the lanes of a wave read consecutive words (in plain
+// order they would be Q apart, an up to 8-way bank conflict that cost
+// add_bucket half of its time).
+template <int Q>
+__device__ __forceinline__ int row_width(int M) { return M / Q + 1; }
+template <int Q>
+__device__ __forceinline__ int row_place(int j, int width) {
+  return static_cast<int>(__umul24(j % static_cast<unsigned>(Q), width)) + j / static_cast<unsigned>(Q);
+}
+
+// The sub-cell lookup of a source in LDS: JQ2 + 1 cells of [0, 1] with the first
+// threshold (athr) at or above the cell and the places of the sub-cells on its
+// two sides; a cell holding several thresholds keeps the first one's rank and
+// scans on.  Made from the plan's table (rank, flag, threshold) at the start.
+constexpr unsigned kScan = 0x80000000u;
+
+template <int Q>
+__device__ __forceinline__ uint2 stage_cell(uint2 c, int width) {
+  const unsigned j = c.x & 0xffffu;
+  if (c.x >> 16) return make_uint2(kScan | j, c.y);
+  return make_uint2(row_place<Q>(j, width) | row_place<Q>(j + 1, width) << 16, c.y);
+}
+
+// Place of the sub-cell of phi (the number of alphas below it).
+template <int Q>
+__device__ __forceinline__ int cell_place(const uint2* __restrict__ lut, const float* __restrict__ athr, int JQ2,
+                                          int width, float phi) {
+  const uint2 c = lut[static_cast<int>(phi * JQ2)];
+  const bool above = __uint_as_float(c.y) <= phi;
+  if (static_cast<int>(c.x) < 0) {
+    // four thresholds at a time (+inf follows the last); some bin sets have
+    // their offsets in clusters, 200 bins over nine decades in eight
+    int j = static_cast<int>(c.x & 0xffffu), n;
+    do {
+      n = (athr[j] <= phi) + (athr[j + 1] <= phi) + (athr[j + 2] <= phi) + (athr[j + 3] <= phi);
+      j += n;
+    } while (n == 4);
+    return row_place<Q>(j, width);
+  }
+  return (above ? c.x >> 16 : c.x) & 0xffffu;
+}
+
+// Adds a bucket's moments to the lane's bins.  row: m0 of the M + 1 sub-cells
+// (row_place), then m1.  The lane's sub-cells are those of its bins, so the
+// prefix sums it needs end in its own registers.
+template <int Q>
+__device__ __forceinline__ void add_bucket(LaneBins<Q>& L, const double* __restrict__ row, int M, int k,
+                                           const double2* __restrict__ line, int T, int lane) {
+  const int width = row_width<Q>(M);
+  double p0[Q], p1[Q];
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    const bool in = lane * Q + q < M;
+    p0[q] = in ? row[q * width + lane] : 0.0;
+    p1[q] = in ? row[(Q + q) * width + lane] : 0.0;
+  }
+  const int last = row_place<Q>(M, width);
+  const double e0 = row[last], e1 = row[Q * width + last];
+#pragma unroll
+  for (int q = 1; q < Q; ++q) {
+    p0[q] += p0[q - 1];
+    p1[q] += p1[q - 1];
+  }
+  const double i0 = wave_scan(p0[Q - 1]), i1 = wave_scan(p1[Q - 1]);
+  const double t0 = last_lane(i0) + e0, t1 = last_lane(i1) + e1;
+  const double x0 = i0 - p0[Q - 1], x1 = i1 - p1[Q - 1];
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    const double P0 = x0 + p0[q], P1 = x1 + p1[q];
+    const int m = L.a[q] - k;
+    const double2 s1 = line[min(static_cast<unsigned>(max(m + 1, 0)), static_cast<unsigned>(T))];
+    const double2 s0 = line[min(static_cast<unsigned>(max(m, 0)), static_cast<unsigned>(T))];
+    // A_e - k = m + alpha = (m - 1) + (alpha + 1)
+    const double C1 = fma(L.alpha[q], s1.y, s1.x), C0 = fma(L.alpha[q] + 1.0, s0.y, s0.x);
+    double v = fma(C1, P0, fma(-s1.y, P1, L.acc[q]));
+    L.acc[q] = fma(C0, t0 - P0, fma(-s0.y, t1 - P1, v));
+  }
+}
+
+// Adds one source to the lane's bins.
+template <int Q>
+__device__ __forceinline__ void add_source(LaneBins<Q>& L, float2 wp, int k, const double2* __restrict__ line, int T) {
+  const double W = wp.x, phi = wp.y;
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    const int right = phi > L.alpha[q];  // the segment before
+    const double2 s = line[min(static_cast<unsigned>(max(L.a[q] - k - right + 1, 0)), static_cast<unsigned>(T))];
+    const double F = fma(-s.y, phi, fma(L.alpha[q] + right, s.y, s.x));
+    L.acc[q] = fma(W, F, L.acc[q]);
+  }
+}
+
+// Launch shape of binned_stream.  The rows (two doubles per sub-cell) and
+// everything else that changes its use share `area` doubles of LDS.
+struct StreamShape {
+  int rows;        // buckets in a window
+  int area;        // doubles
+  int nline;       // entries of the line table in LDS
+  int tail_waves;  // waves that reduce the end of the list, a row each
+  unsigned stage;  // its sources, after those rows
+  unsigned cap;    // list entries of a block
+};
+
+constexpr int kStream = 1024;      // threads of a binned_stream block, one per CU
+constexpr int kSparse = 4;         // list buckets of at most this many sources go source by source
+constexpr int kStageRounds = 3;    // a list that takes more rounds of staging gets a window first
+static_assert(kBinnedMaxNK <= 65535, "list entries keep the bucket in 16 bits");
+
+// The spectrum of one block's particles.  Two launches instead of the passes'
+// five, no sorted copy of the sources; bound by the loads and by vector and LDS
+// issue together (counters at 2^24 particles x 256 bins: VALU 46%, LDS 36% of
+// the cycles).  Block clocks there: 5 us set-up, 76 us stream (5.3 TB/s), 3 us
+// window, 28 us list (18% of the sources); the call 159 -> 122 us.  At 10^6
+// particles 6 us stream, 19 us the rest; 53 us (pair by pair) -> 33 us.
+//   1  The buckets of the first kStream particles pick the window: the `rows`
+//      consecutive buckets holding most of them.
+//   2  Every particle's (k, W, phi) adds W and W phi to its sub-cell of the
+//      window's rows in LDS (ds_add_f64), or goes to the block's list.
+//   3  Each wave takes rows of the window: prefix sums over the sub-cells and
+//      the bins' lines (add_bucket), into FP64 registers.
+//   4  The list.  While it is long, the densest window of its own buckets is
+//      reduced the same way and the other entries are packed together.  What is
+//      left is counting-sorted by bucket into LDS, as much at a time as fits,
+//      and each wave takes a bucket, reduces it into a row of its own and adds
+//      it as in 3 (source by source where there are few).
+//   5  The waves' spectra are added in order into partials[bin][block].
+template <int Q, bool HAS_E, bool NT>
+__global__ void __launch_bounds__(kStream) binned_stream(ParticlesDev D, unsigned n, BinnedDev P, StreamShape S,
+                                                         float2* __restrict__ list_wp,
+                                                         unsigned short* __restrict__ list_k,
+                                                         double* __restrict__ partials) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  constexpr int kWaves = kStream / 64;
+  const int M = P.M, NK = P.NK, JQ2 = min(P.JQ, kLutCells);
+  const int width = row_width<Q>(M), pitch = 2 * Q * width;  // doubles of a row
+  double2* l2 = reinterpret_cast<double2*>(smem);
+  double2* lline = l2 + kLog2Tab;
+  double* area = reinterpret_cast<double*>(lline + S.nline);
+  uint2* lut = reinterpret_cast<uint2*>(area + S.area);
+  float* athr = reinterpret_cast<float*>(lut + JQ2 + 1);
+  unsigned* hist = reinterpret_cast<unsigned*>(athr + M + 4);  // NK
+  unsigned* offs = hist + NK;                                  // NK + 1
+  unsigned short* occ = reinterpret_cast<unsigned short*>(offs + NK + 1);  // NK
+  unsigned char* done = reinterpret_cast<unsigned char*>(occ + NK);        // NK: list buckets dealt with
+  __shared__ unsigned long long s_key[kWaves];
+  __shared__ unsigned s_part[kWaves], s_count;
+  __shared__ int s_w0;
+  const int tid = threadIdx.x, lane = tid & 63, wave = wave_uniform(tid >> 6);
+  const unsigned stride = gridDim.x * kStream;
+  unsigned p = blockIdx.x * kStream + tid;
+  // four particles per thread in flight; past the end, the last one again
+  auto load = [&](unsigned i) { return load_particle32<NT>(D, min(i, n - 1)); };
+  RawParticle ring[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) ring[i] = load(p + i * stride);
+  for (int i = tid; i < S.rows * pitch; i += kStream) area[i] = 0.0;
+  for (int i = tid; i < NK; i += kStream) {
+    hist[i] = 0u;
+    done[i] = 0;
+  }
+  for (int i = tid; i < S.nline; i += kStream) lline[i] = P.line[i];
+  for (int i = tid; i <= JQ2; i += kStream) {
+    lut[i] = stage_cell<Q>(i < JQ2 ? P.sublut[i] : make_uint2(M, 0x7f800000u), width);  // phi rounded to 1
+  }
+  for (int i = tid; i < M + 4; i += kStream) athr[i] = i < M ? P.athr[i] : INFINITY;
+  if (tid < kLog2Tab) l2[tid] = stage_log2(P.l2tab[tid], P);
+  if (tid == 0) s_count = 0u;
+  LaneBins<Q> L;
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    const int r = lane * Q + q;
+    L.acc[q] = 0.0;
+    L.alpha[q] = 0.0;
+    L.a[q] = -(1 << 30);  // no bin: every line is zero
+    if (r < M) {
+      const BinInfo b = P.rinfo[r];
+      L.alpha[q] = b.A;
+      L.a[q] = b.a;
+    }
+  }
+  __syncthreads();
+  StreamSource src;
+  bool in;
+  auto next = [&](RawParticle& r) {
+    in = stream_source<HAS_E>(r, P, l2, src) && p < n;
+    r = load(p + 4 * stride);
+    p += stride;
+  };
+  next(ring[0]);
+  int w0 = 0;
+  const int rows = min(S.rows, NK);
+  if (rows < NK) {
+    if (in) atomicAdd(hist + src.k, 1u);
+    __syncthreads();
+    w0 = densest_window<kStream>(hist, NK, S.rows, s_key, s_part, &s_w0);
+    for (int i = tid; i < NK; i += kStream) hist[i] = 0u;
+    __syncthreads();
+  }
+  float2* my_wp = list_wp + static_cast<size_t>(blockIdx.x) * S.cap;
+  unsigned short* my_k = list_k + static_cast<size_t>(blockIdx.x) * S.cap;
+  // a source into the window's rows; false when its bucket is outside
+  auto into_window = [&](double W, double phi, int k, int place) {
+    const unsigned row = static_cast<unsigned>(k - w0);
+    if (row >= static_cast<unsigned>(rows)) return false;
+    double* m = area + __umul24(row, pitch) + place;
+    atomicAdd(m, W);
+    atomicAdd(m + Q * width, W * phi);
+    return true;
+  };
+  // the wave's active lanes take consecutive list entries (one list per block:
+  // a list per wave leaves 16 times as many half-written lines behind, and the
+  // stream ran 80 instead of 75 us at 2^24)
+  auto to_list = [&](float2 wp, int k) {
+    const unsigned long long mask = __ballot(true);
+    unsigned at = 0;
+    if (lane == __ffsll(mask) - 1) at = atomicAdd(&s_count, static_cast<unsigned>(__popcll(mask)));
+    at = wave_uniform(at) + __builtin_amdgcn_mbcnt_hi(static_cast<unsigned>(mask >> 32),
+                                                      __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(mask), 0u));
+    my_wp[at] = wp;
+    my_k[at] = static_cast<unsigned short>(k);
+  };
+  // Every entry of the list to take(wp, k), four per thread at a time, the next
+  // four in flight.
+  auto sweep_list = [&](unsigned count, auto&& take) {
+    float2 wp[4];
+    int k[4];
+    auto fetch = [&](unsigned i0) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const unsigned i = min(i0 + q * kStream + tid, count - 1);
+        wp[q] = my_wp[i];
+        k[q] = my_k[i];
+      }
+    };
+    fetch(0);
+    for (unsigned i0 = 0; i0 < count; i0 += 4 * kStream) {
+      float2 cwp[4];
+      int ck[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        cwp[q] = wp[q];
+        ck[q] = k[q];
+      }
+      if (i0 + 4 * kStream < count) fetch(i0 + 4 * kStream);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        if (i0 + q * kStream + tid < count) take(cwp[q], ck[q]);
+      }
+    }
+  };
+  auto add_window = [&]() {
+    for (int i = wave; i < rows; i += kWaves) add_bucket<Q>(L, area + i * pitch, M, P.kmin + w0 + i, lline, P.T, lane);
+  };
+  for (unsigned base = blockIdx.x * kStream; base < n; base += 4 * stride) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (in) {
+        const float phi = static_cast<float>(src.phi);
+        if (!into_window(src.W, src.phi, src.k, cell_place<Q>(lut, athr, JQ2, width, phi))) {
+          to_list(make_float2(static_cast<float>(src.W), phi), src.k);
+          atomicAdd(hist + src.k, 1u);
+        }
+      }
+      next(ring[(i + 1) % 4]);
+    }
+  }
+  __syncthreads();
+  add_window();
+  const unsigned listed = s_count;
+  // sources left in the list's buckets, and in the fullest (every thread calls it)
+  auto left = [&](unsigned& most) {
+    unsigned c = 0, m = 0;
+    for (int i = tid; i < NK; i += kStream) {
+      c += hist[i];
+      m = max(m, hist[i]);
+    }
+#pragma unroll
+    for (int w = 32; w > 0; w >>= 1) {
+      c += static_cast<unsigned>(__shfl_xor(static_cast<int>(c), w));
+      m = max(m, static_cast<unsigned>(__shfl_xor(static_cast<int>(m), w)));
+    }
+    __syncthreads();
+    if (lane == 0) s_key[wave] = static_cast<unsigned long long>(m) << 32 | c;
+    __syncthreads();
+    c = 0;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+      c += static_cast<unsigned>(s_key[w]);
+      m = max(m, static_cast<unsigned>(s_key[w] >> 32));
+    }
+    most = m;
+    __syncthreads();
+    return c;
+  };
+  unsigned most, count = left(most);
+  // A long list, or one with a bucket beyond the staging space: its densest
+  // window first.
+  while (count > kStageRounds * S.stage || most > S.stage) {
+    // hist holds the list's bucket counts; offs takes the copy that the window is picked from
+    for (int i = tid; i < NK; i += kStream) offs[i] = hist[i];
+    for (int i = tid; i < rows * pitch; i += kStream) area[i] = 0.0;
+    __syncthreads();
+    w0 = densest_window<kStream>(offs, NK, rows, s_key, s_part, &s_w0);
+    sweep_list(listed, [&](float2 wp, int k) {
+      if (static_cast<unsigned>(k - w0) < static_cast<unsigned>(rows) && !done[k]) {
+        into_window(wp.x, wp.y, k, cell_place<Q>(lut, athr, JQ2, width, wp.y));
+      }
+    });
+    __syncthreads();
+    add_window();
+    for (int i = tid; i < rows; i += kStream) {
+      hist[w0 + i] = 0u;
+      done[w0 + i] = 1;
+    }
+    __syncthreads();
+    count = left(most);
+  }
+  if (count) {
+    block_scan_exclusive<unsigned, kStream>(hist, offs, NK, s_part);
+    if (tid == 0) offs[NK] = count;
+    // the list's buckets, in order
+    unsigned nocc = 0;
+    for (int k0 = 0; k0 < NK; k0 += kStream) {
+      const int k = k0 + tid;
+      const unsigned has = k < NK && hist[k] != 0u;
+      unsigned all;
+      const unsigned at = block_prefix<unsigned, kStream>(has, all, s_part);
+      if (has) occ[nocc + at] = static_cast<unsigned short>(k);
+      nocc += all;
+    }
+    float2* staged = reinterpret_cast<float2*>(area + S.tail_waves * pitch);
+    // rounds of whole buckets that fit the staging space (all of them, mostly)
+    for (unsigned i0 = 0, i1; i0 < nocc; i0 = i1) {
+      const unsigned first = offs[occ[i0]];
+      i1 = nocc;
+      if (count - first > S.stage) {  // the last bucket that still ends inside
+        unsigned lo = i0 + 1, hi = nocc;  // [i0, lo) fits
+        while (lo < hi) {
+          const unsigned mid = (lo + hi + 1) / 2;
+          if (offs[occ[mid - 1] + 1] - first <= S.stage) lo = mid; else hi = mid - 1;
+        }
+        i1 = lo;
+      }
+      for (unsigned i = i0 + tid; i < i1; i += kStream) hist[occ[i]] = offs[occ[i]] - first;  // next free places
+      const int k0 = occ[i0], k1 = occ[i1 - 1];
+      __syncthreads();
+      sweep_list(listed, [&](float2 wp, int k) {
+        if (k >= k0 && k <= k1 && !done[k]) staged[atomicAdd(hist + k, 1u)] = wp;
+      });
+      __syncthreads();
+      if (wave < S.tail_waves) {
+        double* row = area + wave * pitch;
+        for (unsigned i = i0 + wave; i < i1; i += S.tail_waves) {
+          const int kk = wave_uniform(occ[i]), k = P.kmin + kk;
+          const unsigned b0 = wave_uniform(offs[kk]) - first, b1 = wave_uniform(offs[kk + 1]) - first;
+          if (b1 - b0 <= kSparse) {
+            for (unsigned b = b0; b < b1; ++b) add_source<Q>(L, staged[b], k, lline, P.T);
+            continue;
+          }
+          for (int c = lane; c < pitch; c += 64) row[c] = 0.0;
+          wave_lds_fence();
+          for (unsigned b = b0 + lane; b < b1; b += 64) {
+            const float2 wp = staged[b];
+            double* m = row + cell_place<Q>(lut, athr, JQ2, width, wp.y);
+            const double wd = wp.x;
+            atomicAdd(m, wd);
+            atomicAdd(m + Q * width, wd * static_cast<double>(wp.y));
+          }
+          wave_lds_fence();
+          add_bucket<Q>(L, row, M, k, lline, P.T, lane);
+          wave_lds_fence();  // the row has been read
+        }
+      }
+      __syncthreads();
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < Q; ++q) area[(wave * Q + q) * 64 + lane] = L.acc[q];
+  __syncthreads();
+  for (int r = tid; r < M; r += kStream) {
+    const int l = r / Q, q = r % Q;
+    double t = area[q * 64 + l];
+    for (int w = 1; w < kWaves; ++w) t += area[(w * Q + q) * 64 + l];  // fixed order
+    partials[static_cast<size_t>(P.rinfo[r].r) * gridDim.x + blockIdx.x] = t * P.em.rB0;  // W is chi w B0
   }
 }
 
@@ -769,21 +1317,17 @@ __global__ void __launch_bounds__(kThreads) binned_adj_table(BinnedDev P, const 
   const int k = P.kmin + kk;
   double b0 = 0.0, b1 = 0.0;
   for (int r = threadIdx.x; r < P.M; r += kThreads) {
-    double x0 = 0.0, x1 = 0.0;
-    for (int q = P.rptr[r]; q < P.rptr[r + 1]; ++q) {
-      const int e = P.rlist[q];
-      const BinInfo b = P.binfo[e];
-      const double g = static_cast<double>(gbar[e]) * P.bine[e];
-      double Cp, sp, Cm, sm;
-      seg_line(P, b, k, b.a - k, Cp, sp);
-      seg_line(P, b, k, b.a - k - 1, Cm, sm);
-      b0 += g * Cp;
-      b1 += g * sp;
-      x0 += g * (Cm - Cp);
-      x1 += g * (sm - sp);
-    }
-    d0[r] = x0;
-    d1[r] = x1;
+    const BinInfo ri = P.rinfo[r];
+    const int e = ri.r;
+    const BinInfo b{ri.A + ri.a, ri.a, r};  // exactly A_e again
+    const double g = static_cast<double>(gbar[e]) * P.bine[e];
+    double Cp, sp, Cm, sm;
+    seg_line(P, b, k, b.a - k, Cp, sp);
+    seg_line(P, b, k, b.a - k - 1, Cm, sm);
+    b0 += g * Cp;
+    b1 += g * sp;
+    d0[r] = g * (Cm - Cp);
+    d1[r] = g * (sm - sp);
   }
   base0[threadIdx.x] = b0;
   base1[threadIdx.x] = b1;
@@ -858,36 +1402,9 @@ __global__ void __launch_bounds__(STAGE ? kGather : kThreads) binned_adj_gather(
       }
     }
     __syncthreads();
-    // the window of kstage buckets with the most sampled particles (lowest start on ties)
-    const int nw = max(1, P.NK - kstage + 1);
-    unsigned best = 0;
-    int bw = 0x7fffffff;
-    for (int w = threadIdx.x; w < nw; w += NT_) {
-      unsigned c = 0;
-      for (int q = w; q < min(P.NK, w + kstage); ++q) c += hist[q];
-      if (c > best || (c == best && w < bw)) {
-        best = c;
-        bw = w;
-      }
-    }
-    // block arg-max: pack (count, -start) into 64 bits
-    unsigned long long key = (static_cast<unsigned long long>(best) << 32) |
-                             static_cast<unsigned>(0x7fffffff - min(bw, 0x7fffffff));
-#pragma unroll
-    for (int m = 1; m < 64; m <<= 1) {
-      const unsigned long long o = __shfl_xor(key, m);
-      key = o > key ? o : key;
-    }
     __shared__ unsigned long long s_key[NT_ / 64];
-    if ((threadIdx.x & 63) == 0) s_key[threadIdx.x >> 6] = key;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      unsigned long long k2 = s_key[0];
-      for (int i = 1; i < NT_ / 64; ++i) k2 = s_key[i] > k2 ? s_key[i] : k2;
-      s_w0 = 0x7fffffff - static_cast<int>(k2 & 0xffffffffu);
-    }
-    __syncthreads();  // the histogram is read: its LDS takes the rows
-    w0 = min(s_w0, nw - 1);
+    __shared__ unsigned s_part[NT_ / 64];
+    w0 = densest_window<NT_>(hist, P.NK, kstage, s_key, s_part, &s_w0);  // the histogram is read: its LDS takes the rows
     w1 = min(P.NK, w0 + kstage);
     const size_t nrow = static_cast<size_t>(w1 - w0) * M1;
     const double2* src = U + static_cast<size_t>(w0) * M1;
@@ -951,18 +1468,8 @@ static size_t subhist_smem(const SyncPlan& plan) {
          sizeof(unsigned) * (2 * kWin + 65);
 }
 
-void sync_forward_binned(const SyncPlan& plan, const ParticlesDev& D, size_t n, float* out, hipStream_t st) {
-  RGN_REQUIRE(plan.binned_ok && n < kBinnedMaxParticles, RGN_ERR_UNSUPPORTED, "plan outside the binned limits");
+static void forward_passes(const SyncPlan& plan, const ParticlesDev& D, size_t n, float* out, hipStream_t st) {
   const BinnedDev P = binned_view(plan);
-  if (plan.NK == 0 || n == 0) {
-    // a fill kernel rather than a memset node, so the call stays safe to capture
-    if (plan.nbins > 0) {
-      fill_zero<<<static_cast<unsigned>(ceil_div(plan.nbins, kThreads)), kThreads, 0, st>>>(
-        reinterpret_cast<unsigned*>(out), static_cast<size_t>(plan.nbins));
-      RGN_HIP(hipGetLastError());
-    }
-    return;
-  }
   const int G = static_cast<int>(ceil_div(n, kChunk));
   const size_t NK = plan.NK;
   const size_t M1 = plan.M + 1;
@@ -1048,6 +1555,95 @@ void sync_forward_binned(const SyncPlan& plan, const ParticlesDev& D, size_t n, 
   binned_evaluate<<<plan.nbins, kThreads, 0, st>>>(P, P0, P1, out);
   RGN_HIP(hipGetLastError());
   stage_mark(st, "binned_evaluate");
+}
+
+// LDS of a binned_stream block and what fits in it.
+static StreamShape stream_shape(const SyncPlan& plan, int Q, size_t& smem) {
+  StreamShape S{};
+  const size_t M = plan.M, NK = plan.NK;
+  const size_t rest = sizeof(double2) * kLog2Tab + sizeof(uint2) * (std::min(plan.JQ, kLutCells) + 1) +
+                      sizeof(float) * (M + 4) + sizeof(unsigned) * (2 * NK + 1) + 3 * NK;
+  const size_t lines = sizeof(double2) * (static_cast<size_t>(plan.T) + 1);
+  S.nline = plan.T + 1;
+  const size_t fixed = rest + lines + 16;
+  const size_t budget = kLdsPerCU - 512;  // the static words
+  S.area = static_cast<int>((budget - fixed) / sizeof(double)) & ~1;
+  const int pitch = 2 * Q * (plan.M / Q + 1);
+  S.rows = S.area / pitch;
+  // no round of the block's waves for a few rows
+  if (S.rows > kStream / 64 && S.rows % (kStream / 64) <= 2) S.rows -= S.rows % (kStream / 64);
+  S.rows = std::min(plan.NK, S.rows);
+  // the end of the list: a row per wave where that leaves half of the area to its sources
+  S.tail_waves = std::max(1, std::min(kStream / 64, S.area / pitch / 2));
+  S.stage = static_cast<unsigned>(S.area - S.tail_waves * pitch);  // one float2 per double
+  smem = fixed + sizeof(double) * static_cast<size_t>(S.area);
+  return S;
+}
+
+// Which form a plan's forward takes: binned_stream up to 256 bins (and a table
+// whose lines fit in its LDS), the passes above.  A row of M + 1 sub-cells
+// takes 16 (M + 1) bytes of LDS, so with more bins the window narrows and the
+// list grows.  Call times, stream against passes, p = -2.5 and -1.6:
+//   2^24 x 256:  122 and 159 against 160 and 163 us
+//   2^22 x 256:   50 and  59 against  66 and  68
+//   2^20 x 256:   33 and  42 against  46 and  48
+//   2^24 x 512:  201 and 263 against 174 and 174
+//   2^22 x 512:   84 and 106 against  67 and  66
+bool stream_form(const SyncPlan& plan) { return plan.M <= 256 && plan.T <= 1023; }
+
+void sync_forward_binned(const SyncPlan& plan, const ParticlesDev& D, size_t n, float* out, hipStream_t st) {
+  RGN_REQUIRE(plan.binned_ok && n < kBinnedMaxParticles, RGN_ERR_UNSUPPORTED, "plan outside the binned limits");
+  const BinnedDev P = binned_view(plan);
+  if (plan.NK == 0 || n == 0) {
+    // a fill kernel rather than a memset node, so the call stays safe to capture
+    if (plan.nbins > 0) {
+      fill_zero<<<static_cast<unsigned>(ceil_div(plan.nbins, kThreads)), kThreads, 0, st>>>(
+        reinterpret_cast<unsigned*>(out), static_cast<size_t>(plan.nbins));
+      RGN_HIP(hipGetLastError());
+    }
+    return;
+  }
+  if (!stream_form(plan)) {
+    forward_passes(plan, D, n, out, st);
+    return;
+  }
+  size_t smem = 0;
+  const int Q = plan.M <= 64 ? 1 : plan.M <= 128 ? 2 : 4;  // bins per lane
+  StreamShape S = stream_shape(plan, Q, smem);
+  // one block per CU
+  const size_t tiles = ceil_div(n, kStream);
+  const size_t grid = std::min<size_t>(tiles, num_cus());
+  S.cap = static_cast<unsigned>(ceil_div(tiles, grid) * kStream);
+  const size_t entries = grid * S.cap;
+  float2* wp = static_cast<float2*>(scratch(sizeof(float2) * entries, 20));
+  unsigned short* lk = static_cast<unsigned short*>(scratch(sizeof(unsigned short) * entries, 21));
+  double* partials = static_cast<double*>(scratch(sizeof(double) * plan.nbins * grid, 22));
+  const bool has_e = D.e[0] || D.e[1] || D.e[2];
+  // Particles larger than the device's last-level cache (256 MiB on MI355X)
+  // are read non-temporally: they would not be found there on the next call.
+  // Not where the arrays start inside a cache line: a line shared by two waves
+  // is then fetched twice (2^24 + 3 particles: 88 against 84 us of streaming;
+  // aligned, 77 against 82).
+  const size_t in_bytes = sizeof(float) * n * (6 + (has_e ? 3 : 0) + (D.w ? 1 : 0));
+  bool nt = in_bytes > (size_t{256} << 20);
+  for (const float* q : {D.u[0], D.u[1], D.u[2], D.e[0], D.e[1], D.e[2], D.b[0], D.b[1], D.b[2], D.w}) {
+    nt = nt && reinterpret_cast<uintptr_t>(q) % 128 == 0;
+  }
+  const unsigned nn = static_cast<unsigned>(n), g = static_cast<unsigned>(grid);
+  switch (Q * 4 + (has_e ? 2 : 0) + (nt ? 1 : 0)) {
+#define RGN_STREAM_CASE(Q_)                                                                          \
+  case Q_ * 4: binned_stream<Q_, false, false><<<g, kStream, smem, st>>>(D, nn, P, S, wp, lk, partials); break;    \
+  case Q_ * 4 + 1: binned_stream<Q_, false, true><<<g, kStream, smem, st>>>(D, nn, P, S, wp, lk, partials); break; \
+  case Q_ * 4 + 2: binned_stream<Q_, true, false><<<g, kStream, smem, st>>>(D, nn, P, S, wp, lk, partials); break; \
+  case Q_ * 4 + 3: binned_stream<Q_, true, true><<<g, kStream, smem, st>>>(D, nn, P, S, wp, lk, partials); break;
+    RGN_STREAM_CASE(1)
+    RGN_STREAM_CASE(2)
+    RGN_STREAM_CASE(4)
+#undef RGN_STREAM_CASE
+  }
+  RGN_HIP(hipGetLastError());
+  stage_mark(st, "binned_stream");
+  launch_combine(plan, partials, static_cast<int>(grid), out, st);
 }
 
 void sync_adjoint_binned(const SyncPlan& plan, const ParticlesDev& D, size_t n, const float* gbar, float* gw,

@@ -526,8 +526,7 @@ void launch_combine(const SyncPlan& plan, const double* partials, int grid, floa
 }
 
 // Automatic choice between the direct and the factorised kernels from a cost
-// model measured on MI355X (2^16 .. 2^24 particles, 32 .. 512 bins; constants
-// below).  RAGNAR_SYNC_METHOD (direct | binned) overrides the automatic choice.
+// model measured on MI355X (constants below).  RAGNAR_SYNC_METHOD (direct | binned) overrides the automatic choice.
 int resolve_method(const SyncPlan& plan, size_t n, int method, bool adjoint) {
   // the factorised kernels address particles with 32-bit byte offsets
   const bool binned_fits = plan.binned_ok && n < kBinnedMaxParticles;
@@ -537,18 +536,21 @@ int resolve_method(const SyncPlan& plan, size_t n, int method, bool adjoint) {
       if (std::string(m) == "binned" && binned_fits) return RGN_METHOD_BINNED;
     }
     if (!binned_fits) return RGN_METHOD_DIRECT;
-    // Seconds per call, fitted on MI355X to 2^16 .. 2^24 particles at 32 .. 512
-    // bins.  The pair-by-pair kernels cost per particle by NB, the number of
-    // 64-bin blocks (seconds per particle below, by NB); the factorised ones
-    // have a floor of fixed passes, then a cost per particle that hardly
-    // depends on the bin count.
-    static const double c_fwd[9] = {0, 20e-12, 26e-12, 31e-12, 36e-12, 50e-12, 65e-12, 80e-12, 94e-12};
-    static const double c_adj[9] = {0, 27e-12, 34e-12, 43e-12, 52e-12, 63e-12, 74e-12, 84e-12, 95e-12};
+    // Seconds per call, fitted on MI355X to 2^14 .. 2^24 particles of index
+    // -2.5 and -1.7 at 32 .. 512 bins.  The pair-by-pair kernels cost per
+    // particle by NB, the number of 64-bin blocks; the factorised ones a floor
+    // of fixed work, then a cost per particle that hardly depends on the bins.
+    // Forward at 256 bins, pair by pair against factorised: 2^18 22.5 / 29, 2^19
+    // 31.5 / 31, 2^20 48 / 34 us; at 512 bins 2^19 50 / 48 us.
+    static const double c_fwd[9] = {0, 21e-12, 21e-12, 26e-12, 27e-12, 31e-12, 34e-12, 44e-12, 53e-12};
+    static const double c_adj[9] = {0, 25e-12, 27e-12, 39e-12, 39e-12, 61e-12, 61e-12, 67e-12, 67e-12};
     const double nd = static_cast<double>(n);
     const int nbk = std::min(std::max(plan.NB, 1), 8);
-    const double t_direct = adjoint ? 25e-6 + nd * c_adj[nbk] : 18e-6 + nd * c_fwd[nbk];
-    const double t_binned = adjoint ? std::max(33e-6, 28e-6 + nd * 13.5e-12)
-                                    : std::max(62e-6, 35e-6 + nd * 10.1e-12);
+    const double t_direct = adjoint ? 20e-6 + nd * c_adj[nbk] : 18e-6 + nd * c_fwd[nbk];
+    const double t_fwd = !stream_form(plan) ? std::max(47e-6, 35e-6 + nd * 8.2e-12)
+                         : plan.M <= 128    ? 22e-6 + nd * 4.1e-12
+                                            : 28e-6 + nd * 5.7e-12;
+    const double t_binned = adjoint ? std::max(33e-6, 28e-6 + nd * 13.5e-12) : t_fwd;
     return t_binned < t_direct ? RGN_METHOD_BINNED : RGN_METHOD_DIRECT;
   }
   RGN_REQUIRE(method == RGN_METHOD_DIRECT || method == RGN_METHOD_BINNED, RGN_ERR_INVALID,

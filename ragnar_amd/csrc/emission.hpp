@@ -29,11 +29,11 @@ struct SyncPlan {
 
   // Factorised ("binned") form, binned.hip.  With B = k + phi (k integer) and
   // A_e = a_e + alpha_e, a source's value in bin e depends on k and on which
-  // side of alpha_e its phi lies; the sorted distinct alpha_e cut [0, 1) into
-  // M + 1 sub-cells.
+  // side of alpha_e its phi lies; the sorted alpha_e cut [0, 1) into M + 1
+  // sub-cells.
   int T = 0;                       // table nodes
   int kmin = 0, NK = 0;            // integer parts of B that can contribute
-  int M = 0;                       // distinct alpha_e
+  int M = 0;                       // live bins, one alpha_e each
   int JQ = 0;                      // cells of the sub-cell lookup grid on [0, 1)
   bool binned_ok = false;          // the plan fits the factorised kernels' limits
   std::vector<double> A;           // A_e of live bins
@@ -42,11 +42,11 @@ struct SyncPlan {
   DeviceBuffer athr;               // float[M]: smallest float above alpha[i] (so, for a float
                                    //   phi, alpha[i] < phi exactly when athr[i] <= phi)
   DeviceBuffer jlut;               // uint16[JQ]: number of alphas below q / JQ (JQ >= 8 M)
-  DeviceBuffer sublut;             // uint2[min(JQ, 2048)]: the sub-histogram's lookup cells
-  DeviceBuffer rptr;               // int[M + 1]: live bins with alpha rank r are
-  DeviceBuffer rlist;              //   rlist[rptr[r] .. rptr[r + 1]) (ascending e)
+  DeviceBuffer sublut;             // uint2[min(JQ, 2048)]: the forward pass's lookup cells
   DeviceBuffer binfo;              // BinInfo[nbins]
+  DeviceBuffer rinfo;              // BinInfo[M] by rank: (alpha_e, a_e, e)
   DeviceBuffer seg;                // SegInfo[T - 1]
+  DeviceBuffer line;               // double2[T + 1]: the segments as lines in t - s, zero at both ends
   DeviceBuffer l2tab;              // double2[256]: the factorised passes' log2 table
 };
 
@@ -92,6 +92,7 @@ void sync_forward_binned(const SyncPlan& plan, const ParticlesDev& D, size_t n, 
 void sync_adjoint_binned(const SyncPlan& plan, const ParticlesDev& D, size_t n, const float* gbar,
                          float* gw, float* const gu[3], float* const gb[3], float* const ge[3],
                          hipStream_t st);
+bool stream_form(const SyncPlan& plan);  // which factorised forward a plan takes
 int resolve_method(const SyncPlan& plan, size_t n, int method, bool adjoint);
 
 PlanDev device_view(const SyncPlan& plan);
