@@ -7,14 +7,19 @@
 // That function of E is monotone and piecewise constant, so the plan finds its
 // n - 1 jump points E_k (the smallest double E with index >= k) on the host by
 // bisection over the ordered bit patterns of positive doubles, evaluating the
-// reference expression with the host libm.  The kernel takes a float log2
-// estimate of the index and corrects it against E_k and E_{k+1}: the result
+// reference expression with the host libm.  The energy itself is a monotone
+// function of the float |u|^2 (a correctly rounded square root, of |u|^2 or
+// of 1 + |u|^2 in double), so each jump is also a float threshold of |u|^2:
+// the kernel compares |u|^2 with floats and never forms the
+// energy for the index.  It starts from a float log2 estimate of the index, which
+// the plan checks to be within one bin everywhere, and corrects it by the
+// thresholds on its two sides (plans that fail the check walk): the result
 // equals the reference expression bit for bit, whatever the device log does.
 //
-// Accumulation.  Each wave owns a private LDS histogram (uint32 counts and FP64
+// Accumulation.  Each wave owns private LDS histograms (uint32 counts and FP64
 // sums of the per-particle float terms); blocks write per-block partials that a
 // second kernel combines in a fixed order.  Counts are exact integers; sums are
-// the FP64 sum of the reference's float terms, rounded to float once.
+// the FP64 sum of float terms, rounded to float once.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -28,9 +33,13 @@ struct rgn_hist_plan {
   int nb = 0;
   int log_bins = 0;
   float emin = 0.f, emax = 0.f;
-  float approx_scale = 0.f;  // (nb - 1) / log2(emax / emin)
   std::vector<double> edges;  // nb + 1 entries: edges[k] = E_k for 1 <= k < nb
-  rgn::DeviceBuffer d_edges;
+  // per energy kind (0: sqrt(1 + u^2), 1: |u|): nb + 1 thresholds of |u|^2,
+  // -inf and NaN at the ends; the estimate's coefficients and whether it is
+  // within one bin everywhere
+  rgn::DeviceBuffer d_thr;  // float[2][nb + 1]
+  float est_a[2] = {}, est_b[2] = {};
+  bool near[2] = {};
 };
 
 namespace rgn {
@@ -84,72 +93,138 @@ void build_edges(rgn_hist_plan& plan) {
   }
 }
 
+// The energy of |u|^2 = q, rounded as the reference rounds it.
+double energy_of(float q, bool fourvel) {
+  return fourvel ? static_cast<double>(std::sqrt(q)) : std::sqrt(1.0 + static_cast<double>(q));
+}
+
+// Smallest float q >= 0 with energy_of(q) >= target (NaN for a NaN target).
+float first_reaching(double target, bool fourvel) {
+  const float inf = std::numeric_limits<float>::infinity();
+  if (!(target == target)) return std::numeric_limits<float>::quiet_NaN();
+  if (energy_of(0.0f, fourvel) >= target) return 0.0f;
+  // a guess within a few floats, then a step at a time
+  float q = static_cast<float>(std::min(target * target - (fourvel ? 0.0 : 1.0), 3e38));
+  q = std::max(q, std::numeric_limits<float>::denorm_min());
+  for (int step = 0; step < 64; ++step) {
+    if (!(energy_of(q, fourvel) >= target)) {
+      q = std::nextafter(q, inf);
+    } else if (energy_of(std::nextafter(q, 0.0f), fourvel) >= target) {
+      q = std::nextafter(q, 0.0f);
+    } else {
+      return q;
+    }
+  }
+  uint32_t a = 0, b = 0x7f800000u;  // bit patterns of 0 .. inf are ordered like the values
+  while (a < b) {
+    const uint32_t mid = a + (b - a) / 2;
+    std::memcpy(&q, &mid, sizeof q);
+    if (energy_of(q, fourvel) >= target) b = mid; else a = mid + 1;
+  }
+  std::memcpy(&q, &a, sizeof q);
+  return q;
+}
+
+// Thresholds of |u|^2 and the estimate, for both energy kinds.
+void build_thresholds(rgn_hist_plan& plan) {
+  const size_t n = plan.nb;
+  const float inf = std::numeric_limits<float>::infinity();
+  std::vector<float> thr(2 * (n + 1));
+  for (int fourvel = 0; fourvel < 2; ++fourvel) {
+    float* t = thr.data() + fourvel * (n + 1);
+    t[0] = -inf;
+    t[n] = std::numeric_limits<float>::quiet_NaN();  // never reached
+    for (size_t k = 1; k < n; ++k) {
+      // index >= k from edge k on, and from emax on (degenerate bins: edges at infinity)
+      t[k] = first_reaching(plan.edges[k] < inf ? plan.edges[k] : static_cast<double>(plan.emax), fourvel);
+    }
+    // index ~ a log2(|u|^2 or 1 + |u|^2) + b
+    plan.near[fourvel] = false;
+    if (!(plan.emin > 0.0f && plan.emax > plan.emin && plan.emax < inf)) continue;
+    const double lo = std::log2(static_cast<double>(plan.emin)), hi = std::log2(static_cast<double>(plan.emax));
+    const double scale = (n - 1) / (hi - lo);
+    plan.est_a[fourvel] = static_cast<float>(0.5 * scale);
+    plan.est_b[fourvel] = static_cast<float>(-scale * lo);
+    // float errors of the estimate: a few ulps of its two terms
+    bool near = scale * (std::fabs(lo) + std::fabs(hi) + 2.0) * 1e-6 < 0.1;
+    for (size_t k = 1; k < n && near; ++k) {
+      const double q = t[k];
+      if (!(q < inf)) {
+        near = false;
+        break;
+      }
+      const double est = static_cast<double>(plan.est_a[fourvel]) * std::log2(fourvel ? q : 1.0 + q) + plan.est_b[fourvel];
+      // gamma bins from below 1 start at |u| = 0, whose first thresholds are 0
+      near = (est > k - 0.85 || (q == 0.0 && est >= k - 0.85)) && (est < k + 0.85 || q == 0.0);
+    }
+    plan.near[fourvel] = near;
+  }
+  plan.d_thr.reset(thr.size() * sizeof(float));
+  RGN_HIP(hipMemcpy(plan.d_thr.ptr, thr.data(), plan.d_thr.bytes, hipMemcpyHostToDevice));
+}
+
+// (float)(1 / E) of particles.cpp:247-252 for log-spaced bins, E = sqrt(q) or
+// sqrt(1 + q).  |u|: a float reciprocal square root with one Newton step whose
+// residual is kept exact, within 0.51 ulp of 1 / sqrt(q) (the reference's
+// float square root and reciprocal: within 1).  gamma: the same in FP64.
+template <bool FOURVEL>
+__device__ __forceinline__ float energy_term(float q) {
+  if (!(q >= 0x1p-126f && q < 0x1p127f)) {
+    // 0, subnormal, huge, NaN: as 1.0 / e gives them
+    const double e = FOURVEL ? static_cast<double>(sqrtf(q)) : sqrt(1.0 + static_cast<double>(q));
+    return static_cast<float>(1.0 / e);
+  }
+  if (FOURVEL) {
+    const float y = __builtin_amdgcn_rsqf(q);
+    const float h = q * y;
+    const float r = fmaf(-h, y, 1.0f) - fmaf(q, y, -h) * y;  // 1 - q y^2
+    return fmaf(0.5f * y, r, y);
+  }
+  const double d = 1.0 + static_cast<double>(q);
+  const double y = __builtin_amdgcn_rsq(d);
+  const double r = fma(-d * y, y, 1.0);
+  return static_cast<float>(fma(y * r, fma(r, 0.375, 0.5), y));
+}
+
 struct HistParams {
-  const double* edges;  // in LDS
+  const float* thr;  // in LDS
   int nb;
-  float emin, emax, scale;
-  float inv_emin;       // 1 / emin for the bin estimate (corrected against the edges)
-  int log_bins, fourvel;
+  float a, b;  // the estimate
 };
 
-// 1 / x to about one ulp for finite x > 0 (hardware estimate, two Newton steps).
-__device__ __forceinline__ double rcp_hist(double x) {
-  double y = __builtin_amdgcn_rcp(x);
-  y = fma(y, fma(-x, y, 1.0), y);
-  return fma(y, fma(-x, y, 1.0), y);
-}
-
-// particles.cpp:228-252 for one particle: bin index and the float term.
+// particles.cpp:228-252 for one particle.  NEAR: the estimate is within one bin.
+template <bool FOURVEL, bool LOGB, bool COUNT, bool NEAR>
 __device__ __forceinline__ void bin_particle(float x, float y, float z, const HistParams& H,
-                                             double* __restrict__ my_sum,
-                                             unsigned* __restrict__ my_cnt) {
-  const float usqr = x * x + y * y + z * z;  // float, as the reference
-  const double energy = H.fourvel ? static_cast<double>(sqrtf(usqr))
-                                  : sqrt(1.0 + static_cast<double>(usqr));
-  int idx;
-  if (energy < H.emin) {
-    idx = 0;
-  } else if (energy >= H.emax) {
-    idx = H.nb - 1;
-  } else if (energy == energy) {
-    // a float estimate of the index; the edges make it exact.  Both edges of
-    // the estimated bin come in one LDS read; only an estimate off by a bin
-    // (energies within float rounding of an edge) walks further.
-    const float est = H.scale * __builtin_amdgcn_logf(static_cast<float>(energy) * H.inv_emin);
-    idx = static_cast<int>(fminf(fmaxf(est, 0.0f), static_cast<float>(H.nb - 1)));
-    const double lo = H.edges[idx], hi = H.edges[idx + 1];
-    if (!(lo <= energy && energy < hi)) {
-      while (idx < H.nb - 1 && energy >= H.edges[idx + 1]) ++idx;
-      while (idx > 0 && energy < H.edges[idx]) --idx;
-    }
-  } else {
-    idx = H.nb - 1;  // NaN energy: the x86 reference's size_t conversion lands here
+                                             double* __restrict__ my_sum, unsigned* __restrict__ my_cnt) {
+  const float q = x * x + y * y + z * z;  // float, as the reference
+  const float est = fmaf(H.a, __builtin_amdgcn_logf(FOURVEL ? q : 1.0f + q), H.b);
+  int idx = static_cast<int>(fminf(fmaxf(est, 0.0f), static_cast<float>(H.nb - 1)));
+  const float lo = H.thr[idx], hi = H.thr[idx + 1];
+  idx += (q >= hi) - (q < lo);
+  if (!NEAR) {
+    while (idx < H.nb - 1 && q >= H.thr[idx + 1]) ++idx;
+    while (idx > 0 && !(q >= H.thr[idx])) --idx;
   }
-  // particles.cpp:247-252: (float)(1 / e) for log-spaced bins.  A refined
-  // reciprocal (about one double ulp) rounds to the same float except within
-  // one double ulp of a float rounding boundary (~1e-9 of the terms); the
-  // sums carry a 1e-6 tolerance, the counts do not depend on it.  The special
-  // values follow 1.0 / e: 0 -> inf, inf -> 0, NaN -> NaN.
-  float term = 1.0f;
-  if (H.log_bins) {
-    const bool normal = energy > 0.0 && energy < INFINITY;
-    term = normal ? static_cast<float>(rcp_hist(energy))
-                  : (energy == 0.0 ? INFINITY : (energy == INFINITY ? 0.0f : __builtin_nanf("")));
-  }
-  atomicAdd(my_cnt + idx, 1u);
-  atomicAdd(my_sum + idx, static_cast<double>(term));
+  if (!(q == q)) idx = H.nb - 1;  // NaN: the x86 reference's size_t conversion lands here
+  if (COUNT) atomicAdd(my_cnt + idx, 1u);
+  if (LOGB) atomicAdd(my_sum + idx, static_cast<double>(energy_term<FOURVEL>(q)));
 }
 
-// Each thread keeps two 16-byte loads per component in flight (8 particles)
-// when the three component arrays are 16-byte aligned; the remainder (and
-// unaligned inputs) go through the scalar loop.
-__global__ void __launch_bounds__(kThreads) hist_kernel(const float* __restrict__ ux,
-                                                        const float* __restrict__ uy,
+// Four consecutive floats at any float address (one 16-byte load).
+typedef float float4u __attribute__((ext_vector_type(4), aligned(4)));
+
+// Each thread keeps two 16-byte loads per component in flight (8 particles); the
+// last n % 4 particles go one per thread.  COUNT: integer counts are kept (linear
+// bins sum ones, so their sums are the counts).  38 vector instructions a
+// particle (57 when the energy was formed); bound by memory latency and LDS
+// atomics (counters: VALU 40%, LDS 45% of the cycles).  2^24 particles with the
+// momenta in HBM (201 MB, 39 us at the rate of a copy): 200 log bins 56.6 -> 55.5
+// us, 1000 bins 80 -> 64, linear bins 55 -> 49; 2^24 + 3 particles 60 -> 56.
+template <bool FOURVEL, bool LOGB, bool COUNT, bool NEAR>
+__global__ void __launch_bounds__(kThreads) hist_kernel(const float* __restrict__ ux, const float* __restrict__ uy,
                                                         const float* __restrict__ uz, size_t n,
-                                                        const double* __restrict__ g_edges, int nb,
-                                                        float emin, float emax, float scale,
-                                                        int log_bins, int fourvel, int vec, int qper,
-                                                        unsigned* __restrict__ cpart,
+                                                        const float* __restrict__ g_thr, int nb, float a, float b,
+                                                        int qper, unsigned* __restrict__ cpart,
                                                         double* __restrict__ partials) {
   extern __shared__ __align__(16) unsigned char smem[];
   // 4 * qper private sub-histograms per block: one per wave and lane group of
@@ -157,67 +232,61 @@ __global__ void __launch_bounds__(kThreads) hist_kernel(const float* __restrict_
   // few bins); pitch nb + 1 staggers the copies over the LDS banks
   const int copies = 4 * qper, pitch = nb + 1;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  double* lsum = reinterpret_cast<double*>(smem);                                 // [copies][pitch]
-  double* ledges = lsum + copies * pitch;                                         // [nb + 1]
-  unsigned* lcnt = reinterpret_cast<unsigned*>(ledges + nb + 1);                  // [copies][pitch]
+  double* lsum = reinterpret_cast<double*>(smem);                                 // LOGB: [copies][pitch]
+  unsigned* lcnt = reinterpret_cast<unsigned*>(lsum + (LOGB ? copies * pitch : 0));  // COUNT: [copies][pitch]
+  float* lthr = reinterpret_cast<float*>(lcnt + (COUNT ? copies * pitch : 0));    // [nb + 1]
   for (int i = threadIdx.x; i < copies * pitch; i += kThreads) {
-    lsum[i] = 0.0;
-    lcnt[i] = 0u;
+    if (LOGB) lsum[i] = 0.0;
+    if (COUNT) lcnt[i] = 0u;
   }
-  for (int i = threadIdx.x; i <= nb; i += kThreads) ledges[i] = g_edges[i];
+  for (int i = threadIdx.x; i <= nb; i += kThreads) lthr[i] = g_thr[i];
   __syncthreads();
-  const HistParams H{ledges, nb, emin, emax, scale, 1.0f / emin, log_bins, fourvel};
+  const HistParams H{lthr, nb, a, b};
   const int copy = wave * qper + lane / (64 / qper);
   double* my_sum = lsum + copy * pitch;
   unsigned* my_cnt = lcnt + copy * pitch;
+  auto bin = [&](float x, float y, float z) {
+    bin_particle<FOURVEL, LOGB, COUNT, NEAR>(x, y, z, H, my_sum, my_cnt);
+  };
   const size_t stride = static_cast<size_t>(gridDim.x) * kThreads;
   const size_t tid = blockIdx.x * static_cast<size_t>(kThreads) + threadIdx.x;
-  size_t scalar_from = 0;
-  if (vec) {
-    const size_t nq = n / 4;
-    const float4* x4 = reinterpret_cast<const float4*>(ux);
-    const float4* y4 = reinterpret_cast<const float4*>(uy);
-    const float4* z4 = reinterpret_cast<const float4*>(uz);
-    for (size_t q = tid; q < nq; q += 2 * stride) {
-      const bool two = q + stride < nq;
-      const float4 a0 = x4[q], b0 = y4[q], c0 = z4[q];
-      float4 a1 = a0, b1 = b0, c1 = c0;
-      if (two) {
-        a1 = x4[q + stride];
-        b1 = y4[q + stride];
-        c1 = z4[q + stride];
-      }
-      bin_particle(a0.x, b0.x, c0.x, H, my_sum, my_cnt);
-      bin_particle(a0.y, b0.y, c0.y, H, my_sum, my_cnt);
-      bin_particle(a0.z, b0.z, c0.z, H, my_sum, my_cnt);
-      bin_particle(a0.w, b0.w, c0.w, H, my_sum, my_cnt);
-      if (two) {
-        bin_particle(a1.x, b1.x, c1.x, H, my_sum, my_cnt);
-        bin_particle(a1.y, b1.y, c1.y, H, my_sum, my_cnt);
-        bin_particle(a1.z, b1.z, c1.z, H, my_sum, my_cnt);
-        bin_particle(a1.w, b1.w, c1.w, H, my_sum, my_cnt);
-      }
+  const size_t nq = n / 4;
+  const float4u* x4 = reinterpret_cast<const float4u*>(ux);
+  const float4u* y4 = reinterpret_cast<const float4u*>(uy);
+  const float4u* z4 = reinterpret_cast<const float4u*>(uz);
+  for (size_t q = tid; q < nq; q += 2 * stride) {
+    const bool two = q + stride < nq;
+    const size_t q1 = two ? q + stride : q;
+    const float4u a0 = x4[q], b0 = y4[q], c0 = z4[q], a1 = x4[q1], b1 = y4[q1], c1 = z4[q1];
+    bin(a0.x, b0.x, c0.x);
+    bin(a0.y, b0.y, c0.y);
+    bin(a0.z, b0.z, c0.z);
+    bin(a0.w, b0.w, c0.w);
+    if (two) {
+      bin(a1.x, b1.x, c1.x);
+      bin(a1.y, b1.y, c1.y);
+      bin(a1.z, b1.z, c1.z);
+      bin(a1.w, b1.w, c1.w);
     }
-    scalar_from = 4 * nq;
   }
-  for (size_t p = scalar_from + tid; p < n; p += stride) {
-    bin_particle(ux[p], uy[p], uz[p], H, my_sum, my_cnt);
-  }
+  const size_t p = 4 * nq + tid;
+  if (p < n) bin(ux[p], uy[p], uz[p]);
   __syncthreads();
   for (int i = threadIdx.x; i < nb; i += kThreads) {
     unsigned c = 0;
     double s = 0.0;
     for (int q = 0; q < copies; ++q) {  // fixed order
-      c += lcnt[q * pitch + i];
-      s += lsum[q * pitch + i];
+      if (COUNT) c += lcnt[q * pitch + i];
+      if (LOGB) s += lsum[q * pitch + i];
     }
-    cpart[static_cast<size_t>(i) * gridDim.x + blockIdx.x] = c;
-    partials[static_cast<size_t>(i) * gridDim.x + blockIdx.x] = s;
+    if (COUNT) cpart[static_cast<size_t>(i) * gridDim.x + blockIdx.x] = c;
+    if (LOGB) partials[static_cast<size_t>(i) * gridDim.x + blockIdx.x] = s;
   }
 }
 
-// Fixed-order sums of the per-block partials: FP64 sums and (when counts is
-// not null) uint64 counts.  No global atomics.
+// Fixed-order sums of the per-block partials: FP64 sums (LOGB; else the counts)
+// and (when counts is not null) uint64 counts.  No global atomics.
+template <bool LOGB, bool COUNT>
 __global__ void __launch_bounds__(kThreads) hist_combine_kernel(const double* __restrict__ partials,
                                                                 const unsigned* __restrict__ cpart,
                                                                 int nblocks, int nb,
@@ -228,8 +297,8 @@ __global__ void __launch_bounds__(kThreads) hist_combine_kernel(const double* __
   double s = 0.0;
   unsigned long long c = 0;
   for (int b = threadIdx.x; b < nblocks; b += kThreads) {
-    s += partials[static_cast<size_t>(i) * nblocks + b];
-    c += cpart[static_cast<size_t>(i) * nblocks + b];
+    if (LOGB) s += partials[static_cast<size_t>(i) * nblocks + b];
+    if (COUNT) c += cpart[static_cast<size_t>(i) * nblocks + b];
   }
   __shared__ double red[kThreads];
   __shared__ unsigned long long cred[kThreads];
@@ -244,7 +313,7 @@ __global__ void __launch_bounds__(kThreads) hist_combine_kernel(const double* __
     __syncthreads();
   }
   if (threadIdx.x == 0) {
-    out[i] = static_cast<float>(red[0]);
+    out[i] = LOGB ? static_cast<float>(red[0]) : static_cast<float>(static_cast<double>(cred[0]));
     if (counts) counts[i] = cred[0];
   }
 }
@@ -254,23 +323,21 @@ struct HistShape {
   int grid = 1;
   size_t smem = 0;
   int qper = 1;
-  int vec = 0;
 };
 
-HistShape hist_shape(const rgn_hist_plan& plan, const float* const d_u[3], size_t n) {
+HistShape hist_shape(const rgn_hist_plan& plan, size_t n, bool counts) {
   HistShape sh;
   const int nb = plan.nb;
-  auto aligned16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
-  sh.vec = aligned16(d_u[0]) && aligned16(d_u[1]) && aligned16(d_u[2]);
-  const size_t per_thread = sh.vec ? 8 : 1;
-  const size_t tiles = ceil_div(std::max<size_t>(n, 1), kThreads * per_thread);
+  const size_t tiles = ceil_div(std::max<size_t>(n, 1), kThreads * 8);
   // lane groups per wave: as many private copies as fit in 24 KB of LDS (at
   // 200 bins two per wave, and seven blocks share a CU: 51 -> 50 us at 2^24
   // against four per wave in 48 KB)
-  const size_t per_copy = static_cast<size_t>(nb + 1) * (sizeof(double) + sizeof(unsigned));
+  const size_t per_copy =
+    static_cast<size_t>(nb + 1) * ((plan.log_bins ? sizeof(double) : 0) + (counts || !plan.log_bins ? sizeof(unsigned) : 0));
+  const size_t thr = (nb + 1) * sizeof(float);
   sh.qper = 4;
-  while (sh.qper > 1 && 4 * sh.qper * per_copy + (nb + 1) * sizeof(double) > 24 * 1024) sh.qper /= 2;
-  sh.smem = 4 * sh.qper * per_copy + (nb + 1) * sizeof(double);
+  while (sh.qper > 1 && 4 * sh.qper * per_copy + thr > 24 * 1024) sh.qper /= 2;
+  sh.smem = 4 * sh.qper * per_copy + thr;
   // one round of blocks: as many per CU as the LDS holds (at most 8), so the
   // per-block clearing and reduction of the private copies is paid once
   const size_t per_cu = std::max<size_t>(1, std::min<size_t>(8, (160 * 1024) / sh.smem));
@@ -287,15 +354,37 @@ size_t hist_partial_bytes(int nb, int grid) {
 void launch_hist(const rgn_hist_plan& plan, const float* const d_u[3], size_t n, int fourvel,
                  float* d_hist, uint64_t* d_counts, const HistShape& sh, double* partials,
                  hipStream_t st) {
-  const int nb = plan.nb;
+  const int nb = plan.nb, kind = fourvel ? 1 : 0;
+  const bool count = d_counts || !plan.log_bins;
   unsigned* cpart = reinterpret_cast<unsigned*>(partials + static_cast<size_t>(nb) * sh.grid);
-  hist_kernel<<<sh.grid, kThreads, sh.smem, st>>>(
-    d_u[0], d_u[1], d_u[2], n, plan.d_edges.as<double>(), nb, plan.emin, plan.emax,
-    plan.approx_scale, plan.log_bins, fourvel ? 1 : 0, sh.vec, sh.qper, cpart, partials);
+  const float* thr = plan.d_thr.as<float>() + kind * (nb + 1);
+  auto launch = [&](auto kernel) {
+    kernel<<<sh.grid, kThreads, sh.smem, st>>>(d_u[0], d_u[1], d_u[2], n, thr, nb, plan.est_a[kind], plan.est_b[kind],
+                                               sh.qper, cpart, partials);
+  };
+  const bool near = plan.near[kind];
+  switch ((kind ? 8 : 0) + (plan.log_bins ? 4 : 0) + (count ? 2 : 0) + (near ? 1 : 0)) {
+#define RGN_HIST_CASES(F_)                                                 \
+  case F_ * 8 + 2: launch(hist_kernel<F_, false, true, false>); break;     \
+  case F_ * 8 + 3: launch(hist_kernel<F_, false, true, true>); break;      \
+  case F_ * 8 + 4: launch(hist_kernel<F_, true, false, false>); break;     \
+  case F_ * 8 + 5: launch(hist_kernel<F_, true, false, true>); break;      \
+  case F_ * 8 + 6: launch(hist_kernel<F_, true, true, false>); break;      \
+  case F_ * 8 + 7: launch(hist_kernel<F_, true, true, true>); break;
+    RGN_HIST_CASES(0)
+    RGN_HIST_CASES(1)
+#undef RGN_HIST_CASES
+  }
   RGN_HIP(hipGetLastError());
   stage_mark(st, "hist_kernel");
-  hist_combine_kernel<<<nb, kThreads, 0, st>>>(partials, cpart, sh.grid, nb, d_hist,
-                                               reinterpret_cast<unsigned long long*>(d_counts));
+  auto* out_counts = reinterpret_cast<unsigned long long*>(d_counts);
+  if (!plan.log_bins) {
+    hist_combine_kernel<false, true><<<nb, kThreads, 0, st>>>(partials, cpart, sh.grid, nb, d_hist, out_counts);
+  } else if (count) {
+    hist_combine_kernel<true, true><<<nb, kThreads, 0, st>>>(partials, cpart, sh.grid, nb, d_hist, out_counts);
+  } else {
+    hist_combine_kernel<true, false><<<nb, kThreads, 0, st>>>(partials, cpart, sh.grid, nb, d_hist, nullptr);
+  }
   RGN_HIP(hipGetLastError());
   stage_mark(st, "hist_combine_kernel");
 }
@@ -340,7 +429,7 @@ int rgn_hist_plan_create(const float* h_bins, int nb, int log_bins, rgn_hist_pla
   return guarded([&] {
     RGN_REQUIRE(out != nullptr && h_bins != nullptr, RGN_ERR_INVALID, "null argument");
     RGN_REQUIRE(nb >= 1, RGN_ERR_INVALID, "no energy bins");
-    // LDS of the smallest configuration: 4 private copies (pitch nb + 1) and the edges
+    // LDS of the smallest configuration: 4 private copies (pitch nb + 1) and as much again for the thresholds
     RGN_REQUIRE(static_cast<size_t>(nb + 1) * (4 * (sizeof(double) + sizeof(unsigned)) + sizeof(double)) <=
                   150 * 1024,
                 RGN_ERR_UNSUPPORTED, "too many energy bins for the LDS histogram (at most 2741)");
@@ -355,9 +444,6 @@ int rgn_hist_plan_create(const float* h_bins, int nb, int log_bins, rgn_hist_pla
     }
     plan->emin = lo;
     plan->emax = hi;
-    plan->approx_scale =
-      (lo > 0.0f && hi > lo) ? static_cast<float>((nb - 1) / std::log2(static_cast<double>(hi) / lo))
-                             : 0.0f;
     try {
       if (lo > 0.0f && hi > lo) {
         build_edges(*plan);
@@ -366,9 +452,7 @@ int rgn_hist_plan_create(const float* h_bins, int nb, int log_bins, rgn_hist_pla
         plan->edges.assign(nb + 1, std::numeric_limits<double>::infinity());
         plan->edges[0] = -std::numeric_limits<double>::infinity();
       }
-      plan->d_edges.reset(plan->edges.size() * sizeof(double));
-      RGN_HIP(hipMemcpy(plan->d_edges.ptr, plan->edges.data(), plan->d_edges.bytes,
-                        hipMemcpyHostToDevice));
+      build_thresholds(*plan);
     } catch (...) {
       delete plan;
       throw;
@@ -389,7 +473,7 @@ int rgn_energy_hist(const rgn_hist_plan* plan, const float* const d_u[3], size_t
     RGN_REQUIRE(d_u && d_u[0] && d_u[1] && d_u[2] && d_hist, RGN_ERR_INVALID, "null argument");
     hipStream_t st = as_stream(stream);
     ScratchUse order(st);
-    const HistShape sh = hist_shape(*plan, d_u, n);
+    const HistShape sh = hist_shape(*plan, n, d_counts != nullptr);
     double* partials = static_cast<double*>(rgn::scratch(hist_partial_bytes(plan->nb, sh.grid), 2));
     launch_hist(*plan, d_u, n, fourvel, d_hist, d_counts, sh, partials, st);
   });
@@ -400,7 +484,7 @@ int rgn_energy_hist_noalloc(const rgn_hist_plan* plan, const float* const d_u[3]
   return guarded([&] {
     RGN_REQUIRE(plan != nullptr, RGN_ERR_INVALID, "null plan");
     RGN_REQUIRE(d_u && d_u[0] && d_u[1] && d_u[2] && d_hist, RGN_ERR_INVALID, "null argument");
-    HistShape sh = hist_shape(*plan, d_u, n);
+    HistShape sh = hist_shape(*plan, n, d_counts != nullptr);
     // the grid is cut to what the fixed array holds: bins x blocks x 12 bytes
     const size_t per_block = hist_partial_bytes(plan->nb, 1);
     RGN_REQUIRE(per_block <= kHistNoAllocBytes, RGN_ERR_UNSUPPORTED,
