@@ -53,7 +53,7 @@ constexpr int kLutCells = 2048;  // sub-cell lookup cells of the forward pass
 constexpr int kLog2Tab = 256;    // entries of the factorised passes' log2 table
 }  // namespace
 
-void build_binned_tables(SyncPlan& plan, const std::vector<float>& xs, const std::vector<float>& ys) {
+void build_binned_tables(SyncPlan& plan, const std::vector<float>& xs, const std::vector<float>& ys, PlanUpload& up) {
   const int T = plan.T;
   std::vector<double> alphas;
   for (int e = 0; e < plan.nbins; ++e) {
@@ -108,20 +108,15 @@ void build_binned_tables(SyncPlan& plan, const std::vector<float>& xs, const std
   }
   plan.binned_ok = plan.M <= kBinnedMaxM && plan.NK <= kBinnedMaxNK;
 
-  plan.alpha.reset(std::max<size_t>(1, alphas.size()) * sizeof(double));
-  plan.athr.reset(std::max<size_t>(1, alphas.size()) * sizeof(float));
   std::vector<float> athr(alphas.size());
   for (size_t i = 0; i < alphas.size(); ++i) {
     float f = static_cast<float>(alphas[i]);
     if (static_cast<double>(f) <= alphas[i]) f = std::nextafter(f, 2.0f);
     athr[i] = f;
   }
-  if (!alphas.empty()) {
-    RGN_HIP(hipMemcpy(plan.alpha.ptr, alphas.data(), alphas.size() * sizeof(double), hipMemcpyHostToDevice));
-    RGN_HIP(hipMemcpy(plan.athr.ptr, athr.data(), athr.size() * sizeof(float), hipMemcpyHostToDevice));
-  }
-  plan.jlut.reset(jlut.size() * sizeof(unsigned short));
-  RGN_HIP(hipMemcpy(plan.jlut.ptr, jlut.data(), plan.jlut.bytes, hipMemcpyHostToDevice));
+  up.add(plan.alpha, alphas);
+  up.add(plan.athr, athr);
+  up.add(plan.jlut, jlut);
   {
     // the forward pass's lookup cells c of [c / JQ2, (c + 1) / JQ2): the alphas
     // below the cell, a flag for cells holding two alphas or more, and the
@@ -136,27 +131,24 @@ void build_binned_tables(SyncPlan& plan, const std::vector<float>& xs, const std
       std::memcpy(&bits, &thr, sizeof(bits));
       lut[c] = make_uint2(j0 | (jn - j0 >= 2 ? 0x10000u : 0u), bits);
     }
-    plan.sublut.reset(lut.size() * sizeof(uint2));
-    RGN_HIP(hipMemcpy(plan.sublut.ptr, lut.data(), plan.sublut.bytes, hipMemcpyHostToDevice));
+    up.add(plan.sublut, lut);
   }
-  plan.binfo.reset(bi.size() * sizeof(BinInfo));
-  RGN_HIP(hipMemcpy(plan.binfo.ptr, bi.data(), bi.size() * sizeof(BinInfo), hipMemcpyHostToDevice));
-  plan.rinfo.reset(ri.size() * sizeof(BinInfo));
-  RGN_HIP(hipMemcpy(plan.rinfo.ptr, ri.data(), plan.rinfo.bytes, hipMemcpyHostToDevice));
-  plan.seg.reset(seg.size() * sizeof(SegInfo));
-  RGN_HIP(hipMemcpy(plan.seg.ptr, seg.data(), seg.size() * sizeof(SegInfo), hipMemcpyHostToDevice));
-  plan.line.reset(line.size() * sizeof(double2));
-  RGN_HIP(hipMemcpy(plan.line.ptr, line.data(), plan.line.bytes, hipMemcpyHostToDevice));
+  up.add(plan.binfo, bi);
+  up.add(plan.rinfo, ri);
+  up.add(plan.seg, seg);
+  up.add(plan.line, line);
   {
     // log2 table (log2_tab): entry i holds 2 inv_i and -log2 inv_i, inv_i = RN(1 / c_i),
     // c_i = 1 + (i + 1/2) / 256, the logarithm in long double
-    std::vector<double2> l2(kLog2Tab);
-    for (int i = 0; i < kLog2Tab; ++i) {
-      const double inv = 1.0 / (1.0 + (i + 0.5) / kLog2Tab);
-      l2[i] = make_double2(2.0 * inv, static_cast<double>(-std::log2(static_cast<long double>(inv))));
-    }
-    plan.l2tab.reset(l2.size() * sizeof(double2));
-    RGN_HIP(hipMemcpy(plan.l2tab.ptr, l2.data(), plan.l2tab.bytes, hipMemcpyHostToDevice));
+    static const std::vector<double2> l2 = [] {
+      std::vector<double2> t(kLog2Tab);
+      for (int i = 0; i < kLog2Tab; ++i) {
+        const double inv = 1.0 / (1.0 + (i + 0.5) / kLog2Tab);
+        t[i] = make_double2(2.0 * inv, static_cast<double>(-std::log2(static_cast<long double>(inv))));
+      }
+      return t;
+    }();
+    up.add(plan.l2tab, l2);
   }
 }
 

@@ -34,10 +34,11 @@ constexpr int kMaxTableEntries = 12288;  // 96 KiB of (c, s) pairs in LDS
 
 // ---------------------------------------------------------------------------
 // Exact-product representation of the per-bin coordinate U_e: search c near 1
-// such that S = float(U / c) makes c * S closest to U.  One wave per bin.
+// such that S = float(U / c) makes c * S closest to U (the smallest |k| among
+// equals).  One block per bin, sixteen candidates a thread.
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(64) product_pair_kernel(const double* __restrict__ U,
-                                                          float2* __restrict__ out, int n) {
+__global__ void __launch_bounds__(kThreads) product_pair_kernel(const double* __restrict__ U,
+                                                                float2* __restrict__ out, int n) {
   const int e = blockIdx.x;
   if (e >= n) return;
   const double target = U[e];
@@ -45,7 +46,7 @@ __global__ void __launch_bounds__(64) product_pair_kernel(const double* __restri
   int best_k = 0;
   float best_c = 1.0f, best_s = static_cast<float>(target);
   // k in [-2047, 2047]: c = 1 + k 2^-23 above 1, 1 + k 2^-24 below 1
-  for (int k = static_cast<int>(threadIdx.x) - 2047; k <= 2047; k += 64) {
+  for (int k = static_cast<int>(threadIdx.x) - 2047; k <= 2047; k += kThreads) {
     const float c = (k >= 0) ? 1.0f + static_cast<float>(k) * 0x1p-23f
                              : 1.0f + static_cast<float>(k) * 0x1p-24f;
     const float s = static_cast<float>(target / static_cast<double>(c));
@@ -57,20 +58,37 @@ __global__ void __launch_bounds__(64) product_pair_kernel(const double* __restri
       best_s = s;
     }
   }
-  __shared__ double rs[64];
-  __shared__ int ks[64];
-  rs[threadIdx.x] = best_r;
-  ks[threadIdx.x] = best_k;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int arg = 0;
-    for (int i = 1; i < 64; ++i) {
-      if (rs[i] < rs[arg] || (rs[i] == rs[arg] && abs(ks[i]) < abs(ks[arg]))) arg = i;
+  // the winner of the wave, then of the block; one order over (r, |k|, k)
+  auto better = [](double r, int k, double r0, int k0) {
+    return r < r0 || (r == r0 && (abs(k) < abs(k0) || (abs(k) == abs(k0) && k < k0)));
+  };
+  double r0 = best_r;
+  int k0 = best_k;
+#pragma unroll
+  for (int m = 32; m > 0; m >>= 1) {
+    const double r = __shfl_xor(r0, m);
+    const int k = __shfl_xor(k0, m);
+    if (better(r, k, r0, k0)) {
+      r0 = r;
+      k0 = k;
     }
-    ks[0] = arg;
+  }
+  __shared__ double rs[kThreads / 64];
+  __shared__ int ks[kThreads / 64];
+  if ((threadIdx.x & 63) == 0) {
+    rs[threadIdx.x >> 6] = r0;
+    ks[threadIdx.x >> 6] = k0;
   }
   __syncthreads();
-  if (static_cast<int>(threadIdx.x) == ks[0]) out[e] = make_float2(best_c, best_s);
+  for (int w = 0; w < kThreads / 64; ++w) {
+    if (better(rs[w], ks[w], r0, k0)) {
+      r0 = rs[w];
+      k0 = ks[w];
+    }
+  }
+  // k picks the thread: its candidates are k0 modulo the block (nothing found,
+  // for a U that is not finite: thread 2047 % kThreads writes its first guess)
+  if ((k0 + 2047) % kThreads == static_cast<int>(threadIdx.x)) out[e] = make_float2(best_c, best_s);
 }
 
 struct ParticleSourceFn {
@@ -418,8 +436,8 @@ void build_sync_plan(SyncPlan& plan, const rgn_ftable* table, const float* h_bin
       tab[j] = make_float2(static_cast<float>(yb - ub * s), static_cast<float>(s));
     }
   }
-  plan.table.reset(plan.TP * sizeof(float2));
-  RGN_HIP(hipMemcpy(plan.table.ptr, tab.data(), plan.table.bytes, hipMemcpyHostToDevice));
+  PlanUpload up;
+  up.add(plan.table, tab);
 
   // Per-bin coordinates; dead bins and padding lanes reuse the lowest live A.
   plan.NB = static_cast<int>(ceil_div(nbins, 64));
@@ -436,14 +454,9 @@ void build_sync_plan(SyncPlan& plan, const rgn_ftable* table, const float* h_bin
       bine[e] = h_bins[e];
     }
   }
-  DeviceBuffer dU(alloc * sizeof(double));
-  RGN_HIP(hipMemcpy(dU.ptr, U.data(), dU.bytes, hipMemcpyHostToDevice));
-  plan.bincs.reset(alloc * sizeof(float2));
-  product_pair_kernel<<<alloc, 64>>>(dU.as<double>(), plan.bincs.as<float2>(), alloc);
-  RGN_HIP(hipGetLastError());
-  plan.bine.reset(alloc * sizeof(float));
-  RGN_HIP(hipMemcpy(plan.bine.ptr, bine.data(), plan.bine.bytes, hipMemcpyHostToDevice));
-  RGN_HIP(hipDeviceSynchronize());  // dU goes out of scope
+  up.add(plan.coord, U);
+  up.add(plan.bincs, static_cast<const float2*>(nullptr), alloc);
+  up.add(plan.bine, bine);
 
   plan.win_lo = amin - plan.Z;
   plan.win_hi = amax;
@@ -458,7 +471,11 @@ void build_sync_plan(SyncPlan& plan, const rgn_ftable* table, const float* h_bin
   plan.T = T;
   plan.A = A;
   plan.live = live;
-  build_binned_tables(plan, xs, y);
+  build_binned_tables(plan, xs, y, up);
+  up.finish(plan.device);
+  product_pair_kernel<<<alloc, kThreads>>>(plan.coord.as<double>(), plan.bincs.as<float2>(), alloc);
+  RGN_HIP(hipGetLastError());
+  RGN_HIP(hipDeviceSynchronize());  // the plan may be used on any stream from here on
 }
 
 PlanDev device_view(const SyncPlan& plan) {

@@ -23,9 +23,11 @@ struct SyncPlan {
   float v_safe = 0.f;
   float ublk[8] = {};       // largest U_e of the live bins of each 64-bin block
   std::vector<float> bins;  // host copy of the photon bins
-  DeviceBuffer table;       // float2[TP]
-  DeviceBuffer bincs;       // float2[nbins_pad]
-  DeviceBuffer bine;        // float[nbins_pad]
+  DeviceBuffer device;      // the arrays below, one after another
+  PlanArray table;          // float2[TP]
+  PlanArray coord;          // double[...]: U_e, which bincs is made from
+  PlanArray bincs;       // float2[nbins_pad]
+  PlanArray bine;        // float[nbins_pad]
 
   // Factorised ("binned") form, binned.hip.  With B = k + phi (k integer) and
   // A_e = a_e + alpha_e, a source's value in bin e depends on k and on which
@@ -38,16 +40,16 @@ struct SyncPlan {
   bool binned_ok = false;          // the plan fits the factorised kernels' limits
   std::vector<double> A;           // A_e of live bins
   std::vector<char> live;          // bin e has e_e > 0
-  DeviceBuffer alpha;              // double[M], sorted
-  DeviceBuffer athr;               // float[M]: smallest float above alpha[i] (so, for a float
+  PlanArray alpha;              // double[M], sorted
+  PlanArray athr;               // float[M]: smallest float above alpha[i] (so, for a float
                                    //   phi, alpha[i] < phi exactly when athr[i] <= phi)
-  DeviceBuffer jlut;               // uint16[JQ]: number of alphas below q / JQ (JQ >= 8 M)
-  DeviceBuffer sublut;             // uint2[min(JQ, 2048)]: the forward pass's lookup cells
-  DeviceBuffer binfo;              // BinInfo[nbins]
-  DeviceBuffer rinfo;              // BinInfo[M] by rank: (alpha_e, a_e, e)
-  DeviceBuffer seg;                // SegInfo[T - 1]
-  DeviceBuffer line;               // double2[T + 1]: the segments as lines in t - s, zero at both ends
-  DeviceBuffer l2tab;              // double2[256]: the factorised passes' log2 table
+  PlanArray jlut;               // uint16[JQ]: number of alphas below q / JQ (JQ >= 8 M)
+  PlanArray sublut;             // uint2[min(JQ, 2048)]: the forward pass's lookup cells
+  PlanArray binfo;              // BinInfo[nbins]
+  PlanArray rinfo;              // BinInfo[M] by rank: (alpha_e, a_e, e)
+  PlanArray seg;                // SegInfo[T - 1]
+  PlanArray line;               // double2[T + 1]: the segments as lines in t - s, zero at both ends
+  PlanArray l2tab;              // double2[256]: the factorised passes' log2 table
 };
 
 // The plan's emission constants with the correctly rounded reciprocals of the
@@ -86,7 +88,7 @@ struct SegInfo {
   double tau, y, sigma;
 };
 
-void build_binned_tables(SyncPlan& plan, const std::vector<float>& xs, const std::vector<float>& ys);
+void build_binned_tables(SyncPlan& plan, const std::vector<float>& xs, const std::vector<float>& ys, PlanUpload& up);
 void sync_forward_binned(const SyncPlan& plan, const ParticlesDev& D, size_t n, float* out,
                          hipStream_t st);
 void sync_adjoint_binned(const SyncPlan& plan, const ParticlesDev& D, size_t n, const float* gbar,

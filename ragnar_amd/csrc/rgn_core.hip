@@ -90,6 +90,12 @@ void DeviceBuffer::release() {
   }
 }
 
+void PlanUpload::finish(DeviceBuffer& buffer) {
+  buffer.reset(std::max<size_t>(host_.size(), 256));
+  if (!host_.empty()) RGN_HIP(hipMemcpy(buffer.ptr, host_.data(), host_.size(), hipMemcpyHostToDevice));
+  for (auto& a : arrays_) a.first->ptr = static_cast<unsigned char*>(buffer.ptr) + a.second;
+}
+
 namespace {
 thread_local StageScope* t_stages = nullptr;
 }

@@ -5,9 +5,12 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <cstring>
 #include <mutex>
 #include <stdexcept>
 #include <string>
+#include <utility>
+#include <vector>
 
 #include "ragnar_hip.h"
 
@@ -69,6 +72,35 @@ struct DeviceBuffer {
   void release();
   template <class T>
   T* as() const { return static_cast<T*>(ptr); }
+};
+
+// A plan's device arrays in one allocation, uploaded by one copy (an
+// allocation, a copy and a free apiece for a dozen small arrays took most of a
+// call that makes its own plan).
+struct PlanArray {
+  void* ptr = nullptr;  // inside the plan's DeviceBuffer
+  template <class T>
+  T* as() const { return static_cast<T*>(ptr); }
+};
+
+class PlanUpload {
+ public:
+  // Room for n elements, filled from data unless that is null.
+  template <class T>
+  void add(PlanArray& a, const T* data, size_t n) {
+    const size_t at = host_.size();
+    host_.resize(at + (n * sizeof(T) + 255) / 256 * 256);
+    if (data && n) std::memcpy(host_.data() + at, data, n * sizeof(T));
+    arrays_.push_back({&a, at});
+  }
+  template <class T>
+  void add(PlanArray& a, const std::vector<T>& v) { add(a, v.data(), v.size()); }
+  // Allocates `buffer`, copies and sets the arrays' pointers.
+  void finish(DeviceBuffer& buffer);
+
+ private:
+  std::vector<unsigned char> host_;
+  std::vector<std::pair<PlanArray*, size_t>> arrays_;
 };
 
 // Scratch of the library's device, one buffer per slot, reused by every call
