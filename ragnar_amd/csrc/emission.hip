@@ -92,6 +92,7 @@ __global__ void __launch_bounds__(kThreads) product_pair_kernel(const double* __
 }
 
 struct ParticleSourceFn {
+  static constexpr bool kReach = true;  // sorted by the blocks they reach
   ParticlesDev D;
   using Raw = RawParticle;
   __device__ Raw load(size_t p) const { return load_particle(D, p); }
@@ -101,6 +102,7 @@ struct ParticleSourceFn {
 // synchrotron.hpp:72-95: eps = e_at * gb * gb / (g_syn * g_syn) in float;
 // the weight is f (times gb for log-spaced distribution bins).
 struct DistSourceFn {
+  static constexpr bool kReach = false;  // few blocks, bound by latency: every pair, straight through
   const float* gbeta;
   const float* f;
   int dist_log;
@@ -149,15 +151,20 @@ __global__ void __launch_bounds__(kThreads) forward_kernel(SourceFn fn, size_t n
     if (p < n) s = fn.make(raw, P);
     // the next tile's inputs load while this tile is evaluated
     if (p + stride < n) raw = fn.load(p + stride);
-    int count[NB + 1];
-    const int slot = class_slot<NB>(blocks_reached<NB>(s, P), count);
+    int count[NB + 1], slot = lane;
+    if constexpr (SourceFn::kReach) slot = class_slot<NB>(blocks_reached<NB>(s, P), count);
     wave_lds_fence();  // the wave's previous sources have been read
     tile[wave * 64 + slot] = make_float4(s.W, s.vhi, s.vlo, 0.0f);
     wave_lds_fence();
     float acc[NB];
 #pragma unroll
     for (int k = 0; k < NB; ++k) acc[k] = 0.0f;
-    eval_classes<NB, NB>(tile + wave * 64, 0, count, c, S, ltab, acc);
+    if constexpr (SourceFn::kReach) {
+      eval_classes<NB, NB>(tile + wave * 64, 0, count, c, S, ltab, acc);
+    } else {
+      int j = 0;
+      eval_blocks<NB, NB>(tile + wave * 64, j, 64, c, S, ltab, acc);
+    }
 #pragma unroll
     for (int k = 0; k < NB; ++k) dacc[k] += static_cast<double>(acc[k]);
   }
@@ -183,6 +190,52 @@ __global__ void __launch_bounds__(kThreads) forward_kernel(SourceFn fn, size_t n
       partials[static_cast<size_t>(e) * gridDim.x + blockIdx.x] = v;
     }
   }
+}
+
+// Spectrum of a tabulated distribution of few sources: a wave per photon bin.
+// A block makes the sources (kDistThreads at a time) in LDS and each of its
+// waves sums them over its lanes for one bin, so that the bins spread over the
+// device and nothing is combined afterwards.  Bound by latency: 200 sources x
+// 200 bins in one block of the forward kernel (each wave a share of the sources,
+// all bins) took 7.0 us, this 3.3.  Every block makes all the sources, which pays
+// up to about 5000 of them: calls on 4096 sources 13.8 (512 bins: 17.5) -> 11.0
+// us, on 8192 13.8 (17.5) -> 20, so more go to the forward kernel.
+constexpr int kDistThreads = 512;
+constexpr int kDistMax = 4096;
+
+__global__ void __launch_bounds__(kDistThreads) dist_kernel(DistSourceFn fn, int ng, PlanDev P,
+                                                            float* __restrict__ out) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  float4* tile = reinterpret_cast<float4*>(smem);
+  float2* ltab = reinterpret_cast<float2*>(smem + kDistThreads * sizeof(float4));
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int e = min(static_cast<int>(blockIdx.x) * (kDistThreads / 64) + wave, P.nbins - 1);
+  DistSourceFn::Raw raw{};
+  if (static_cast<int>(threadIdx.x) < ng) raw = fn.load(threadIdx.x);
+  const float2 cs_e = P.bincs[e];
+  const float ee = P.bine[e];
+  for (int j = threadIdx.x; j < P.TP; j += kDistThreads) ltab[j] = P.table[j];
+  double acc = 0.0;
+  for (int base = 0; base < ng; base += kDistThreads) {
+    const int g = base + static_cast<int>(threadIdx.x);
+    Source s{0.0f, P.v_safe, 0.0f};
+    if (g < ng) s = fn.make(raw, P);
+    if (g + kDistThreads < ng) raw = fn.load(g + kDistThreads);
+    __syncthreads();  // the previous sources have been read
+    tile[threadIdx.x] = make_float4(s.W, s.vhi, s.vlo, 0.0f);
+    __syncthreads();
+    const int m = min(ng - base, kDistThreads);
+#pragma unroll 4
+    for (int j = lane; j < m; j += 64) {
+      const float4 q = tile[j];
+      const float u = fmaf(cs_e.x, cs_e.y, q.y) + q.z;
+      const float2 cs = ltab[cvt_sat_u32(u)];
+      acc += static_cast<double>(q.x) * static_cast<double>(fmaf(u, cs.y, cs.x));
+    }
+  }
+#pragma unroll
+  for (int w = 32; w > 0; w >>= 1) acc += __shfl_xor(acc, w);
+  if (lane == 0) out[e] = (ee == 0.0f) ? 0.0f : static_cast<float>(static_cast<double>(ee) * acc);
 }
 
 // out[e] = e_e * sum_b partials[e][b] (fixed order), 0 for dead bins.
@@ -737,17 +790,20 @@ int rgn_sync_fromdist(const rgn_sync_plan* plan, const float* d_gbeta, const flo
     RGN_REQUIRE(d_gbeta != nullptr && d_f != nullptr && d_out != nullptr, RGN_ERR_INVALID,
                 "null argument");
     RGN_REQUIRE(ng >= 0, RGN_ERR_INVALID, "negative distribution size");
-    ScratchUse order(as_stream(stream));
     const SyncPlan& p = plan->p;
+    hipStream_t st = as_stream(stream);
+    if (ng <= kDistMax) {  // no scratch, so no order with other calls
+      const unsigned blocks = static_cast<unsigned>(ceil_div(p.nbins, kDistThreads / 64));
+      const size_t smem = kDistThreads * sizeof(float4) + p.TP * sizeof(float2);
+      dist_kernel<<<blocks, kDistThreads, smem, st>>>(DistSourceFn{d_gbeta, d_f, dist_log}, ng, device_view(p), d_out);
+      RGN_HIP(hipGetLastError());
+      stage_mark(st, "dist_kernel");
+      return;
+    }
+    ScratchUse order(st);
     const int grid = forward_grid(static_cast<size_t>(ng), 4);
     double* partials =
       static_cast<double*>(scratch(sizeof(double) * p.nbins_pad * static_cast<size_t>(grid), 1));
-    hipStream_t st = as_stream(stream);
-    if (grid == 1) {  // one block: it writes the spectrum, no combine launch
-      launch_forward(p, DistSourceFn{d_gbeta, d_f, dist_log}, static_cast<size_t>(ng), grid, partials, st,
-                     d_out);
-      return;
-    }
     launch_forward(p, DistSourceFn{d_gbeta, d_f, dist_log}, static_cast<size_t>(ng), grid,
                    partials, st);
     launch_combine(p, partials, grid, d_out, st);
