@@ -1,5 +1,5 @@
 // Spatially resolved spectra: S[c, e] for ncells particle slices (CSR offsets)
-// in one persistent launch plus a fixed-order combine, captured in a hipGraph.
+// in one persistent launch plus a fixed-order combine.
 //
 // Balance.  The particle range [off[0], off[ncells]) is cut into G equal chunks
 // of Q particles, one per block, regardless of cell boundaries, so ragged cell
@@ -16,7 +16,6 @@
 // the cell and particle counts) and cached in a JSON file (RAGNAR_TUNE_CACHE,
 // default ~/.cache/ragnar_amd/tune.json; RAGNAR_TUNE=0 disables tuning: 4
 // blocks per CU).
-// RAGNAR_CELLS_GRAPH=0 launches without the graph.
 #include <algorithm>
 #include <cstdio>
 #include <cstdlib>
@@ -236,29 +235,6 @@ int log2_bucket(int64_t v) {
   return b;
 }
 
-// ---------------------------------------------------------------------------
-// Graph cache keyed by every launch argument.
-// ---------------------------------------------------------------------------
-struct GraphKey {
-  const void* plan;
-  const void* ptrs[10];
-  const void* off;
-  const void* records;
-  const void* out;
-  int ncells;
-  int64_t Q;
-  int grid;
-  bool operator<(const GraphKey& o) const {
-    return std::lexicographical_compare(reinterpret_cast<const char*>(this),
-                                        reinterpret_cast<const char*>(this) + sizeof(GraphKey),
-                                        reinterpret_cast<const char*>(&o),
-                                        reinterpret_cast<const char*>(&o) + sizeof(GraphKey));
-  }
-};
-
-std::mutex g_graph_mutex;
-std::map<GraphKey, hipGraphExec_t> g_graphs;
-
 }  // namespace
 
 static void run_cells(const SyncPlan& plan, const ParticlesDev& D, const int64_t* h_off, int ncells,
@@ -270,7 +246,6 @@ static void run_cells(const SyncPlan& plan, const ParticlesDev& D, const int64_t
   }
   RGN_REQUIRE(h_off[0] >= 0, RGN_ERR_INVALID, "negative cell offset");
   const int64_t total = h_off[ncells] - h_off[0];
-  // offsets to a scratch buffer (outside any graph), then the launch
   int64_t* d_off = static_cast<int64_t*>(scratch(sizeof(int64_t) * (ncells + 1), 4));
   RGN_HIP(hipMemcpyAsync(d_off, h_off, sizeof(int64_t) * (ncells + 1), hipMemcpyHostToDevice, st));
 
@@ -325,59 +300,11 @@ static void run_cells(const SyncPlan& plan, const ParticlesDev& D, const int64_t
 
   int64_t Q;
   const int grid = plan_grid(bpc, Q);
-  const char* graph_env = std::getenv("RAGNAR_CELLS_GRAPH");
-  const bool use_graph = !(graph_env && std::string(graph_env) == "0");
-  if (!use_graph) {
-    launch_cells(plan, D, d_off, ncells, Q, grid, records, out, st);
-    return;
-  }
-  GraphKey gk{};
-  gk.plan = &plan;
-  for (int k = 0; k < 3; ++k) {
-    gk.ptrs[k] = D.u[k];
-    gk.ptrs[3 + k] = D.e[k];
-    gk.ptrs[6 + k] = D.b[k];
-  }
-  gk.ptrs[9] = D.w;
-  gk.off = d_off;
-  gk.records = records;
-  gk.out = out;
-  gk.ncells = ncells;
-  gk.Q = Q;
-  gk.grid = grid;
-  std::lock_guard<std::mutex> lk(g_graph_mutex);
-  auto it = g_graphs.find(gk);
-  if (it == g_graphs.end()) {
-    hipStream_t cap;
-    RGN_HIP(hipStreamCreateWithFlags(&cap, hipStreamNonBlocking));
-    hipGraph_t graph;
-    RGN_HIP(hipStreamBeginCapture(cap, hipStreamCaptureModeThreadLocal));
-    launch_cells(plan, D, d_off, ncells, Q, grid, records, out, cap);
-    RGN_HIP(hipStreamEndCapture(cap, &graph));
-    hipGraphExec_t exec;
-    RGN_HIP(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
-    RGN_HIP(hipGraphDestroy(graph));
-    RGN_HIP(hipStreamDestroy(cap));
-    if (g_graphs.size() >= 16) {
-      RGN_HIP(hipGraphExecDestroy(g_graphs.begin()->second));
-      g_graphs.erase(g_graphs.begin());
-    }
-    it = g_graphs.emplace(gk, exec).first;
-  }
-  RGN_HIP(hipGraphLaunch(it->second, st));
-}
-
-// Drops cached graphs of a plan that is being destroyed.
-void forget_plan_graphs(const void* plan) {
-  std::lock_guard<std::mutex> lk(g_graph_mutex);
-  for (auto it = g_graphs.begin(); it != g_graphs.end();) {
-    if (it->first.plan == plan) {
-      (void)hipGraphExecDestroy(it->second);
-      it = g_graphs.erase(it);
-    } else {
-      ++it;
-    }
-  }
+  // Two plain launches.  A graph of them holds the caller's buffers: replaying
+  // it cost more than the launches (64 cells of 1000 particles 61 against 30 us,
+  // 4096 of 4000 646 against 500), capturing it for new ones far more (1024
+  // cells of 200, a new result tensor each call, 228 against 51 us).
+  launch_cells(plan, D, d_off, ncells, Q, grid, records, out, st);
 }
 
 }  // namespace rgn

@@ -668,7 +668,6 @@ int rgn_sync_plan_create(const rgn_ftable* table, const float* h_bins, int nbins
 }
 
 int rgn_sync_plan_destroy(rgn_sync_plan* plan) {
-  if (plan) forget_plan_graphs(&plan->p);
   delete plan;
   return RGN_OK;
 }

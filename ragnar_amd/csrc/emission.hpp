@@ -107,9 +107,6 @@ void launch_combine(const SyncPlan& plan, const double* partials, int grid, floa
 ParticlesDev make_particles_checked(const float* const d_u[3], const float* const d_e[3],
                                     const float* const d_b[3], const float* d_w, size_t n);
 
-// Drops the cached cell graphs that reference a plan being destroyed.
-void forget_plan_graphs(const void* plan);
-
 }  // namespace rgn
 
 struct rgn_sync_plan {
