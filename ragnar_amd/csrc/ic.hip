@@ -11,13 +11,21 @@
 // are summed in FP64 in a fixed order, so results are reproducible bit for bit.
 //
 // Layout: one workgroup per (output bin, chunk of gamma bins), enough of them
-// to fill the device; the threads take the soft-photon bins (the two
-// distributions are a few KB and stay in cache); a fixed-order tree per block
-// and a second pass adding the chunks in order.  No table or plan.  The kernel
-// is bound by its VALU work (IEEE float and double divides), so the quotients
-// that depend on one operand only -- e_ic / g per gamma bin, f_s / e_s per
-// soft-photon bin -- are formed once (the same float values the reference
-// forms per triple) and the triples loop over gamma bins staged in LDS.
+// to fill the device; its threads take the chunk's (gamma, e_soft) pairs in
+// turn, both staged in LDS; a fixed-order tree per block and, with more than one
+// chunk, a second pass adding the chunks in order.  No table or plan.
+//
+// The kernel is bound by its VALU work, so what depends on one operand only is
+// formed once per block.  With x = e_ic / g (the reference's float value)
+//     q = [x / (4 g (1 - x))] (1 / e_s),   Gamma q = x / (1 - x),
+// so a pair's q is one product, KN's quotient (Gamma q)^2 / (1 + Gamma q) is the
+// gamma bin's, and the kinematic limit is q = 1: no divide is left in the loop.
+// Pairs where rounding could decide differently (q within 2e-6 / (1 - x) of 1:
+// the reference's limit is good to 2.4e-7 / (1 - x)) and operands outside the
+// ranges below take the reference's own operations.
+// Per call, before and after: 200^3 27.7 and 16.2 us (of it the kernel 23.4 and
+// 11.5: the loop's 125000 wave steps take 4.4, loading, staging and the reduction
+// the rest), 500^3 243 and 92, 1000^3 1596 and 552 us (87 clocks a step of 64 pairs).
 #include <algorithm>
 #include <cmath>
 
@@ -27,7 +35,9 @@ namespace rgn {
 namespace {
 
 constexpr int kIcThreads = 256;
-constexpr int kIcStage = 1024;  // gamma bins staged in LDS at a time
+constexpr int kIcGamma = 128;  // gamma bins and
+static_assert(kIcGamma <= kIcThreads, "one gamma bin a thread");
+constexpr int kIcSoft = 512;   // soft-photon bins staged in LDS at a time
 
 // ic.hpp:20-25.  2 * q * log(q) is float; the 0.5 literal makes the rest double.
 __device__ __forceinline__ float kn_func(float Gamma, float q) {
@@ -39,64 +49,153 @@ __device__ __forceinline__ float kn_func(float Gamma, float q) {
   return static_cast<float>(static_cast<double>(first) + rest);
 }
 
-// One workgroup per (output bin, chunk of gamma bins): its threads take the
-// soft-photon bins, and each thread runs its bins over the chunk's gamma bins,
-// staged kIcStage at a time; the block's FP64 partial goes to
-// partial[chunk][bin].  Summation order: per thread, stage by stage, soft-photon
-// bin by bin, gamma bin by gamma bin; then a fixed tree over the threads.
+// ic.hpp:62-85, float arithmetic in the reference's order.
+__device__ __noinline__ float ic_term(float g_prtls, float f_prtls, float e_soft, float fs_es, float e_ic, int g_log) {
+  const float Gamma = 4.0f * g_prtls * e_soft;
+  if (e_ic > g_prtls * Gamma / (1.0f + Gamma)) return 0.0f;
+  const float x = e_ic / g_prtls;
+  const float q = x / (Gamma * (1.0f - x));
+  const float kn = kn_func(Gamma, q);
+  return g_log ? f_prtls * fs_es * e_ic * e_ic * kn / g_prtls
+               : f_prtls * fs_es * e_ic * e_ic * kn / (g_prtls * g_prtls);
+}
+
+// 1 / x to about one ulp (hardware estimate, two Newton steps).
+__device__ __forceinline__ double ic_rcp(double x) {
+  double y = __builtin_amdgcn_rcp(x);
+  y = fma(fma(-x, y, 1.0), y, y);
+  return fma(fma(-x, y, 1.0), y, y);
+}
+
+struct __align__(16) IcGamma {
+  float c;       // x / (4 g (1 - x)); NaN: outside the ranges, every pair by ic_term
+  float lo, hi;  // below lo (from kIcMinQ): a term; above hi: none; between: ic_term
+  float f;
+  double h;  // (Gamma q)^2 / (1 + Gamma q) / 2
+  float ig;  // 1 / g, or 1 / g^2 for linear gamma bins
+  float g;
+};
+constexpr float kIcMinQ = 1e-30f;
+
+__device__ __forceinline__ IcGamma ic_gamma(float g, float f, float e_ic, int g_log) {
+  IcGamma o;
+  const float x = e_ic / g, one_x = 1.0f - x;
+  const bool ok = g >= 1e-6f && g <= 1e12f && x >= 1e-20f && fabsf(one_x) >= 4e-6f && x < INFINITY;
+  const double gq = static_cast<double>(x) * ic_rcp(one_x);
+  // past the limit for every e_soft where x > 1
+  o.c = !ok ? NAN : one_x > 0.0f ? static_cast<float>(0.25 * gq * ic_rcp(g)) : INFINITY;
+  const float margin = 2e-6f * __builtin_amdgcn_rcpf(fabsf(one_x));
+  o.lo = 1.0f - margin;
+  o.hi = 1.0f + margin;
+  o.f = f;
+  o.h = 0.5 * gq * gq * ic_rcp(1.0 + gq);
+  o.ig = 1.0f / (g_log ? g : g * g);
+  o.g = g;
+  return o;
+}
+
+// One workgroup per (output bin, chunk of gamma bins).  The pairs of a stage go
+// to the threads in turn, soft-photon bins fastest, so that every lane has a
+// pair whatever the counts; the block's FP64 sum goes to partial[chunk][bin], or
+// to the result where there is one chunk.  Summation order: per thread, stage by
+// stage, its pairs in order; then a fixed tree over the threads.
 __global__ void __launch_bounds__(kIcThreads) ic_kernel(const float* __restrict__ g, const float* __restrict__ fg,
                                                         int ng, int g_log, const float* __restrict__ es,
                                                         const float* __restrict__ fes, int nes,
                                                         const float* __restrict__ eic, int gper,
-                                                        double* __restrict__ partial) {
+                                                        double* __restrict__ partial, float* __restrict__ out) {
   __shared__ double red[kIcThreads];
-  __shared__ float s_g[kIcStage], s_f[kIcStage], s_x[kIcStage];
-  const int e = blockIdx.x, neic = gridDim.x;
+  __shared__ IcGamma s_g[kIcGamma];
+  __shared__ float s_r[kIcSoft], s_f[kIcSoft];  // 1 / e_soft (NaN: outside the range), f_s / e_soft
+  const int e = blockIdx.x, neic = gridDim.x, tid = threadIdx.x;
   const float e_ic = eic[e];
   const int g0 = blockIdx.y * gper, g1 = min(ng, g0 + gper);
   double acc = 0.0;
-  for (int gs = g0; gs < g1; gs += kIcStage) {
-    const int m = min(kIcStage, g1 - gs);
-    __syncthreads();  // the previous stage has been read
-    for (int i = threadIdx.x; i < m; i += kIcThreads) {
-      const float gp = g[gs + i];
-      s_g[i] = gp;
-      s_f[i] = fg[gs + i];
-      s_x[i] = e_ic / gp;
-    }
-    __syncthreads();
-    for (int si = threadIdx.x; si < nes; si += kIcThreads) {
-      // ic.hpp:62-85, float arithmetic in the reference's order
-      const float e_soft = es[si];
-      const float fs_es = fes[si] / e_soft;
-      for (int i = 0; i < m; ++i) {
-        const float g_prtls = s_g[i], f_prtls = s_f[i], x = s_x[i];
-        const float Gamma = 4.0f * g_prtls * e_soft;
-        if (e_ic > g_prtls * Gamma / (1.0f + Gamma)) continue;
-        const float q = x / (Gamma * (1.0f - x));
-        const float kn = kn_func(Gamma, q);
-        const float term = g_log ? f_prtls * fs_es * e_ic * e_ic * kn / g_prtls
-                                 : f_prtls * fs_es * e_ic * e_ic * kn / (g_prtls * g_prtls);
-        acc += static_cast<double>(term);
+  for (int ss = 0; ss < nes; ss += kIcSoft) {
+    const int ms = min(kIcSoft, nes - ss);
+    const int di = kIcThreads / ms, ds = kIcThreads % ms;  // a step of kIcThreads pairs
+    for (int gs = g0; gs < g1; gs += kIcGamma) {
+      const int mg = min(kIcGamma, g1 - gs);
+      // all loads of a stage at once: in a small call they are most of a block's time
+      float soft[kIcSoft / kIcThreads], fsoft[kIcSoft / kIcThreads];
+      if (gs == g0) {
+#pragma unroll
+        for (int j = 0; j < kIcSoft / kIcThreads; ++j) {
+          const int i = min(tid + j * kIcThreads, ms - 1);
+          soft[j] = es[ss + i];
+          fsoft[j] = fes[ss + i];
+        }
+      }
+      const int ig = gs + min(tid, mg - 1);
+      const float gv = g[ig], fv = fg[ig];
+      __syncthreads();  // the previous stage has been read
+      if (tid < mg) s_g[tid] = ic_gamma(gv, fv, e_ic, g_log);
+      if (gs == g0) {
+#pragma unroll
+        for (int j = 0; j < kIcSoft / kIcThreads; ++j) {
+          if (tid + j * kIcThreads < ms) {
+            s_r[tid + j * kIcThreads] = soft[j] >= 1e-15f && soft[j] <= 1e15f ? 1.0f / soft[j] : NAN;
+            s_f[tid + j * kIcThreads] = fsoft[j] / soft[j];
+          }
+        }
+      }
+      __syncthreads();
+      int i = tid / ms, si = tid % ms;
+      while (i < mg) {
+        const IcGamma G = s_g[i];
+        const float fs_es = s_f[si], q = G.c * s_r[si];
+        if (!(q > G.hi)) {
+          float term;
+          if (q <= G.lo && q >= kIcMinQ) {
+            const float first = 2.0f * q * (__builtin_amdgcn_logf(q) * 0.6931471805599453f);
+            const float kn = static_cast<float>(fma(static_cast<double>(1.0f - q),
+                                                    static_cast<double>(1.0f + 2.0f * q) + G.h,
+                                                    static_cast<double>(first)));
+            term = G.f * fs_es * e_ic * e_ic * kn * G.ig;
+          } else {
+            term = ic_term(G.g, G.f, es[ss + si], fs_es, e_ic, g_log);
+          }
+          acc += static_cast<double>(term);
+        }
+        i += di;
+        si += ds;
+        if (si >= ms) {
+          si -= ms;
+          ++i;
+        }
       }
     }
   }
-  red[threadIdx.x] = acc;
+  red[tid] = acc;
   __syncthreads();
   for (int w = kIcThreads / 2; w > 0; w >>= 1) {
-    if (static_cast<int>(threadIdx.x) < w) red[threadIdx.x] += red[threadIdx.x + w];
+    if (tid < w) red[tid] += red[tid + w];
     __syncthreads();
   }
-  if (threadIdx.x == 0) partial[static_cast<size_t>(blockIdx.y) * neic + e] = red[0];
+  if (tid == 0) {
+    if (gridDim.y == 1) {
+      out[e] = static_cast<float>(red[0]);
+    } else {
+      partial[static_cast<size_t>(blockIdx.y) * neic + e] = red[0];
+    }
+  }
 }
 
-// out[e] = the chunk partials of bin e, summed in chunk order.
-__global__ void __launch_bounds__(kIcThreads) ic_combine(const double* __restrict__ partial, int nchunk, int neic,
+// out[e] = the chunk partials of bin e, summed in chunk order, eight in flight.
+constexpr int kIcCombine = 64;
+
+__global__ void __launch_bounds__(kIcCombine) ic_combine(const double* __restrict__ partial, int nchunk, int neic,
                                                          float* __restrict__ out) {
-  const int e = blockIdx.x * kIcThreads + threadIdx.x;
+  const int e = blockIdx.x * kIcCombine + threadIdx.x;
   if (e >= neic) return;
   double s = 0.0;
-  for (int c = 0; c < nchunk; ++c) s += partial[static_cast<size_t>(c) * neic + e];
+  for (int c = 0; c < nchunk; c += 8) {
+    double v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = partial[static_cast<size_t>(min(c + k, nchunk - 1)) * neic + e];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) s += c + k < nchunk ? v[k] : 0.0;
+  }
   out[e] = static_cast<float>(s);
 }
 
@@ -118,16 +217,23 @@ int rgn_ic_spectrum(const float* d_g, const float* d_fg, int ng, int g_log, cons
                 "null argument");
     hipStream_t st = as_stream(stream);
     ScratchUse order(st);
-    // enough workgroups to fill the device: gamma bins split into chunks
-    const int chunks = std::min(std::max(1, (8 * num_cus() + neic - 1) / neic), std::max(ng, 1));
+    // Gamma bins in chunks: up to 16 blocks per CU (500^3: 8 blocks 100 us, 16 93),
+    // but at least kIcPairs pairs a block, below which its staging and reduction
+    // outweigh them (200^3 of 2048, 4096, 8192 pairs: 18.1, 16.2, 18.1 us; 50^3 as
+    // 20 chunks and a second pass 15.6, as one 12.6 us)
+    constexpr double kIcPairs = 4096.0;
+    const double most = std::max(1, (16 * num_cus() + neic - 1) / neic);
+    const double pairs = static_cast<double>(ng) * nes;
+    const int chunks = std::max(1, static_cast<int>(std::min({most, static_cast<double>(ng), pairs / kIcPairs})));
     const int gper = std::max(1, (ng + chunks - 1) / chunks);
-    const int nchunk = std::max(1, (ng + gper - 1) / gper);  // at most chunks <= 8 CUs + 1
+    const int nchunk = std::max(1, (ng + gper - 1) / gper);  // at most 16 CUs + 1
     double* partial = static_cast<double*>(scratch(sizeof(double) * nchunk * static_cast<size_t>(neic), 17));
     ic_kernel<<<dim3(neic, nchunk), kIcThreads, 0, st>>>(d_g, d_fg, ng, g_log ? 1 : 0, d_es, d_fes, nes, d_eic,
-                                                         gper, partial);
+                                                         gper, partial, d_out);
     RGN_HIP(hipGetLastError());
     stage_mark(st, "ic_kernel");
-    ic_combine<<<(neic + kIcThreads - 1) / kIcThreads, kIcThreads, 0, st>>>(partial, nchunk, neic, d_out);
+    if (nchunk == 1) return;
+    ic_combine<<<(neic + kIcCombine - 1) / kIcCombine, kIcCombine, 0, st>>>(partial, nchunk, neic, d_out);
     RGN_HIP(hipGetLastError());
     stage_mark(st, "ic_combine");
   });
