@@ -28,7 +28,7 @@ namespace rgn {
 
 namespace {
 
-constexpr int kTN = 256;        // columns (photon bins) per workgroup
+constexpr int kTN = 256;        // columns (photon bins) of the largest tile; K is padded to it
 constexpr int kKB = 64;         // g per block (one scale exponent)
 constexpr int kLd = kKB + 8;    // LDS row pitch in halves (bank spread)
 
@@ -122,8 +122,9 @@ __global__ void __launch_bounds__(256) pack_kernel_matrix(PlanDev P, const float
   }
 }
 
-// Matrix kernel: a 64 x 256 tile per 4-wave workgroup, two workgroups per CU.
-// Each wave owns 64 columns (2 x 2 MFMA tiles over all 64 rows).  Only the
+// Matrix kernel: a tile of RT x 32 rows by CT x 128 columns (launch_tiles; the
+// figures here are of 64 x 256) per 4-wave workgroup, two workgroups per CU.
+// Each wave owns CT x 32 columns (RT x CT MFMA tiles over all rows).  Only the
 // f tile is shared by the waves, so only it goes through LDS, double
 // buffered: while the matrix cores work on block kb, the waves split block
 // kb + 1 (already in registers) into the other buffer, and one barrier per
@@ -143,7 +144,7 @@ __global__ void __launch_bounds__(256) pack_kernel_matrix(PlanDev P, const float
 // from HBM; issued last, the f load has the rescale, the barrier and the next
 // block's first step to arrive in.  The column scales of a block are loaded
 // at its start and used at its end.
-constexpr int kTM2 = 64;
+constexpr int kTM2 = 64;  // rows of the largest tile
 constexpr int kThreads2 = 256;
 
 // Rows of f given as terms instead of values (GEN): a power law with an
@@ -185,8 +186,9 @@ __device__ __forceinline__ void stage_grid_terms(const float* __restrict__ grid,
   }
 }
 
-// f rows as the matrix kernels read them: thread (row ar, quarter aq) of a
-// 256-thread workgroup holds 16 consecutive g of row d0 + ar of one g block.
+// f rows as the matrix kernels read them: thread (row ar, part aq) of a
+// 256-thread workgroup holds PER (16 or 8) consecutive g of row d0 + ar of one
+// g block.
 //   LOAD 0  scalar loads, each element checked against nd and ng;
 //   LOAD 1  16-byte loads (rows 16-byte aligned, ng % 4 == 0), each checked;
 //   LOAD 2  16-byte loads of whole blocks (and ng % 64 == 0): rows past nd
@@ -197,16 +199,16 @@ __device__ __forceinline__ void stage_grid_terms(const float* __restrict__ grid,
 // load(kb, ra, count): block kb into ra; with count (GEN), the block's
 // values also go into the row's norm (each block is counted once, though the
 // kernels' branch-free loops load the last block more than once).
-template <int LOAD, bool GEN>
+template <int LOAD, bool GEN, int PER>
 struct RowBlocks {
-  const float* row;      // LOAD 2: start of this thread's row and quarter
+  const float* row;      // LOAD 2: start of this thread's part of its row
   const float* A;
-  int nd, ng, d, g_off;  // g_off = 16 aq
+  int nd, ng, d, g_off;  // g_off = PER aq
   const double* gL;      // GEN: LDS grid terms L_g, x_g, w_g
   double gp, gc, go, nsum;
 
   __device__ RowBlocks(const float* A_, int nd_, int ng_, int d_, int aq, const GenRows& gen, const double* gterms)
-      : row(nullptr), A(A_), nd(nd_), ng(ng_), d(d_), g_off(16 * aq), gL(gterms), gp(0.0), gc(0.0), go(0.0),
+      : row(nullptr), A(A_), nd(nd_), ng(ng_), d(d_), g_off(PER * aq), gL(gterms), gp(0.0), gc(0.0), go(0.0),
         nsum(0.0) {
     const int dc = min(d, nd - 1);
     if (LOAD == 2 && !GEN) row = A + static_cast<size_t>(dc) * ng + g_off;
@@ -221,12 +223,12 @@ struct RowBlocks {
     }
   }
 
-  __device__ __forceinline__ void load(int kb, float (&ra)[16], bool count) {
+  __device__ __forceinline__ void load(int kb, float (&ra)[PER], bool count) {
     const int g0 = kb * kKB + g_off;
     if (GEN) {
       double s = 0.0;
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
+      for (int i = 0; i < PER; ++i) {
         const bool in = LOAD == 2 || g0 + i < ng;
         ra[i] = in ? gen_value(gp, gc, go, gL[g0 + i], gL[ng + g0 + i]) : 0.0f;
         s = fma(static_cast<double>(ra[i]), in ? gL[2 * ng + g0 + i] : 0.0, s);
@@ -234,7 +236,7 @@ struct RowBlocks {
       if (count) nsum += s;
     } else if (LOAD == 2) {
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
+      for (int k = 0; k < PER / 4; ++k) {
         const float4 v = *reinterpret_cast<const float4*>(row + kb * kKB + 4 * k);
         ra[4 * k] = v.x;
         ra[4 * k + 1] = v.y;
@@ -243,7 +245,7 @@ struct RowBlocks {
       }
     } else if (LOAD == 1) {
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
+      for (int k = 0; k < PER / 4; ++k) {
         float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         if (d < nd && g0 + 4 * k < ng) v = *reinterpret_cast<const float4*>(A + static_cast<size_t>(d) * ng + g0 + 4 * k);
         ra[4 * k] = v.x;
@@ -253,58 +255,61 @@ struct RowBlocks {
       }
     } else {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) ra[i] = (d < nd && g0 + i < ng) ? A[static_cast<size_t>(d) * ng + g0 + i] : 0.0f;
+      for (int i = 0; i < PER; ++i) ra[i] = (d < nd && g0 + i < ng) ? A[static_cast<size_t>(d) * ng + g0 + i] : 0.0f;
     }
   }
 
-  // GEN: 1 / N_d of this thread's row (the row's four threads each hold a
-  // quarter of the sum; every thread of the workgroup calls this)
+  // GEN: 1 / N_d of this thread's row (the row's 64 / PER threads each hold a
+  // part of the sum; every thread of the workgroup calls this)
   __device__ __forceinline__ float inv_norm() const {
     double t = nsum;
     t += __shfl_xor(t, 1);
     t += __shfl_xor(t, 2);
+    if (PER == 8) t += __shfl_xor(t, 4);
     return static_cast<float>(1.0 / t);
   }
 };
 
-template <int NPROD, int LOAD, bool GEN = false>
+template <int NPROD, int LOAD, int RT, int CT, bool GEN = false>
 __global__ void __launch_bounds__(kThreads2, 2) mfma_contract2(const float* __restrict__ A, int nd, int ng,
                                                                const _Float16* __restrict__ Bh,
                                                                const _Float16* __restrict__ Bl,
                                                                const float* __restrict__ rB, int nb, int nbp,
                                                                int nkb, int ntn, float* __restrict__ out,
                                                                GenRows gen = GenRows{}) {
-  __shared__ __align__(16) _Float16 Ah[2][kTM2][kLd];
-  __shared__ __align__(16) _Float16 Al[2][kTM2][kLd];
-  __shared__ __align__(16) float rA[2][kTM2];
+  constexpr int TM = 32 * RT, TN = 128 * CT, kParts = kThreads2 / TM, kPer = kKB / kParts;
+  __shared__ __align__(16) _Float16 Ah[2][TM][kLd];
+  __shared__ __align__(16) _Float16 Al[2][TM][kLd];
+  __shared__ __align__(16) float rA[2][TM];
   // tile of this workgroup: the ntn column tiles of a row block on one XCD
   const unsigned T = gridDim.x;
   unsigned q = blockIdx.x;
   if (T % 8 == 0) q = (blockIdx.x % 8) * (T / 8) + blockIdx.x / 8;
-  const int d0 = static_cast<int>(q / ntn) * kTM2;
-  const int c0 = static_cast<int>(q % ntn) * kTN;
+  const int d0 = static_cast<int>(q / ntn) * TM;
+  const int c0 = static_cast<int>(q % ntn) * TN;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int wc = wave * 64;
-  // f producer: four threads per row, 16 consecutive g each
-  const int ar = threadIdx.x >> 2, aq = threadIdx.x & 3;
+  const int wc = wave * 32 * CT;
+  // f producer: kParts threads per row, kPer consecutive g each
+  const int ar = threadIdx.x / kParts, aq = threadIdx.x % kParts;
   // generated rows: the grid terms in LDS (read by every row)
   extern __shared__ __align__(16) double gterms[];  // GEN: [3][ng]
   if (GEN) {
     stage_grid_terms(gen.grid, ng, gterms);
     __syncthreads();
   }
-  RowBlocks<LOAD, GEN> src(A, nd, ng, d0 + ar, aq, gen, gterms);
-  float ra[16];
+  RowBlocks<LOAD, GEN, kPer> src(A, nd, ng, d0 + ar, aq, gen, gterms);
+  float ra[kPer];
   auto split_a = [&](int buf) {
     float m = 0.0f;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) m = fmaxf(m, fabsf(ra[i]));
+    for (int i = 0; i < kPer; ++i) m = fmaxf(m, fabsf(ra[i]));
     m = fmaxf(m, __shfl_xor(m, 1));
     m = fmaxf(m, __shfl_xor(m, 2));
+    if (kParts == 8) m = fmaxf(m, __shfl_xor(m, 4));
     const int sc = block_exp(m);
-    rA[buf][ar] = ldexpf(1.0f, -sc);  // the row's four threads store the same value
+    rA[buf][ar] = ldexpf(1.0f, -sc);  // the row's threads store the same value
 #pragma unroll
-    for (int k = 0; k < 2; ++k) {
+    for (int k = 0; k < kPer / 8; ++k) {
       half8 h, l;
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
@@ -313,8 +318,8 @@ __global__ void __launch_bounds__(kThreads2, 2) mfma_contract2(const float* __re
         h[i] = hi;
         l[i] = lo;
       }
-      *reinterpret_cast<half8*>(&Ah[buf][ar][aq * 16 + k * 8]) = h;
-      if (NPROD == 3) *reinterpret_cast<half8*>(&Al[buf][ar][aq * 16 + k * 8]) = l;
+      *reinterpret_cast<half8*>(&Ah[buf][ar][aq * kPer + k * 8]) = h;
+      if (NPROD == 3) *reinterpret_cast<half8*>(&Al[buf][ar][aq * kPer + k * 8]) = l;
     }
   };
   // K fragments of this wave (step-major layout): column wc + 32 j + lane % 32,
@@ -325,11 +330,11 @@ __global__ void __launch_bounds__(kThreads2, 2) mfma_contract2(const float* __re
   auto ldb = [&](const _Float16* B, int s, int j) {
     return *reinterpret_cast<const half8*>(B + b0 + static_cast<size_t>(s) * nbp * 16 + j * 512);
   };
-  float16v acc[2][2];
+  float16v acc[RT][CT];
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
+  for (int i = 0; i < RT; ++i) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
+    for (int j = 0; j < CT; ++j) {
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
     }
@@ -337,23 +342,23 @@ __global__ void __launch_bounds__(kThreads2, 2) mfma_contract2(const float* __re
   src.load(0, ra, true);
   split_a(0);
   src.load(min(1, nkb - 1), ra, nkb > 1);
-  half8 bh[2], bl[2];
+  half8 bh[CT], bl[CT];
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
+  for (int j = 0; j < CT; ++j) {
     bh[j] = ldb(Bh, 0, j);
     if (NPROD == 3) bl[j] = ldb(Bl, 0, j);
   }
   __syncthreads();
   for (int kb = 0; kb < nkb; ++kb) {
     const int cur = kb & 1;
-    float sc[2];
+    float sc[CT];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) sc[j] = rB[static_cast<size_t>(kb) * nbp + c0 + wc + j * 32 + (lane & 31)];
-    float16v tmp[2][2];
+    for (int j = 0; j < CT; ++j) sc[j] = rB[static_cast<size_t>(kb) * nbp + c0 + wc + j * 32 + (lane & 31)];
+    float16v tmp[RT][CT];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < RT; ++i) {
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
+      for (int j = 0; j < CT; ++j) {
 #pragma unroll
         for (int v = 0; v < 16; ++v) tmp[i][j][v] = 0.0f;
       }
@@ -362,23 +367,23 @@ __global__ void __launch_bounds__(kThreads2, 2) mfma_contract2(const float* __re
     for (int ks = 0; ks < kKB / 16; ++ks) {
       // next step's K fragments (the next block's first step after the last)
       const int sn = min(kb * (kKB / 16) + ks + 1, nsteps - 1);
-      half8 nbh[2], nbl[2];
+      half8 nbh[CT], nbl[CT];
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
+      for (int j = 0; j < CT; ++j) {
         nbh[j] = ldb(Bh, sn, j);
         if (NPROD == 3) nbl[j] = ldb(Bl, sn, j);
       }
       const int kk = ks * 16 + kofs;
-      half8 ah[2], al[2];
+      half8 ah[RT], al[RT];
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
+      for (int i = 0; i < RT; ++i) {
         ah[i] = *reinterpret_cast<const half8*>(&Ah[cur][i * 32 + (lane & 31)][kk]);
         if (NPROD == 3) al[i] = *reinterpret_cast<const half8*>(&Al[cur][i * 32 + (lane & 31)][kk]);
       }
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
+      for (int i = 0; i < RT; ++i) {
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
+        for (int j = 0; j < CT; ++j) {
           tmp[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[i], bh[j], tmp[i][j], 0, 0, 0);
           if (NPROD == 3) {
             tmp[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[i], bl[j], tmp[i][j], 0, 0, 0);
@@ -387,7 +392,7 @@ __global__ void __launch_bounds__(kThreads2, 2) mfma_contract2(const float* __re
         }
       }
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
+      for (int j = 0; j < CT; ++j) {
         bh[j] = nbh[j];
         if (NPROD == 3) bl[j] = nbl[j];
       }
@@ -397,9 +402,9 @@ __global__ void __launch_bounds__(kThreads2, 2) mfma_contract2(const float* __re
     // acc += tmp 2^-(s_row + s_col); output element v of a lane sits at
     // row 8 (v / 4) + 4 (lane / 32) + v % 4, column lane % 32 of its 32x32 tile
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
+    for (int j = 0; j < CT; ++j) {
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
+      for (int i = 0; i < RT; ++i) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const float4 sr = *reinterpret_cast<const float4*>(&rA[cur][i * 32 + 8 * r + 4 * (lane >> 5)]);
@@ -413,16 +418,16 @@ __global__ void __launch_bounds__(kThreads2, 2) mfma_contract2(const float* __re
     __syncthreads();  // buffer cur is free; buffer cur ^ 1 is written
   }
   // generated rows: divide by the row norms (via LDS, like the row scales)
-  __shared__ float rnorm[GEN ? kTM2 : 1];
+  __shared__ float rnorm[GEN ? TM : 1];
   if (GEN) {
     const float r = src.inv_norm();
-    rnorm[ar] = r;  // the row's four threads store the same value
+    rnorm[ar] = r;  // the row's threads store the same value
     __syncthreads();
   }
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
+  for (int i = 0; i < RT; ++i) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
+    for (int j = 0; j < CT; ++j) {
       const int c = c0 + wc + j * 32 + (lane & 31);
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
@@ -446,7 +451,7 @@ __global__ void __launch_bounds__(kThreads2, 2) mfma_contract2(const float* __re
 // vector work is the split of f (about 7 instructions per element) and the
 // kernel is bound by the matrix cores (six products against three for the
 // split-FP16 form, which spends more vector work than matrix work).
-// Tiling as mfma_contract2: 64 x 256 per 4-wave workgroup, two per CU, f
+// Tiling as mfma_contract2: RT x 32 by CT x 128 per 4-wave workgroup, f
 // double buffered in LDS, K fragments from the packed layout in L2.
 // ---------------------------------------------------------------------------
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -481,33 +486,34 @@ __global__ void __launch_bounds__(256) pack_kernel_matrix_bf16(PlanDev P, const 
   }
 }
 
-template <int LOAD, bool GEN>
+template <int LOAD, int RT, int CT, bool GEN>
 __global__ void __launch_bounds__(kThreads2, 2) mfma_contract_bf16(const float* __restrict__ A, int nd, int ng,
                                                                    const __bf16* __restrict__ Bh,
                                                                    const __bf16* __restrict__ Bm,
                                                                    const __bf16* __restrict__ Bl, int nb, int nbp,
                                                                    int nkb, int ntn, float* __restrict__ out,
                                                                    GenRows gen) {
-  __shared__ __align__(16) __bf16 As[2][3][kTM2][kLd];
+  constexpr int TM = 32 * RT, TN = 128 * CT, kParts = kThreads2 / TM, kPer = kKB / kParts;
+  __shared__ __align__(16) __bf16 As[2][3][TM][kLd];
   const unsigned T = gridDim.x;
   unsigned q = blockIdx.x;
   if (T % 8 == 0) q = (blockIdx.x % 8) * (T / 8) + blockIdx.x / 8;
-  const int d0 = static_cast<int>(q / ntn) * kTM2;
-  const int c0 = static_cast<int>(q % ntn) * kTN;
+  const int d0 = static_cast<int>(q / ntn) * TM;
+  const int c0 = static_cast<int>(q % ntn) * TN;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int wc = wave * 64;
-  const int ar = threadIdx.x >> 2, aq = threadIdx.x & 3;
+  const int wc = wave * 32 * CT;
+  const int ar = threadIdx.x / kParts, aq = threadIdx.x % kParts;
   // generated rows: the grid terms in LDS (read by every row)
   extern __shared__ __align__(16) double gterms[];  // GEN: [3][ng]
   if (GEN) {
     stage_grid_terms(gen.grid, ng, gterms);
     __syncthreads();
   }
-  RowBlocks<LOAD, GEN> src(A, nd, ng, d0 + ar, aq, gen, gterms);
-  float ra[16];
+  RowBlocks<LOAD, GEN, kPer> src(A, nd, ng, d0 + ar, aq, gen, gterms);
+  float ra[kPer];
   auto split_a = [&](int buf) {
 #pragma unroll
-    for (int k = 0; k < 2; ++k) {
+    for (int k = 0; k < kPer / 8; ++k) {
       bf16x8 h, m, l;
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
@@ -517,19 +523,19 @@ __global__ void __launch_bounds__(kThreads2, 2) mfma_contract_bf16(const float* 
         m[i] = b;
         l[i] = c;
       }
-      *reinterpret_cast<bf16x8*>(&As[buf][0][ar][aq * 16 + k * 8]) = h;
-      *reinterpret_cast<bf16x8*>(&As[buf][1][ar][aq * 16 + k * 8]) = m;
-      *reinterpret_cast<bf16x8*>(&As[buf][2][ar][aq * 16 + k * 8]) = l;
+      *reinterpret_cast<bf16x8*>(&As[buf][0][ar][aq * kPer + k * 8]) = h;
+      *reinterpret_cast<bf16x8*>(&As[buf][1][ar][aq * kPer + k * 8]) = m;
+      *reinterpret_cast<bf16x8*>(&As[buf][2][ar][aq * kPer + k * 8]) = l;
     }
   };
   const int kofs = (lane >> 5) * 8;
   const size_t b0 = packed_index(0, c0 + wc + (lane & 31), kofs, nbp);
   const int nsteps = nkb * (kKB / 16);
-  float16v acc[2][2];
+  float16v acc[RT][CT];
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
+  for (int i = 0; i < RT; ++i) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
+    for (int j = 0; j < CT; ++j) {
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
     }
@@ -539,11 +545,11 @@ __global__ void __launch_bounds__(kThreads2, 2) mfma_contract_bf16(const float* 
   src.load(min(1, nkb - 1), ra, nkb > 1);
   // K fragments two 16-g steps ahead: b? holds step s, n1? step s + 1; steps
   // past the last re-read the last
-  bf16x8 bh[2], bm[2], bl[2], n1h[2], n1m[2], n1l[2];
+  bf16x8 bh[CT], bm[CT], bl[CT], n1h[CT], n1m[CT], n1l[CT];
   auto load_b = [&](int step, bf16x8* h, bf16x8* m, bf16x8* l) {
     const size_t at = b0 + static_cast<size_t>(min(step, nsteps - 1)) * nbp * 16;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
+    for (int j = 0; j < CT; ++j) {
       h[j] = *reinterpret_cast<const bf16x8*>(Bh + at + j * 512);
       m[j] = *reinterpret_cast<const bf16x8*>(Bm + at + j * 512);
       l[j] = *reinterpret_cast<const bf16x8*>(Bl + at + j * 512);
@@ -556,20 +562,20 @@ __global__ void __launch_bounds__(kThreads2, 2) mfma_contract_bf16(const float* 
     const int cur = kb & 1;
 #pragma unroll
     for (int ks = 0; ks < kKB / 16; ++ks) {
-      bf16x8 nbh[2], nbm[2], nbl[2];
+      bf16x8 nbh[CT], nbm[CT], nbl[CT];
       load_b(kb * (kKB / 16) + ks + 2, nbh, nbm, nbl);
       const int kk = ks * 16 + kofs;
-      bf16x8 ah[2], am[2], al[2];
+      bf16x8 ah[RT], am[RT], al[RT];
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
+      for (int i = 0; i < RT; ++i) {
         ah[i] = *reinterpret_cast<const bf16x8*>(&As[cur][0][i * 32 + (lane & 31)][kk]);
         am[i] = *reinterpret_cast<const bf16x8*>(&As[cur][1][i * 32 + (lane & 31)][kk]);
         al[i] = *reinterpret_cast<const bf16x8*>(&As[cur][2][i * 32 + (lane & 31)][kk]);
       }
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
+      for (int i = 0; i < RT; ++i) {
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
+        for (int j = 0; j < CT; ++j) {
           // small terms first
           acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(am[i], bm[j], acc[i][j], 0, 0, 0);
           acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al[i], bh[j], acc[i][j], 0, 0, 0);
@@ -580,7 +586,7 @@ __global__ void __launch_bounds__(kThreads2, 2) mfma_contract_bf16(const float* 
         }
       }
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
+      for (int j = 0; j < CT; ++j) {
         bh[j] = n1h[j];
         bm[j] = n1m[j];
         bl[j] = n1l[j];
@@ -594,16 +600,16 @@ __global__ void __launch_bounds__(kThreads2, 2) mfma_contract_bf16(const float* 
     __syncthreads();  // buffer cur is free; buffer cur ^ 1 is written
   }
   // generated rows: divide by the row norms (via LDS, like the row scales)
-  __shared__ float rnorm[GEN ? kTM2 : 1];
+  __shared__ float rnorm[GEN ? TM : 1];
   if (GEN) {
     const float r = src.inv_norm();
-    rnorm[ar] = r;  // the row's four threads store the same value
+    rnorm[ar] = r;  // the row's threads store the same value
     __syncthreads();
   }
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
+  for (int i = 0; i < RT; ++i) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
+    for (int j = 0; j < CT; ++j) {
       const int c = c0 + wc + j * 32 + (lane & 31);
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
@@ -613,6 +619,43 @@ __global__ void __launch_bounds__(kThreads2, 2) mfma_contract_bf16(const float* 
         if (dd < nd && c < nb) __builtin_nontemporal_store(val, out + static_cast<size_t>(dd) * nb + c);
       }
     }
+  }
+}
+
+// Tile of a workgroup: RT x 32 rows by CT x 128 columns.
+template <int RT_, int CT_>
+struct Tile {
+  static constexpr int RT = RT_, CT = CT_;
+};
+
+// The 64 x 256 tile does the least work per product and is the one that keeps the
+// matrix cores busy, but a call with few of them leaves CUs idle through their
+// serial loop over g (3001 x 300 x 200 is 47 workgroups), and 256 columns waste
+// half of the last one where the bins end in its first half.  Measured, us per
+// call (rows given, split-BF16; generated), tiles 64 x 256, 32 x 256, 32 x 128:
+//     3001 x 300 x 200:   24.0 19.8 17.3;   34.4 25.7 21.8
+//     9000 x 512 x 512:   47.4 42.9 37.6;   50.8 43.3 49.6
+//    12000 x 512 x 512:   47.2 43.2 48.1;   51.3 46.5 57.1
+//    16384 x 512 x 512:   51.1 54.2 56.8;   55.4 59.0 72.4
+//    65536 x 512 x 512:  175.9 194.2 198.8; 188.6 200.8 255.9
+//    65536 x 512 x 128:   83.5 93.3 59.5;   89.9 96.1 73.1
+//    65536 x 300 x 300:  110.8 125.4 101.0; 138.8 140.3 133.6
+// So: 32 x 128 while five of them a CU hold the batch (one where rows are
+// generated: each column tile generates its rows again) and wherever 128 columns
+// come out odd; 32 x 256 while three a CU do.
+template <class Launch>
+void launch_tiles(size_t nd, int nb, bool generated, Launch launch) {
+  auto tiles = [&](int rt, int ct) { return ceil_div(nd, 32 * rt) * ceil_div(nb, 128 * ct); };
+  auto with = [&](auto t) {
+    launch(t, static_cast<unsigned>(tiles(t.RT, t.CT)), static_cast<int>(ceil_div(nb, 128 * t.CT)));
+  };
+  const size_t cus = num_cus();
+  if (ceil_div(nb, 128) % 2 == 1 || tiles(1, 1) <= (generated ? 1 : 5) * cus) {
+    with(Tile<1, 1>{});
+  } else if (tiles(1, 2) <= 3 * cus) {
+    with(Tile<1, 2>{});
+  } else {
+    with(Tile<2, 2>{});
   }
 }
 
@@ -638,11 +681,11 @@ void contraction_f16(const SyncPlan& plan, const float* d_gbeta, int ng, int dis
   // blocks when ng is a multiple of 64
   const bool vec = ng % 4 == 0 && reinterpret_cast<uintptr_t>(d_f) % 16 == 0;
   const int nd_i = static_cast<int>(nd);
-  const int ntn = nbp / kTN;
-  const unsigned grid = static_cast<unsigned>(ceil_div(nd, kTM2) * ntn);
   const int load = vec ? (ng % kKB == 0 ? 2 : 1) : 0;
-#define RGN_CONTRACT(P_, L_) \
-  mfma_contract2<P_, L_><<<grid, kThreads2, 0, st>>>(d_f, nd_i, ng, Bh, Bl, rB, nb, nbp, nkb, ntn, d_out)
+#define RGN_CONTRACT(P_, L_)                                                                                        \
+  launch_tiles(nd, nb, false, [&](auto t, unsigned grid, int ntn) {                                                      \
+    mfma_contract2<P_, L_, t.RT, t.CT><<<grid, kThreads2, 0, st>>>(d_f, nd_i, ng, Bh, Bl, rB, nb, nbp, nkb, ntn, d_out); \
+  })
 #define RGN_CONTRACT_P(P_)                   \
   do {                                       \
     if (load == 2) RGN_CONTRACT(P_, 2);      \
@@ -677,12 +720,12 @@ void contraction_f16_plaw(const SyncPlan& plan, const float* d_gbeta, int ng, in
   stage_mark(st, "pack_kernel_matrix");
   const GenRows gen{d_index, d_cutoff, d_gbeta};
   const size_t gsmem = 3 * sizeof(double) * static_cast<size_t>(ng);
-  const int ntn = nbp / kTN;
-  const unsigned grid = static_cast<unsigned>(ceil_div(nd, kTM2) * ntn);
   const int nd_i = static_cast<int>(nd);
 #define RGN_CONTRACT_GEN(P_, L_)                                                                            \
-  mfma_contract2<P_, L_, true><<<grid, kThreads2, gsmem, st>>>(nullptr, nd_i, ng, Bh, Bl, rB, nb, nbp, nkb, ntn, \
-                                                              d_out, gen)
+  launch_tiles(nd, nb, true, [&](auto t, unsigned grid, int ntn) {                                              \
+    mfma_contract2<P_, L_, t.RT, t.CT, true><<<grid, kThreads2, gsmem, st>>>(nullptr, nd_i, ng, Bh, Bl, rB, nb, \
+                                                                             nbp, nkb, ntn, d_out, gen);        \
+  })
   const bool full = ng % kKB == 0;
   if (nprod == 3) {
     if (full) RGN_CONTRACT_GEN(3, 2); else RGN_CONTRACT_GEN(3, 0);
@@ -715,24 +758,20 @@ void contraction_bf16(const SyncPlan& plan, const float* d_gbeta, int ng, int di
   RGN_HIP(hipGetLastError());
   stage_mark(st, "pack_kernel_matrix_bf16");
   const GenRows gen{d_index, d_cutoff, d_gbeta};
-  const int ntn = nbp / kTN;
-  const unsigned grid = static_cast<unsigned>(ceil_div(nd, kTM2) * ntn);
   const int nd_i = static_cast<int>(nd);
   const bool vec = ng % 4 == 0 && reinterpret_cast<uintptr_t>(d_f) % 16 == 0;
   const size_t gsmem = 3 * sizeof(double) * static_cast<size_t>(ng);
-  if (generated && ng % kKB == 0) {
-    mfma_contract_bf16<2, true><<<grid, kThreads2, gsmem, st>>>(nullptr, nd_i, ng, Bh, Bm, Bl, nb, nbp, nkb, ntn,
-                                                                d_out, gen);
-  } else if (generated) {
-    mfma_contract_bf16<0, true><<<grid, kThreads2, gsmem, st>>>(nullptr, nd_i, ng, Bh, Bm, Bl, nb, nbp, nkb, ntn,
-                                                                d_out, gen);
-  } else if (vec && ng % kKB == 0) {
-    mfma_contract_bf16<2, false><<<grid, kThreads2, 0, st>>>(d_f, nd_i, ng, Bh, Bm, Bl, nb, nbp, nkb, ntn, d_out, gen);
-  } else if (vec) {
-    mfma_contract_bf16<1, false><<<grid, kThreads2, 0, st>>>(d_f, nd_i, ng, Bh, Bm, Bl, nb, nbp, nkb, ntn, d_out, gen);
-  } else {
-    mfma_contract_bf16<0, false><<<grid, kThreads2, 0, st>>>(d_f, nd_i, ng, Bh, Bm, Bl, nb, nbp, nkb, ntn, d_out, gen);
-  }
+  launch_tiles(nd, nb, generated, [&](auto t, unsigned grid, int ntn) {
+#define RGN_CONTRACT_BF16(L_, G_)                                                                                   \
+  mfma_contract_bf16<L_, t.RT, t.CT, G_><<<grid, kThreads2, G_ ? gsmem : 0, st>>>(G_ ? nullptr : d_f, nd_i, ng, Bh, Bm, \
+                                                                                  Bl, nb, nbp, nkb, ntn, d_out, gen)
+    if (generated && ng % kKB == 0) RGN_CONTRACT_BF16(2, true);
+    else if (generated) RGN_CONTRACT_BF16(0, true);
+    else if (vec && ng % kKB == 0) RGN_CONTRACT_BF16(2, false);
+    else if (vec) RGN_CONTRACT_BF16(1, false);
+    else RGN_CONTRACT_BF16(0, false);
+#undef RGN_CONTRACT_BF16
+  });
   RGN_HIP(hipGetLastError());
   stage_mark(st, "mfma_contract_bf16");
 }
