@@ -337,28 +337,6 @@ __device__ __forceinline__ int densest_window(unsigned* hist, int NK, int len, u
 // A value that is the same in every lane of the wave, in a scalar register.
 __device__ __forceinline__ unsigned wave_uniform(unsigned v) { return __builtin_amdgcn_readfirstlane(v); }
 
-// v moved by a DPP control (lanes without a source, and rows outside ROW_MASK,
-// read 0).
-template <int CTRL, int ROW_MASK = 0xf>
-__device__ __forceinline__ double dpp_d(double v) {
-  constexpr bool kBound = ROW_MASK == 0xf;  // bound_ctrl supplies the zero: no register to clear first
-  const unsigned long long b = __double_as_longlong(v);
-  const unsigned lo = __builtin_amdgcn_update_dpp(0, static_cast<int>(b), CTRL, ROW_MASK, 0xf, kBound);
-  const unsigned hi = __builtin_amdgcn_update_dpp(0, static_cast<int>(b >> 32), CTRL, ROW_MASK, 0xf, kBound);
-  return __longlong_as_double(static_cast<unsigned long long>(hi) << 32 | lo);
-}
-
-// Inclusive sum over the lanes of a wave.
-__device__ __forceinline__ double wave_scan(double v) {
-  v += dpp_d<0x111>(v);  // row_shr 1, 2, 4, 8: within rows of 16 lanes
-  v += dpp_d<0x112>(v);
-  v += dpp_d<0x114>(v);
-  v += dpp_d<0x118>(v);
-  v += dpp_d<kDppRowBcast15, 0xa>(v);
-  v += dpp_d<kDppRowBcast31, 0xc>(v);
-  return v;
-}
-
 __device__ __forceinline__ double last_lane(double v) {
   const unsigned long long b = __double_as_longlong(v);
   const unsigned lo = __builtin_amdgcn_readlane(static_cast<int>(b), 63);
@@ -567,7 +545,7 @@ static_assert(kBinnedMaxNK <= 65535, "list entries keep the bucket in 16 bits");
 //      left is counting-sorted by bucket into LDS, as much at a time as fits,
 //      and each wave takes a bucket, reduces it into a row of its own and adds
 //      it as in 3 (source by source where there are few).
-//   5  The waves' spectra are added in order into partials[bin][block].
+//   5  The waves' spectra are added in order into partials[block][bin].
 template <int Q, bool HAS_E, bool NT>
 __global__ void __launch_bounds__(kStream) binned_stream(ParticlesDev D, unsigned n, BinnedDev P, StreamShape S,
                                                          float2* __restrict__ list_wp,
@@ -825,7 +803,7 @@ __global__ void __launch_bounds__(kStream) binned_stream(ParticlesDev D, unsigne
     const int l = r / Q, q = r % Q;
     double t = area[q * 64 + l];
     for (int w = 1; w < kWaves; ++w) t += area[(w * Q + q) * 64 + l];  // fixed order
-    partials[static_cast<size_t>(P.rinfo[r].r) * gridDim.x + blockIdx.x] = t * P.em.rB0;  // W is chi w B0
+    partials[static_cast<size_t>(blockIdx.x) * P.nbins + P.rinfo[r].r] = t * P.em.rB0;  // W is chi w B0
   }
 }
 
@@ -1635,7 +1613,7 @@ void sync_forward_binned(const SyncPlan& plan, const ParticlesDev& D, size_t n, 
   }
   RGN_HIP(hipGetLastError());
   stage_mark(st, "binned_stream");
-  launch_combine(plan, partials, static_cast<int>(grid), out, st);
+  launch_combine(plan, partials, plan.nbins, static_cast<int>(grid), out, st);
 }
 
 void sync_adjoint_binned(const SyncPlan& plan, const ParticlesDev& D, size_t n, const float* gbar, float* gw,

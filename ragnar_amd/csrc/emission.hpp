@@ -100,7 +100,7 @@ int resolve_method(const SyncPlan& plan, size_t n, int method, bool adjoint);
 PlanDev device_view(const SyncPlan& plan);
 size_t forward_smem(const SyncPlan& plan);
 int forward_grid(size_t n, int blocks_per_cu);
-void launch_combine(const SyncPlan& plan, const double* partials, int grid, float* out,
+void launch_combine(const SyncPlan& plan, const double* partials, int pitch, int grid, float* out,
                     hipStream_t st);
 
 // Particle pointers of the C ABI; they may be null only when n == 0.

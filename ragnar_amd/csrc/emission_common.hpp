@@ -542,4 +542,26 @@ __device__ __forceinline__ float wave_sum_to_lane63(float v) {
   return v;
 }
 
+// v moved by a DPP control (lanes without a source, and rows outside ROW_MASK,
+// read 0).
+template <int CTRL, int ROW_MASK = 0xf>
+__device__ __forceinline__ double dpp_d(double v) {
+  constexpr bool kBound = ROW_MASK == 0xf;  // bound_ctrl supplies the zero: no register to clear first
+  const unsigned long long b = __double_as_longlong(v);
+  const unsigned lo = __builtin_amdgcn_update_dpp(0, static_cast<int>(b), CTRL, ROW_MASK, 0xf, kBound);
+  const unsigned hi = __builtin_amdgcn_update_dpp(0, static_cast<int>(b >> 32), CTRL, ROW_MASK, 0xf, kBound);
+  return __longlong_as_double(static_cast<unsigned long long>(hi) << 32 | lo);
+}
+
+// Inclusive sum over the lanes of a wave.
+__device__ __forceinline__ double wave_scan(double v) {
+  v += dpp_d<0x111>(v);  // row_shr 1, 2, 4, 8: within rows of 16 lanes
+  v += dpp_d<0x112>(v);
+  v += dpp_d<0x114>(v);
+  v += dpp_d<0x118>(v);
+  v += dpp_d<kDppRowBcast15, 0xa>(v);
+  v += dpp_d<kDppRowBcast31, 0xc>(v);
+  return v;
+}
+
 }  // namespace rgn
