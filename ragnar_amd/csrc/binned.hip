@@ -1239,21 +1239,23 @@ __global__ void __launch_bounds__(kThreads) binned_evaluate(BinnedDev P, const d
                                                             float* __restrict__ out) {
   const int e = blockIdx.x;
   const BinInfo b = P.binfo[e];
+  const float ee = P.bine[e];
   __shared__ double red[kThreads / 64];
   const int M1 = P.M + 1;
+  const double alpha = b.A - b.a;
   double acc = 0.0;
   if (b.r >= 0) {
     const int klo = max(P.kmin, b.a - (P.T - 1)), khi = min(P.kmin + P.NK - 1, b.a);
     for (int k = klo + static_cast<int>(threadIdx.x); k <= khi; k += kThreads) {
       const int kk = k - P.kmin;
       const int m = b.a - k;
-      double Cp, sp, Cm, sm;
-      seg_line(P, b, k, m, Cp, sp);
-      seg_line(P, b, k, m - 1, Cm, sm);
+      // the bin's lines in this bucket (padded table: no branch ahead of the loads)
+      const double2 s1 = P.line[min(max(m + 1, 0), P.T)], s0 = P.line[min(max(m, 0), P.T)];
       const double* r0 = P0 + static_cast<size_t>(kk) * M1;
       const double* r1 = P1 + static_cast<size_t>(kk) * M1;
       const double p0 = r0[b.r], p1 = r1[b.r], t0 = r0[P.M], t1 = r1[P.M];
-      acc += (Cp * p0 - sp * p1) + (Cm * (t0 - p0) - sm * (t1 - p1));
+      const double Cp = fma(alpha, s1.y, s1.x), Cm = fma(alpha + 1.0, s0.y, s0.x);
+      acc += (Cp * p0 - s1.y * p1) + (Cm * (t0 - p0) - s0.y * (t1 - p1));
     }
   }
   // a fixed shuffle tree per wave, then the four wave sums in order
@@ -1264,7 +1266,6 @@ __global__ void __launch_bounds__(kThreads) binned_evaluate(BinnedDev P, const d
   if (threadIdx.x == 0) {
     double t = red[0];
     for (int w = 1; w < kThreads / 64; ++w) t += red[w];
-    const float ee = P.bine[e];
     out[e] = (b.r < 0 || ee == 0.0f) ? 0.0f : static_cast<float>(static_cast<double>(ee) * t);
   }
 }
