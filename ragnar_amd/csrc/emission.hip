@@ -239,20 +239,21 @@ __global__ void __launch_bounds__(kDistThreads) dist_kernel(DistSourceFn fn, int
 }
 
 // out[e] = e_e * sum_b partials[b][e] (fixed order), 0 for dead bins; pitch:
-// doubles of a row.  A block takes 16 bins, a cache line of each row, with 64
-// threads to a bin.  4 us, its launch and one trip to memory, whatever the split (4
-// to 16 bins a block, or a bin a block of partials[e][b]); rows instead of columns
-// are for the kernels that write them, a block's lines being its own: the forward
-// kernel at 2e5 particles and 200 bins 15.1 -> 13.5 us.
-constexpr int kCombineBins = 16;
+// doubles of a row.  A block takes BINS bins of each row: 16, a cache line, or 4
+// where 16 would leave a few blocks to read all rows (40 bins, 4096 rows: a call
+// of 38.5 us with 16, 34.8 with 4; 256 bins: 47.4 and 48.4).  Up to a thousand
+// rows it takes 4 us, its launch and one trip to memory, whatever the split;
+// rows instead of columns are for the kernels that write them, a block's lines
+// being its own: the forward kernel at 2e5 particles and 200 bins 15.1 -> 13.5 us.
 constexpr int kCombineThreads = 1024;
 
+template <int BINS>
 __global__ void __launch_bounds__(kCombineThreads) combine_kernel(const double* __restrict__ partials, int pitch,
                                                                   int nblocks, const float* __restrict__ bine,
                                                                   int nbins, float* __restrict__ out) {
-  constexpr int kParts = kCombineThreads / kCombineBins;
-  const int bin = threadIdx.x % kCombineBins, part = threadIdx.x / kCombineBins;
-  const int e = blockIdx.x * kCombineBins + bin;
+  constexpr int kParts = kCombineThreads / BINS;
+  const int bin = threadIdx.x % BINS, part = threadIdx.x / BINS;
+  const int e = blockIdx.x * BINS + bin;
   const double* column = partials + min(e, nbins - 1);
   const float ee = e < nbins ? bine[e] : 0.0f;
   double s = 0.0;
@@ -263,13 +264,13 @@ __global__ void __launch_bounds__(kCombineThreads) combine_kernel(const double* 
 #pragma unroll
     for (int k = 0; k < 8; ++k) s += v[k];
   }
-  // the wave's four parts, then the waves
-  s += __shfl_xor(s, 16);
-  s += __shfl_xor(s, 32);
-  __shared__ double red[kCombineThreads / 64][kCombineBins];
-  if ((threadIdx.x & 63) < kCombineBins) red[threadIdx.x / 64][bin] = s;
+  // the wave's parts, then the waves
+#pragma unroll
+  for (int w = BINS; w < 64; w <<= 1) s += __shfl_xor(s, w);
+  __shared__ double red[kCombineThreads / 64][BINS];
+  if ((threadIdx.x & 63) < BINS) red[threadIdx.x / 64][bin] = s;
   __syncthreads();
-  if (threadIdx.x < kCombineBins && e < nbins) {
+  if (threadIdx.x < BINS && e < nbins) {
     double t = red[0][bin];
 #pragma unroll
     for (int w = 1; w < kCombineThreads / 64; ++w) t += red[w][bin];
@@ -607,8 +608,13 @@ void launch_forward(const SyncPlan& plan, SourceFn fn, size_t n, int grid, doubl
 
 void launch_combine(const SyncPlan& plan, const double* partials, int pitch, int grid, float* out,
                     hipStream_t st) {
-  const unsigned blocks = static_cast<unsigned>(ceil_div(plan.nbins, kCombineBins));
-  combine_kernel<<<blocks, kCombineThreads, 0, st>>>(partials, pitch, grid, plan.bine.as<float>(), plan.nbins, out);
+  if (plan.nbins <= 64) {
+    combine_kernel<4><<<static_cast<unsigned>(ceil_div(plan.nbins, 4)), kCombineThreads, 0, st>>>(
+      partials, pitch, grid, plan.bine.as<float>(), plan.nbins, out);
+  } else {
+    combine_kernel<16><<<static_cast<unsigned>(ceil_div(plan.nbins, 16)), kCombineThreads, 0, st>>>(
+      partials, pitch, grid, plan.bine.as<float>(), plan.nbins, out);
+  }
   RGN_HIP(hipGetLastError());
   stage_mark(st, "combine_kernel");
 }
