@@ -130,7 +130,7 @@ __global__ void __launch_bounds__(256) pack_kernel_matrix(PlanDev P, const float
 // kb + 1 (already in registers) into the other buffer, and one barrier per
 // block orders the buffers.  K fragments are read by each wave straight from
 // the packed layout (1 MB for 512 x 512, resident in L2), one 16-g step
-// ahead.  The two workgroups of a CU meet at their own barriers only, so one's
+// ahead (DEEP: four).  The two workgroups of a CU meet at their own barriers only, so one's
 // rescale overlaps the other's matrix work.  Row and column scales are floats
 // (2^-s), so the rescale is one multiply and one FMA per element.  Workgroups
 // are numbered so that the column tiles of a row block run on one XCD (one
@@ -270,7 +270,7 @@ struct RowBlocks {
   }
 };
 
-template <int NPROD, int LOAD, int RT, int CT, bool GEN = false>
+template <int NPROD, int LOAD, int RT, int CT, bool DEEP, bool GEN = false>
 __global__ void __launch_bounds__(kThreads2, 2) mfma_contract2(const float* __restrict__ A, int nd, int ng,
                                                                const _Float16* __restrict__ Bh,
                                                                const _Float16* __restrict__ Bl,
@@ -342,11 +342,16 @@ __global__ void __launch_bounds__(kThreads2, 2) mfma_contract2(const float* __re
   src.load(0, ra, true);
   split_a(0);
   src.load(min(1, nkb - 1), ra, nkb > 1);
-  half8 bh[CT], bl[CT];
+  // K fragments kAhead steps ahead (slot d: step s + d)
+  constexpr int kAhead = DEEP ? 4 : 1;
+  half8 ring_h[kAhead][CT], ring_l[kAhead][CT];
 #pragma unroll
-  for (int j = 0; j < CT; ++j) {
-    bh[j] = ldb(Bh, 0, j);
-    if (NPROD == 3) bl[j] = ldb(Bl, 0, j);
+  for (int d = 0; d < kAhead; ++d) {
+#pragma unroll
+    for (int j = 0; j < CT; ++j) {
+      ring_h[d][j] = ldb(Bh, d, j);
+      if (NPROD == 3) ring_l[d][j] = ldb(Bl, d, j);
+    }
   }
   __syncthreads();
   for (int kb = 0; kb < nkb; ++kb) {
@@ -365,13 +370,15 @@ __global__ void __launch_bounds__(kThreads2, 2) mfma_contract2(const float* __re
     }
 #pragma unroll
     for (int ks = 0; ks < kKB / 16; ++ks) {
-      // next step's K fragments (the next block's first step after the last)
-      const int sn = min(kb * (kKB / 16) + ks + 1, nsteps - 1);
-      half8 nbh[CT], nbl[CT];
+      // the step's K fragments, and those of kAhead steps on in their place
+      const int sn = min(kb * (kKB / 16) + ks + kAhead, nsteps - 1);
+      half8 bh[CT], bl[CT];
 #pragma unroll
       for (int j = 0; j < CT; ++j) {
-        nbh[j] = ldb(Bh, sn, j);
-        if (NPROD == 3) nbl[j] = ldb(Bl, sn, j);
+        bh[j] = ring_h[ks % kAhead][j];
+        if (NPROD == 3) bl[j] = ring_l[ks % kAhead][j];
+        ring_h[ks % kAhead][j] = ldb(Bh, sn, j);
+        if (NPROD == 3) ring_l[ks % kAhead][j] = ldb(Bl, sn, j);
       }
       const int kk = ks * 16 + kofs;
       half8 ah[RT], al[RT];
@@ -390,11 +397,6 @@ __global__ void __launch_bounds__(kThreads2, 2) mfma_contract2(const float* __re
             tmp[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[i], bh[j], tmp[i][j], 0, 0, 0);
           }
         }
-      }
-#pragma unroll
-      for (int j = 0; j < CT; ++j) {
-        bh[j] = nbh[j];
-        if (NPROD == 3) bl[j] = nbl[j];
       }
       if (ks == 1) split_a(cur ^ 1);                                  // the next block's f
       if (ks == kKB / 16 - 1) src.load(min(kb + 2, nkb - 1), ra, kb + 2 < nkb);  // the one after
@@ -486,7 +488,7 @@ __global__ void __launch_bounds__(256) pack_kernel_matrix_bf16(PlanDev P, const 
   }
 }
 
-template <int LOAD, int RT, int CT, bool GEN>
+template <int LOAD, int RT, int CT, bool DEEP, bool GEN>
 __global__ void __launch_bounds__(kThreads2, 2) mfma_contract_bf16(const float* __restrict__ A, int nd, int ng,
                                                                    const __bf16* __restrict__ Bh,
                                                                    const __bf16* __restrict__ Bm,
@@ -543,9 +545,10 @@ __global__ void __launch_bounds__(kThreads2, 2) mfma_contract_bf16(const float* 
   src.load(0, ra, true);
   split_a(0);
   src.load(min(1, nkb - 1), ra, nkb > 1);
-  // K fragments two 16-g steps ahead: b? holds step s, n1? step s + 1; steps
-  // past the last re-read the last
-  bf16x8 bh[CT], bm[CT], bl[CT], n1h[CT], n1m[CT], n1l[CT];
+  // K fragments kAhead 16-g steps ahead: slot d of the ring holds step s + d;
+  // steps past the last re-read the last
+  constexpr int kAhead = DEEP ? 4 : 2;
+  bf16x8 ring_h[kAhead][CT], ring_m[kAhead][CT], ring_l[kAhead][CT];
   auto load_b = [&](int step, bf16x8* h, bf16x8* m, bf16x8* l) {
     const size_t at = b0 + static_cast<size_t>(min(step, nsteps - 1)) * nbp * 16;
 #pragma unroll
@@ -555,15 +558,21 @@ __global__ void __launch_bounds__(kThreads2, 2) mfma_contract_bf16(const float* 
       l[j] = *reinterpret_cast<const bf16x8*>(Bl + at + j * 512);
     }
   };
-  load_b(0, bh, bm, bl);
-  load_b(1, n1h, n1m, n1l);
+#pragma unroll
+  for (int d = 0; d < kAhead; ++d) load_b(d, ring_h[d], ring_m[d], ring_l[d]);
   __syncthreads();
   for (int kb = 0; kb < nkb; ++kb) {
     const int cur = kb & 1;
 #pragma unroll
     for (int ks = 0; ks < kKB / 16; ++ks) {
-      bf16x8 nbh[CT], nbm[CT], nbl[CT];
-      load_b(kb * (kKB / 16) + ks + 2, nbh, nbm, nbl);
+      bf16x8 bh[CT], bm[CT], bl[CT];
+#pragma unroll
+      for (int j = 0; j < CT; ++j) {
+        bh[j] = ring_h[ks % kAhead][j];
+        bm[j] = ring_m[ks % kAhead][j];
+        bl[j] = ring_l[ks % kAhead][j];
+      }
+      load_b(kb * (kKB / 16) + ks + kAhead, ring_h[ks % kAhead], ring_m[ks % kAhead], ring_l[ks % kAhead]);
       const int kk = ks * 16 + kofs;
       bf16x8 ah[RT], am[RT], al[RT];
 #pragma unroll
@@ -584,15 +593,6 @@ __global__ void __launch_bounds__(kThreads2, 2) mfma_contract_bf16(const float* 
           acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[i], bm[j], acc[i][j], 0, 0, 0);
           acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[i], bh[j], acc[i][j], 0, 0, 0);
         }
-      }
-#pragma unroll
-      for (int j = 0; j < CT; ++j) {
-        bh[j] = n1h[j];
-        bm[j] = n1m[j];
-        bl[j] = n1l[j];
-        n1h[j] = nbh[j];
-        n1m[j] = nbm[j];
-        n1l[j] = nbl[j];
       }
       if (ks == 1) split_a(cur ^ 1);                                  // the next block's f
       if (ks == kKB / 16 - 1) src.load(min(kb + 2, nkb - 1), ra, kb + 2 < nkb);  // the one after
@@ -622,10 +622,12 @@ __global__ void __launch_bounds__(kThreads2, 2) mfma_contract_bf16(const float* 
   }
 }
 
-// Tile of a workgroup: RT x 32 rows by CT x 128 columns.
-template <int RT_, int CT_>
+// Tile of a workgroup: RT x 32 rows by CT x 128 columns.  DEEP: K fragments four
+// 16-g steps ahead instead of one (split FP16) or two.
+template <int RT_, int CT_, bool DEEP_ = false>
 struct Tile {
   static constexpr int RT = RT_, CT = CT_;
+  static constexpr bool DEEP = DEEP_;
 };
 
 // The 64 x 256 tile does the least work per product and is the one that keeps the
@@ -642,15 +644,21 @@ struct Tile {
 //    65536 x 300 x 300:  110.8 125.4 101.0; 138.8 140.3 133.6
 // So: 32 x 128 while five of them a CU hold the batch (one where rows are
 // generated: each column tile generates its rows again) and wherever 128 columns
-// come out odd; 32 x 256 while three a CU do.
-template <class Launch>
-void launch_tiles(size_t nd, int nb, bool generated, Launch launch) {
+// come out odd; 32 x 256 while three a CU do.  A CU with one or two workgroups
+// waits for its K fragments in L2, so the smallest batches of given rows take
+// them four steps ahead (3001 x 512 x 512, FP16 24.7 -> 18.7 us, BF16 23.6 -> 21.2;
+// 3001 x 300 x 200, 16.8 -> 16.4); with more of them the registers cost more waves
+// (12000 x 512 x 512: 34.0 against 39.6 us), and generated rows gain nothing.
+template <bool GEN, class Launch>
+void launch_tiles(size_t nd, int nb, Launch launch) {
   auto tiles = [&](int rt, int ct) { return ceil_div(nd, 32 * rt) * ceil_div(nb, 128 * ct); };
   auto with = [&](auto t) {
     launch(t, static_cast<unsigned>(tiles(t.RT, t.CT)), static_cast<int>(ceil_div(nb, 128 * t.CT)));
   };
   const size_t cus = num_cus();
-  if (ceil_div(nb, 128) % 2 == 1 || tiles(1, 1) <= (generated ? 1 : 5) * cus) {
+  if (!GEN && tiles(1, 1) <= cus + cus / 2) {
+    with(Tile<1, 1, !GEN>{});
+  } else if (ceil_div(nb, 128) % 2 == 1 || tiles(1, 1) <= (GEN ? 1 : 5) * cus) {
     with(Tile<1, 1>{});
   } else if (tiles(1, 2) <= 3 * cus) {
     with(Tile<1, 2>{});
@@ -683,8 +691,8 @@ void contraction_f16(const SyncPlan& plan, const float* d_gbeta, int ng, int dis
   const int nd_i = static_cast<int>(nd);
   const int load = vec ? (ng % kKB == 0 ? 2 : 1) : 0;
 #define RGN_CONTRACT(P_, L_)                                                                                        \
-  launch_tiles(nd, nb, false, [&](auto t, unsigned grid, int ntn) {                                                      \
-    mfma_contract2<P_, L_, t.RT, t.CT><<<grid, kThreads2, 0, st>>>(d_f, nd_i, ng, Bh, Bl, rB, nb, nbp, nkb, ntn, d_out); \
+  launch_tiles<false>(nd, nb, [&](auto t, unsigned grid, int ntn) {                                                      \
+    mfma_contract2<P_, L_, t.RT, t.CT, t.DEEP><<<grid, kThreads2, 0, st>>>(d_f, nd_i, ng, Bh, Bl, rB, nb, nbp, nkb, ntn, d_out); \
   })
 #define RGN_CONTRACT_P(P_)                   \
   do {                                       \
@@ -722,8 +730,8 @@ void contraction_f16_plaw(const SyncPlan& plan, const float* d_gbeta, int ng, in
   const size_t gsmem = 3 * sizeof(double) * static_cast<size_t>(ng);
   const int nd_i = static_cast<int>(nd);
 #define RGN_CONTRACT_GEN(P_, L_)                                                                            \
-  launch_tiles(nd, nb, true, [&](auto t, unsigned grid, int ntn) {                                              \
-    mfma_contract2<P_, L_, t.RT, t.CT, true><<<grid, kThreads2, gsmem, st>>>(nullptr, nd_i, ng, Bh, Bl, rB, nb, \
+  launch_tiles<true>(nd, nb, [&](auto t, unsigned grid, int ntn) {                                              \
+    mfma_contract2<P_, L_, t.RT, t.CT, t.DEEP, true><<<grid, kThreads2, gsmem, st>>>(nullptr, nd_i, ng, Bh, Bl, rB, nb, \
                                                                              nbp, nkb, ntn, d_out, gen);        \
   })
   const bool full = ng % kKB == 0;
@@ -761,17 +769,17 @@ void contraction_bf16(const SyncPlan& plan, const float* d_gbeta, int ng, int di
   const int nd_i = static_cast<int>(nd);
   const bool vec = ng % 4 == 0 && reinterpret_cast<uintptr_t>(d_f) % 16 == 0;
   const size_t gsmem = 3 * sizeof(double) * static_cast<size_t>(ng);
-  launch_tiles(nd, nb, generated, [&](auto t, unsigned grid, int ntn) {
-#define RGN_CONTRACT_BF16(L_, G_)                                                                                   \
-  mfma_contract_bf16<L_, t.RT, t.CT, G_><<<grid, kThreads2, G_ ? gsmem : 0, st>>>(G_ ? nullptr : d_f, nd_i, ng, Bh, Bm, \
-                                                                                  Bl, nb, nbp, nkb, ntn, d_out, gen)
-    if (generated && ng % kKB == 0) RGN_CONTRACT_BF16(2, true);
-    else if (generated) RGN_CONTRACT_BF16(0, true);
-    else if (vec && ng % kKB == 0) RGN_CONTRACT_BF16(2, false);
-    else if (vec) RGN_CONTRACT_BF16(1, false);
-    else RGN_CONTRACT_BF16(0, false);
+#define RGN_CONTRACT_BF16(L_, G_)                                                                                     \
+  launch_tiles<G_>(nd, nb, [&](auto t, unsigned grid, int ntn) {                                                     \
+    mfma_contract_bf16<L_, t.RT, t.CT, t.DEEP, G_><<<grid, kThreads2, G_ ? gsmem : 0, st>>>(                         \
+      G_ ? nullptr : d_f, nd_i, ng, Bh, Bm, Bl, nb, nbp, nkb, ntn, d_out, gen);                                      \
+  })
+  if (generated && ng % kKB == 0) RGN_CONTRACT_BF16(2, true);
+  else if (generated) RGN_CONTRACT_BF16(0, true);
+  else if (vec && ng % kKB == 0) RGN_CONTRACT_BF16(2, false);
+  else if (vec) RGN_CONTRACT_BF16(1, false);
+  else RGN_CONTRACT_BF16(0, false);
 #undef RGN_CONTRACT_BF16
-  });
   RGN_HIP(hipGetLastError());
   stage_mark(st, "mfma_contract_bf16");
 }

@@ -30,7 +30,7 @@ def test_tiles_agree(precision, ng, nb):
     made = T.sync_fromdist_batched_plaw(plan, grid, p, xc, True, precision)
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     n128, n256 = -(-nb // 128), -(-nb // 256)
-    edges = [32 * (5 * cus // n128), 32 * (3 * cus // n256), 32 * (cus // n128)]
+    edges = [32 * (3 * cus // 2 // n128), 32 * (5 * cus // n128), 32 * (3 * cus // n256), 32 * (cus // n128)]
     for nd in sorted({1, 31, 32, 33, 65, *edges, *(e + 1 for e in edges)}):
         if nd >= MANY:
             continue
