@@ -462,12 +462,33 @@ __device__ __forceinline__ int cell_place(const uint2* __restrict__ lut, const f
   return (above ? c.x >> 16 : c.x) & 0xffffu;
 }
 
+// The table as its nodes see it: for node m = -1 .. T (index m + 1; zero at both
+// ends) the lines after and before it, each as value at the node and slope.  A
+// source in bucket k and a bin of m = a - k give
+//     F = value + slope (alpha - phi)
+// of the line after the node when phi <= alpha, else of the one before: one index
+// per bin and bucket, where lines starting at their own nodes took two (and
+// alpha + 1; 18 VALU instructions per bin instead of 14, and registers: the form
+// with E spilled).  5e6 particles with E at 200 bins 76.0 -> 74.4 us, 1e6 at 256
+// bins 34.4 -> 34.1; the bucket loop itself (7.5 us there) did not move, its LDS
+// reads hold it.
+__device__ __forceinline__ void stage_nodes(double2* __restrict__ node, const double2* __restrict__ line, int T,
+                                            int i) {
+  const double2 before = line[min(max(i - 1, 0), T)];
+  node[2 * i] = line[min(i, T)];
+  node[2 * i + 1] = make_double2(before.x + before.y, before.y);
+}
+
+__device__ __forceinline__ const double2* node_of(const double2* __restrict__ node, int T, int m) {
+  return node + 2 * min(static_cast<unsigned>(max(m + 1, 0)), static_cast<unsigned>(T + 1));
+}
+
 // Adds a bucket's moments to the lane's bins.  row: m0 of the M + 1 sub-cells
 // (row_place), then m1.  The lane's sub-cells are those of its bins, so the
 // prefix sums it needs end in its own registers.
 template <int Q>
 __device__ __forceinline__ void add_bucket(LaneBins<Q>& L, const double* __restrict__ row, int M, int k,
-                                           const double2* __restrict__ line, int T, int lane) {
+                                           const double2* __restrict__ node, int T, int lane) {
   const int width = row_width<Q>(M);
   double p0[Q], p1[Q];
 #pragma unroll
@@ -489,26 +510,23 @@ __device__ __forceinline__ void add_bucket(LaneBins<Q>& L, const double* __restr
 #pragma unroll
   for (int q = 0; q < Q; ++q) {
     const double P0 = x0 + p0[q], P1 = x1 + p1[q];
-    const int m = L.a[q] - k;
-    const double2 s1 = line[min(static_cast<unsigned>(max(m + 1, 0)), static_cast<unsigned>(T))];
-    const double2 s0 = line[min(static_cast<unsigned>(max(m, 0)), static_cast<unsigned>(T))];
-    // A_e - k = m + alpha = (m - 1) + (alpha + 1)
-    const double C1 = fma(L.alpha[q], s1.y, s1.x), C0 = fma(L.alpha[q] + 1.0, s0.y, s0.x);
-    double v = fma(C1, P0, fma(-s1.y, P1, L.acc[q]));
-    L.acc[q] = fma(C0, t0 - P0, fma(-s0.y, t1 - P1, v));
+    const double2* n = node_of(node, T, L.a[q] - k);
+    const double2 after = n[0], before = n[1];
+    const double C1 = fma(L.alpha[q], after.y, after.x), C0 = fma(L.alpha[q], before.y, before.x);
+    const double v = fma(C1, P0, fma(-after.y, P1, L.acc[q]));
+    L.acc[q] = fma(C0, t0 - P0, fma(-before.y, t1 - P1, v));
   }
 }
 
 // Adds one source to the lane's bins.
 template <int Q>
-__device__ __forceinline__ void add_source(LaneBins<Q>& L, float2 wp, int k, const double2* __restrict__ line, int T) {
+__device__ __forceinline__ void add_source(LaneBins<Q>& L, float2 wp, int k, const double2* __restrict__ node, int T) {
   const double W = wp.x, phi = wp.y;
 #pragma unroll
   for (int q = 0; q < Q; ++q) {
-    const int right = phi > L.alpha[q];  // the segment before
-    const double2 s = line[min(static_cast<unsigned>(max(L.a[q] - k - right + 1, 0)), static_cast<unsigned>(T))];
-    const double F = fma(-s.y, phi, fma(L.alpha[q] + right, s.y, s.x));
-    L.acc[q] = fma(W, F, L.acc[q]);
+    const int before = phi > L.alpha[q];
+    const double2 b = node_of(node, T, L.a[q] - k)[before];
+    L.acc[q] = fma(W, fma(b.y, L.alpha[q] - phi, b.x), L.acc[q]);
   }
 }
 
@@ -517,7 +535,7 @@ __device__ __forceinline__ void add_source(LaneBins<Q>& L, float2 wp, int k, con
 struct StreamShape {
   int rows;        // buckets in a window
   int area;        // doubles
-  int nline;       // entries of the line table in LDS
+  int nnode;       // entries of the node table in LDS
   int tail_waves;  // waves that reduce the end of the list, a row each
   unsigned stage;  // its sources, after those rows
   unsigned cap;    // list entries of a block
@@ -556,8 +574,8 @@ __global__ void __launch_bounds__(kStream) binned_stream(ParticlesDev D, unsigne
   const int M = P.M, NK = P.NK, JQ2 = min(P.JQ, kLutCells);
   const int width = row_width<Q>(M), pitch = 2 * Q * width;  // doubles of a row
   double2* l2 = reinterpret_cast<double2*>(smem);
-  double2* lline = l2 + kLog2Tab;
-  double* area = reinterpret_cast<double*>(lline + S.nline);
+  double2* node = l2 + kLog2Tab;
+  double* area = reinterpret_cast<double*>(node + S.nnode);
   uint2* lut = reinterpret_cast<uint2*>(area + S.area);
   float* athr = reinterpret_cast<float*>(lut + JQ2 + 1);
   unsigned* hist = reinterpret_cast<unsigned*>(athr + M + 4);  // NK
@@ -580,7 +598,7 @@ __global__ void __launch_bounds__(kStream) binned_stream(ParticlesDev D, unsigne
     hist[i] = 0u;
     done[i] = 0;
   }
-  for (int i = tid; i < S.nline; i += kStream) lline[i] = P.line[i];
+  for (int i = tid; i < S.nnode / 2; i += kStream) stage_nodes(node, P.line, P.T, i);
   for (int i = tid; i <= JQ2; i += kStream) {
     lut[i] = stage_cell<Q>(i < JQ2 ? P.sublut[i] : make_uint2(M, 0x7f800000u), width);  // phi rounded to 1
   }
@@ -593,7 +611,7 @@ __global__ void __launch_bounds__(kStream) binned_stream(ParticlesDev D, unsigne
     const int r = lane * Q + q;
     L.acc[q] = 0.0;
     L.alpha[q] = 0.0;
-    L.a[q] = -(1 << 30);  // no bin: every line is zero
+    L.a[q] = -(1 << 30);  // no bin: every node is zero
     if (r < M) {
       const BinInfo b = P.rinfo[r];
       L.alpha[q] = b.A;
@@ -671,7 +689,7 @@ __global__ void __launch_bounds__(kStream) binned_stream(ParticlesDev D, unsigne
     }
   };
   auto add_window = [&]() {
-    for (int i = wave; i < rows; i += kWaves) add_bucket<Q>(L, area + i * pitch, M, P.kmin + w0 + i, lline, P.T, lane);
+    for (int i = wave; i < rows; i += kWaves) add_bucket<Q>(L, area + i * pitch, M, P.kmin + w0 + i, node, P.T, lane);
   };
   for (unsigned base = blockIdx.x * kStream; base < n; base += 4 * stride) {
 #pragma unroll
@@ -776,7 +794,7 @@ __global__ void __launch_bounds__(kStream) binned_stream(ParticlesDev D, unsigne
           const int kk = wave_uniform(occ[i]), k = P.kmin + kk;
           const unsigned b0 = wave_uniform(offs[kk]) - first, b1 = wave_uniform(offs[kk + 1]) - first;
           if (b1 - b0 <= kSparse) {
-            for (unsigned b = b0; b < b1; ++b) add_source<Q>(L, staged[b], k, lline, P.T);
+            for (unsigned b = b0; b < b1; ++b) add_source<Q>(L, staged[b], k, node, P.T);
             continue;
           }
           for (int c = lane; c < pitch; c += 64) row[c] = 0.0;
@@ -789,7 +807,7 @@ __global__ void __launch_bounds__(kStream) binned_stream(ParticlesDev D, unsigne
             atomicAdd(m + Q * width, wd * static_cast<double>(wp.y));
           }
           wave_lds_fence();
-          add_bucket<Q>(L, row, M, k, lline, P.T, lane);
+          add_bucket<Q>(L, row, M, k, node, P.T, lane);
           wave_lds_fence();  // the row has been read
         }
       }
@@ -1534,9 +1552,8 @@ static StreamShape stream_shape(const SyncPlan& plan, int Q, size_t& smem) {
   const size_t M = plan.M, NK = plan.NK;
   const size_t rest = sizeof(double2) * kLog2Tab + sizeof(uint2) * (std::min(plan.JQ, kLutCells) + 1) +
                       sizeof(float) * (M + 4) + sizeof(unsigned) * (2 * NK + 1) + 3 * NK;
-  const size_t lines = sizeof(double2) * (static_cast<size_t>(plan.T) + 1);
-  S.nline = plan.T + 1;
-  const size_t fixed = rest + lines + 16;
+  S.nnode = 2 * (plan.T + 2);
+  const size_t fixed = rest + sizeof(double2) * S.nnode + 16;
   const size_t budget = kLdsPerCU - 512;  // the static words
   S.area = static_cast<int>((budget - fixed) / sizeof(double)) & ~1;
   const int pitch = 2 * Q * (plan.M / Q + 1);
