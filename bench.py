@@ -254,9 +254,9 @@ def summarize_compute(trace_dir, pmc_dir):
           "Made by `python bench.py --summarize-compute <trace> <pmc>` from two rocprofv3 runs of",
           "`bench.py --profile-compute` (commands in profiles/README.md): the pair-by-pair",
           "forward at 2^24 particles x 256 bins, the batched contraction at 65536 x 512 x 512",
-          "(split FP16 `mfma_contract2<3, 2, 2, 2, false>`: three products, f read as whole 64-g blocks,",
-          "`<1, 2, 2, 2, false>`: one product; split BF16 `mfma_contract_bf16<2, 2, 2, false>`: six products;",
-          "`mfma_contract2<3, 2, 2, 2, true>` and `mfma_contract_bf16<2, 2, 2, true>`: rows generated in the",
+          "(split FP16 `mfma_contract2<3, 2, 2, 2, false, false>`: three products, f read as whole 64-g blocks,",
+          "`<1, 2, 2, 2, false, false>`: one product; split BF16 `mfma_contract_bf16<2, 2, 2, false, false>`: six products;",
+          "`mfma_contract2<3, 2, 2, 2, false, true>` and `mfma_contract_bf16<2, 2, 2, false, true>`: rows generated in the",
           "kernel) and the inverse-Compton",
           "spectrum at 1000 gamma x 1000 soft-photon x 1000 output bins (`ic_kernel`).  The",
           "matrix rate counts every product pass (2 x 65536 x 512 x 512 flop each) over the traced",
