@@ -23,9 +23,9 @@
 // Pairs where rounding could decide differently (q within 2e-6 / (1 - x) of 1:
 // the reference's limit is good to 2.4e-7 / (1 - x)) and operands outside the
 // ranges below take the reference's own operations.
-// Per call, before and after: 200^3 27.7 and 16.2 us (of it the kernel 23.4 and
-// 11.5: the loop's 125000 wave steps take 4.4, loading, staging and the reduction
-// the rest), 500^3 243 and 92, 1000^3 1596 and 552 us (87 clocks a step of 64 pairs).
+// Per call, before and after: 200^3 27.6 and 15.5 us (of it the kernel 23.4 and
+// 11: the loop's 125000 wave steps take 4.4, loading, staging and the reduction
+// the rest), 500^3 243 and 75, 1000^3 1596 and 452 us (71 clocks a step of 64 pairs).
 #include <algorithm>
 #include <cmath>
 
@@ -94,11 +94,16 @@ __device__ __forceinline__ IcGamma ic_gamma(float g, float f, float e_ic, int g_
   return o;
 }
 
-// One workgroup per (output bin, chunk of gamma bins).  The pairs of a stage go
-// to the threads in turn, soft-photon bins fastest, so that every lane has a
-// pair whatever the counts; the block's FP64 sum goes to partial[chunk][bin], or
-// to the result where there is one chunk.  Summation order: per thread, stage by
-// stage, its pairs in order; then a fixed tree over the threads.
+// One workgroup per (output bin, chunk of gamma bins); its FP64 sum goes to
+// partial[chunk][bin], or to the result where there is one chunk.  The pairs of a
+// stage go to the threads
+//   ROWS   64 soft-photon bins to a wave at a time, every fourth gamma bin: a soft-
+//          photon bin's factors stay in registers;
+//   else   in turn, soft-photon bins fastest, so that every lane has a pair
+//          whatever the counts.
+// Summation order: per thread, stage by stage, its pairs in order; then a fixed
+// tree over the threads.
+template <bool ROWS>
 __global__ void __launch_bounds__(kIcThreads) ic_kernel(const float* __restrict__ g, const float* __restrict__ fg,
                                                         int ng, int g_log, const float* __restrict__ es,
                                                         const float* __restrict__ fes, int nes,
@@ -110,7 +115,22 @@ __global__ void __launch_bounds__(kIcThreads) ic_kernel(const float* __restrict_
   const int e = blockIdx.x, neic = gridDim.x, tid = threadIdx.x;
   const float e_ic = eic[e];
   const int g0 = blockIdx.y * gper, g1 = min(ng, g0 + gper);
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   double acc = 0.0;
+  auto pair = [&](const IcGamma& G, float r, float fs_es, int si) {
+    const float q = G.c * r;
+    if (q > G.hi) return;
+    float term;
+    if (q <= G.lo && q >= kIcMinQ) {
+      const float first = 2.0f * q * (__builtin_amdgcn_logf(q) * 0.6931471805599453f);
+      const float kn = static_cast<float>(fma(static_cast<double>(1.0f - q),
+                                              static_cast<double>(1.0f + 2.0f * q) + G.h, static_cast<double>(first)));
+      term = G.f * fs_es * e_ic * e_ic * kn * G.ig;
+    } else {
+      term = ic_term(G.g, G.f, es[si], fs_es, e_ic, g_log);
+    }
+    acc += static_cast<double>(term);
+  };
   for (int ss = 0; ss < nes; ss += kIcSoft) {
     const int ms = min(kIcSoft, nes - ss);
     const int di = kIcThreads / ms, ds = kIcThreads % ms;  // a step of kIcThreads pairs
@@ -140,28 +160,21 @@ __global__ void __launch_bounds__(kIcThreads) ic_kernel(const float* __restrict_
         }
       }
       __syncthreads();
-      int i = tid / ms, si = tid % ms;
-      while (i < mg) {
-        const IcGamma G = s_g[i];
-        const float fs_es = s_f[si], q = G.c * s_r[si];
-        if (!(q > G.hi)) {
-          float term;
-          if (q <= G.lo && q >= kIcMinQ) {
-            const float first = 2.0f * q * (__builtin_amdgcn_logf(q) * 0.6931471805599453f);
-            const float kn = static_cast<float>(fma(static_cast<double>(1.0f - q),
-                                                    static_cast<double>(1.0f + 2.0f * q) + G.h,
-                                                    static_cast<double>(first)));
-            term = G.f * fs_es * e_ic * e_ic * kn * G.ig;
-          } else {
-            term = ic_term(G.g, G.f, es[ss + si], fs_es, e_ic, g_log);
-          }
-          acc += static_cast<double>(term);
+      if constexpr (ROWS) {
+        for (int si = lane; si < ms; si += 64) {
+          const float r = s_r[si], fs_es = s_f[si];
+          for (int i = wave; i < mg; i += kIcThreads / 64) pair(s_g[i], r, fs_es, ss + si);
         }
-        i += di;
-        si += ds;
-        if (si >= ms) {
-          si -= ms;
-          ++i;
+      } else {
+        int i = tid / ms, si = tid % ms;
+        while (i < mg) {
+          pair(s_g[i], s_r[si], s_f[si], ss + si);
+          i += di;
+          si += ds;
+          if (si >= ms) {
+            si -= ms;
+            ++i;
+          }
         }
       }
     }
@@ -228,8 +241,13 @@ int rgn_ic_spectrum(const float* d_g, const float* d_fg, int ng, int g_log, cons
     const int gper = std::max(1, (ng + chunks - 1) / chunks);
     const int nchunk = std::max(1, (ng + gper - 1) / gper);  // at most 16 CUs + 1
     double* partial = static_cast<double*>(scratch(sizeof(double) * nchunk * static_cast<size_t>(neic), 17));
-    ic_kernel<<<dim3(neic, nchunk), kIcThreads, 0, st>>>(d_g, d_fg, ng, g_log ? 1 : 0, d_es, d_fes, nes, d_eic,
-                                                         gper, partial, d_out);
+    // Rows where they fill three quarters of their lanes and a block has 8000
+    // pairs: 500^3 92 -> 76 us, 300 x 300 x 400 32.5 -> 30.2; with fewer they are
+    // slower (400 x 300 x 60, 4100 pairs a block: 15.6 against 16.5).
+    const bool rows = 4 * nes >= 3 * ((nes + 63) / 64 * 64) && pairs >= 8000.0 * nchunk;
+    auto kernel = rows ? ic_kernel<true> : ic_kernel<false>;
+    kernel<<<dim3(neic, nchunk), kIcThreads, 0, st>>>(d_g, d_fg, ng, g_log ? 1 : 0, d_es, d_fes, nes, d_eic, gper,
+                                                      partial, d_out);
     RGN_HIP(hipGetLastError());
     stage_mark(st, "ic_kernel");
     if (nchunk == 1) return;

@@ -1,6 +1,7 @@
 """The inverse-Compton kernel forms a pair's q from per-bin factors and decides
 the kinematic limit by q away from it.  Counts at the edges of its stages (128
-gamma bins, 512 soft-photon bins, 256 threads) and of its chunks, and operands
+gamma bins, 512 soft-photon bins, 256 threads), of its chunks and of its row form
+(8000 pairs a block, rows three quarters full), and operands
 it must leave to the reference's own operations: output energies at and next to
 gamma (x = 1), zero output and soft-photon energies, tiny and huge values.
 
@@ -38,7 +39,8 @@ def _check(orc, g, fg, g_log, es, fes, E):
 
 
 @pytest.mark.parametrize("ng,ns,ne", [(1, 1, 60), (128, 1, 40), (129, 3, 40), (127, 255, 30), (257, 256, 7),
-                                      (40, 513, 30), (3, 511, 300), (300, 512, 2), (131, 257, 1)])
+                                      (40, 513, 30), (3, 511, 300), (300, 512, 2), (131, 257, 1),
+                                      (150, 64, 2100), (130, 560, 1100), (90, 111, 4100)])
 @pytest.mark.parametrize("g_log", [True, False])
 def test_ic_counts(orc, ng, ns, ne, g_log):
     rng = np.random.default_rng(ng * 1000 + ns)
