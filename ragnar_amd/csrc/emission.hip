@@ -637,10 +637,15 @@ int resolve_method(const SyncPlan& plan, size_t n, int method, bool adjoint) {
     // Forward at 256 bins, pair by pair against factorised: 2^18 22.5 / 29, 2^19
     // 31.5 / 31, 2^20 48 / 34 us; at 512 bins 2^19 50 / 48 us.
     static const double c_fwd[9] = {0, 21e-12, 21e-12, 26e-12, 27e-12, 31e-12, 34e-12, 44e-12, 53e-12};
-    static const double c_adj[9] = {0, 25e-12, 27e-12, 39e-12, 39e-12, 61e-12, 61e-12, 67e-12, 67e-12};
+    // Adjoint: between 1.5e5 and 3.3e5 particles the pair-by-pair form is up to 4 us
+    // faster since it skips blocks, but where a particle's terms nearly cancel its
+    // FP32 sums are further off (a log-residual loss at 2.7e5 particles and 149
+    // bins: 1.3e-5 against 1.1e-5 of the gradient's norm), so the line stays where
+    // the two once met.
+    static const double c_adj[9] = {0, 27e-12, 34e-12, 43e-12, 52e-12, 63e-12, 74e-12, 84e-12, 95e-12};
     const double nd = static_cast<double>(n);
     const int nbk = std::min(std::max(plan.NB, 1), 8);
-    const double t_direct = adjoint ? 20e-6 + nd * c_adj[nbk] : 18e-6 + nd * c_fwd[nbk];
+    const double t_direct = adjoint ? 25e-6 + nd * c_adj[nbk] : 18e-6 + nd * c_fwd[nbk];
     const double t_fwd = !stream_form(plan) ? std::max(47e-6, 35e-6 + nd * 8.2e-12)
                          : plan.M <= 128    ? 22e-6 + nd * 4.1e-12
                                             : 28e-6 + nd * 5.7e-12;
