@@ -768,6 +768,7 @@ __global__ void __launch_bounds__(kStream) binned_stream(ParticlesDev D, unsigne
       if (has) occ[nocc + at] = static_cast<unsigned short>(k);
       nocc += all;
     }
+    __syncthreads();  // occ and offs[NK] are in LDS: every wave reads them for its rounds
     float2* staged = reinterpret_cast<float2*>(area + S.tail_waves * pitch);
     // rounds of whole buckets that fit the staging space (all of them, mostly)
     for (unsigned i0 = 0, i1; i0 < nocc; i0 = i1) {

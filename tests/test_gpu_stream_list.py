@@ -1,0 +1,46 @@
+"""The factorised forward's list of sources outside the window, against the FP64
+sum of the plan's interpolant to 1e-6 of the spectrum's norm (each source is a
+float weight times an FP64 value: float rounding, 6e-8).
+
+Sparse lists: one to a few hundred sources in buckets far below or far above
+the window, so that the waves which own those buckets are few and the others
+have nothing to store before the rounds begin."""
+import numpy as np
+import pytest
+import torch
+
+from ragnar_amd import torch_ops as T
+from test_gpu_stream_form import _reference
+
+pytestmark = pytest.mark.gpu
+
+
+def _isotropic(gamma, seed=11):
+    """u of the given moduli, B = z."""
+    n = len(gamma)
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    c = 2 * torch.rand(n, generator=g, device="cuda", dtype=torch.float64) - 1
+    phi = 2 * np.pi * torch.rand(n, generator=g, device="cuda", dtype=torch.float64)
+    s = torch.sqrt(1 - c * c)
+    u = (torch.stack([s * torch.cos(phi), s * torch.sin(phi), c]) * torch.as_tensor(gamma, device="cuda")).float()
+    b = torch.zeros(3, n, device="cuda")
+    b[2] = 1.0
+    return u.contiguous(), b
+
+
+@pytest.mark.parametrize("low,high", [(1, 0), (0, 1), (2, 3), (0, 40), (300, 0), (70, 300)])
+@pytest.mark.parametrize("nb", [64, 256])
+def test_sparse_list(low, high, nb):
+    n = 40009
+    rng = np.random.default_rng(low * 1000 + high)
+    gamma = 30.0 * 1.5 ** rng.random(n)
+    at = rng.permutation(n)[: low + high]
+    gamma[at[:low]] = 1.5 * 1.6 ** rng.random(low)
+    gamma[at[low:]] = 500.0 * 2.0 ** rng.random(high)
+    u, b = _isotropic(gamma)
+    table = T.default_table()
+    plan = T.SyncPlan(table, np.logspace(-2, 6, nb).astype(np.float32))
+    ref = _reference(plan, table, u, b, None, None)
+    for _ in range(3):
+        got = T.sync_spectrum(plan, u, b, method="binned").double()
+        assert torch.linalg.norm(got - ref) <= 1e-6 * torch.linalg.norm(ref)
