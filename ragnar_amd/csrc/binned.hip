@@ -352,7 +352,7 @@ __device__ __forceinline__ double rsqrt_nr(double x) {
   return fma(y * e, fma(e, 0.375, 0.5), y);
 }
 
-// One particle of the forward pass in FP64: its weight W times B0, and B = k +
+// One particle of the forward pass in FP64: its weight W = chi w, and B = k +
 // phi (k counted from kmin); false when it contributes nowhere.  With G = gamma
 // V = gamma E + u x B and Q = |G|^2 - (u.E)^2 = gamma^2 rootQ^2, the emission
 // terms need one reciprocal square root y = (Q gamma^2)^(-1/2):
@@ -388,7 +388,8 @@ __device__ __forceinline__ bool stream_source(const RawParticle& r, const Binned
   const double x = Q * g2;
   const double y = rsqrt_nr(x);
   const double e = x * y * P.c_peak;
-  o.W = Q * y * static_cast<double>(r.w);
+  // W in the plan's units (fields over B0): the list keeps it as a float
+  o.W = Q * y * P.em.rB0 * static_cast<double>(r.w);
   const unsigned long long bits = __double_as_longlong(e);
   const unsigned hi = static_cast<unsigned>(bits >> 32);
   constexpr unsigned kLo = (1023u - 149u) << 20, kHi = (1023u + 128u) << 20;  // 2^-149 <= e < 2^128
@@ -822,7 +823,7 @@ __global__ void __launch_bounds__(kStream) binned_stream(ParticlesDev D, unsigne
     const int l = r / Q, q = r % Q;
     double t = area[q * 64 + l];
     for (int w = 1; w < kWaves; ++w) t += area[(w * Q + q) * 64 + l];  // fixed order
-    partials[static_cast<size_t>(blockIdx.x) * P.nbins + P.rinfo[r].r] = t * P.em.rB0;  // W is chi w B0
+    partials[static_cast<size_t>(blockIdx.x) * P.nbins + P.rinfo[r].r] = t;
   }
 }
 

@@ -4,13 +4,17 @@ float weight times an FP64 value: float rounding, 6e-8).
 
 Sparse lists: one to a few hundred sources in buckets far below or far above
 the window, so that the waves which own those buckets are few and the others
-have nothing to store before the rounds begin."""
+have nothing to store before the rounds begin.
+
+Units: fields and B0 scaled together, with particle weights such that chi w is
+an ordinary float while its product with B0 is beyond, or below, a float's
+range.  The spectrum is that of the unscaled fields times the weight."""
 import numpy as np
 import pytest
 import torch
 
 from ragnar_amd import torch_ops as T
-from test_gpu_stream_form import _reference
+from test_gpu_stream_form import _population, _reference
 
 pytestmark = pytest.mark.gpu
 
@@ -44,3 +48,16 @@ def test_sparse_list(low, high, nb):
     for _ in range(3):
         got = T.sync_spectrum(plan, u, b, method="binned").double()
         assert torch.linalg.norm(got - ref) <= 1e-6 * torch.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("b0,weight", [(1e12, 1e27), (1e-20, 1e-22), (1e-12, 1e-28), (1e30, 1.0)])
+def test_units_of_the_fields(b0, weight):
+    b0 = 2.0 ** round(np.log2(b0))  # exact: the scaled fields are the same multiples of B0
+    n = 300007
+    u, b = _population("power", n)
+    table = T.default_table()
+    bins = np.logspace(-2, 6, 256).astype(np.float32)
+    plan = T.SyncPlan(table, bins, B0=b0)
+    got = T.sync_spectrum(plan, u, b * b0, torch.full((n,), weight, device="cuda"), method="binned").double()
+    ref = _reference(plan, table, u, b, None, None) * float(np.float32(weight))
+    assert torch.linalg.norm(got - ref) <= 1e-6 * torch.linalg.norm(ref)
