@@ -352,6 +352,14 @@ __device__ __forceinline__ double rsqrt_nr(double x) {
   return fma(y * e, fma(e, 0.375, 0.5), y);
 }
 
+// The largest of three absolute values; a NaN among them may be left out.
+// (fmaxf would quiet each operand first, three instructions more.)
+__device__ __forceinline__ float max3_abs(float a, float b, float c) {
+  float r;
+  asm("v_max3_f32 %0, |%1|, |%2|, |%3|" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
+}
+
 // One particle of the forward pass in FP64: its weight W = chi w, and B = k +
 // phi (k counted from kmin); false when it contributes nowhere.  With G = gamma
 // V = gamma E + u x B and Q = |G|^2 - (u.E)^2 = gamma^2 rootQ^2, the emission
@@ -361,7 +369,10 @@ __device__ __forceinline__ double rsqrt_nr(double x) {
 // momenta, chi and e_peak); half the instructions of omega_terms_approx and
 // log2_tab, in a pass that issues vector instructions most of its time.
 // e_peak outside the float range (0, infinite, negative, NaN) drops the
-// particle, as synchrotron.hpp:162 does.  tab: stage_log2's table.
+// particle, as synchrotron.hpp:162 does; so do a chi that rounds to zero or
+// infinity as a float, and a momentum whose square overflows one, for which the
+// reference's e_peak (and that of the other kernels) is zero, infinite or NaN.
+// tab: stage_log2's table.
 struct StreamSource {
   double W, phi;
   int k;
@@ -388,12 +399,15 @@ __device__ __forceinline__ bool stream_source(const RawParticle& r, const Binned
   const double x = Q * g2;
   const double y = rsqrt_nr(x);
   const double e = x * y * P.c_peak;
-  // W in the plan's units (fields over B0): the list keeps it as a float
-  o.W = Q * y * P.em.rB0 * static_cast<double>(r.w);
+  // chi and W in the plan's units (fields over B0): the list keeps W as a float
+  const double chi = Q * y * P.em.rB0;
+  o.W = chi * static_cast<double>(r.w);
   const unsigned long long bits = __double_as_longlong(e);
   const unsigned hi = static_cast<unsigned>(bits >> 32);
-  constexpr unsigned kLo = (1023u - 149u) << 20, kHi = (1023u + 128u) << 20;  // 2^-149 <= e < 2^128
-  const bool in_range = hi - kLo < kHi - kLo;
+  const unsigned hi_chi = static_cast<unsigned>(__double_as_longlong(chi) >> 32);
+  constexpr unsigned kLo = (1023u - 149u) << 20, kHi = (1023u + 128u) << 20;  // 2^-149 <= e, chi < 2^128
+  const bool in_range = (hi - kLo < kHi - kLo) & (hi_chi - kLo < kHi - kLo) &
+                        (max3_abs(r.ux, r.uy, r.uz) < 0x1p64f);  // the first float whose square overflows
   const double mf = __longlong_as_double(static_cast<long long>(
     (bits & 0x000fffffffffffffull) | 0x3fe0000000000000ull));  // [0.5, 1)
   const double2 t = tab[(hi >> 12) & (kLog2Tab - 1)];

@@ -8,7 +8,11 @@ have nothing to store before the rounds begin.
 
 Units: fields and B0 scaled together, with particle weights such that chi w is
 an ordinary float while its product with B0 is beyond, or below, a float's
-range.  The spectrum is that of the unscaled fields times the weight."""
+range.  The spectrum is that of the unscaled fields times the weight.
+
+Particles that the reference's float steps drop (a momentum whose square
+overflows, a chi that overflows or vanishes as a float) add nothing, as in the
+pair-by-pair form."""
 import numpy as np
 import pytest
 import torch
@@ -61,3 +65,25 @@ def test_units_of_the_fields(b0, weight):
     got = T.sync_spectrum(plan, u, b * b0, torch.full((n,), weight, device="cuda"), method="binned").double()
     ref = _reference(plan, table, u, b, None, None) * float(np.float32(weight))
     assert torch.linalg.norm(got - ref) <= 1e-6 * torch.linalg.norm(ref)
+
+
+def test_particles_outside_the_float_range():
+    u, b = _population("power", 6000)
+    bins = np.logspace(-2, 6, 200).astype(np.float32)
+    # momenta around 2^64, the first float whose square is infinite, one component at a time
+    edge = np.float32(2.0 ** 64)
+    plan = T.SyncPlan(T.default_table(), bins, g_syn=1e19)
+    one = torch.zeros(3, 6000, device="cuda")
+    m = torch.tensor(np.array([edge, np.nextafter(edge, np.float32(0)), edge / 8, 1.5 * edge], np.float32), device="cuda")
+    i = torch.arange(6000, device="cuda")
+    one[i % 3, i] = m[i % 4]
+    for un in (one, u / u.norm(dim=0) * float(edge)):
+        want = T.sync_spectrum(plan, un, b, method="direct").double()
+        got = T.sync_spectrum(plan, un, b, method="binned").double()
+        assert 0 < torch.linalg.norm(want)
+        assert torch.linalg.norm(got - want) <= 1e-6 * torch.linalg.norm(want)
+    # chi beyond, and below, a float's range with e_peak inside it
+    for field, b0, g_syn in ((1e38, 1e-3, 1e18), (1e-43, 1e5, 1e-17)):
+        plan = T.SyncPlan(T.default_table(), bins, B0=b0, g_syn=g_syn)
+        for method in ("direct", "binned"):
+            assert not torch.any(T.sync_spectrum(plan, u, b * field, method=method)), (field, method)
