@@ -13,7 +13,9 @@
 // the kernel compares |u|^2 with floats and never forms the
 // energy for the index.  It starts from a float log2 estimate of the index, which
 // the plan checks to be within one bin everywhere, and corrects it by the
-// thresholds on its two sides (plans that fail the check walk): the result
+// thresholds on its two sides (plans that fail the check walk, and so do those
+// with a threshold among the subnormals, whose log2 the hardware takes to be
+// that of zero): the result
 // equals the reference expression bit for bit, whatever the device log does.
 //
 // Accumulation.  Each wave owns private LDS histograms (uint32 counts and FP64
@@ -160,7 +162,8 @@ void build_thresholds(rgn_hist_plan& plan) {
     bool near = scale * (std::fabs(lo) + std::fabs(hi) + 2.0) * 1e-6 < 0.1;
     for (size_t k = 1; k < n && near; ++k) {
       const double q = t[k];
-      if (!(q < inf)) {
+      // the kernel's log2 reads a subnormal |u|^2 as zero
+      if (!(q < inf) || (fourvel && q > 0.0 && q < std::numeric_limits<float>::min())) {
         near = false;
         break;
       }
