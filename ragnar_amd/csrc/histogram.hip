@@ -21,7 +21,7 @@
 // Accumulation.  Each wave owns private LDS histograms (uint32 counts and FP64
 // sums of the per-particle float terms); blocks write per-block partials that a
 // second kernel combines in a fixed order.  Counts are exact integers; sums are
-// the FP64 sum of float terms, rounded to float once.
+// the FP64 sum of the reference's float terms, rounded to float once.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -177,10 +177,11 @@ void build_thresholds(rgn_hist_plan& plan) {
   RGN_HIP(hipMemcpy(plan.d_thr.ptr, thr.data(), plan.d_thr.bytes, hipMemcpyHostToDevice));
 }
 
-// (float)(1 / E) of particles.cpp:247-252 for log-spaced bins, E = sqrt(q) or
-// sqrt(1 + q).  |u|: a float reciprocal square root with one Newton step whose
-// residual is kept exact, within 0.51 ulp of 1 / sqrt(q) (the reference's
-// float square root and reciprocal: within 1).  gamma: the same in FP64.
+// (float)(1 / E) of particles.cpp:247-252 for log-spaced bins, E = sqrtf(q) or
+// sqrt(1 + q), from an FP64 reciprocal square root y (hardware estimate, one
+// third-order step).  |u|: E is the root rounded to float, and one Newton step
+// from y gives 1 / E to about one double ulp.  The terms are the reference's
+// except within a few double ulps of a float rounding boundary (~1e-9 of them).
 template <bool FOURVEL>
 __device__ __forceinline__ float energy_term(float q) {
   if (!(q >= 0x1p-126f && q < 0x1p127f)) {
@@ -188,16 +189,13 @@ __device__ __forceinline__ float energy_term(float q) {
     const double e = FOURVEL ? static_cast<double>(sqrtf(q)) : sqrt(1.0 + static_cast<double>(q));
     return static_cast<float>(1.0 / e);
   }
-  if (FOURVEL) {
-    const float y = __builtin_amdgcn_rsqf(q);
-    const float h = q * y;
-    const float r = fmaf(-h, y, 1.0f) - fmaf(q, y, -h) * y;  // 1 - q y^2
-    return fmaf(0.5f * y, r, y);
-  }
-  const double d = 1.0 + static_cast<double>(q);
-  const double y = __builtin_amdgcn_rsq(d);
-  const double r = fma(-d * y, y, 1.0);
-  return static_cast<float>(fma(y * r, fma(r, 0.375, 0.5), y));
+  const double d = FOURVEL ? static_cast<double>(q) : 1.0 + static_cast<double>(q);
+  const double y0 = __builtin_amdgcn_rsq(d);
+  const double r = fma(-d * y0, y0, 1.0);
+  const double y = fma(y0 * r, fma(r, 0.375, 0.5), y0);
+  if (!FOURVEL) return static_cast<float>(y);
+  const double e = static_cast<double>(static_cast<float>(d * y));
+  return static_cast<float>(fma(y, fma(-e, y, 1.0), y));
 }
 
 struct HistParams {
@@ -229,8 +227,8 @@ typedef float float4u __attribute__((ext_vector_type(4), aligned(4)));
 
 // Each thread keeps two 16-byte loads per component in flight (8 particles); the
 // last n % 4 particles go one per thread.  COUNT: integer counts are kept (linear
-// bins sum ones, so their sums are the counts).  38 vector instructions a
-// particle (57 when the energy was formed); bound by memory latency and LDS
+// bins sum ones, so their sums are the counts).  37 vector instructions a
+// particle, 14 of them FP64 (57 when the energy was formed); bound by memory latency and LDS
 // atomics (counters: VALU 40%, LDS 45% of the cycles).  2^24 particles with the
 // momenta in HBM (201 MB, 39 us at the rate of a copy): 200 log bins 56.6 -> 55.5
 // us, 1000 bins 80 -> 64, linear bins 55 -> 49; 2^24 + 3 particles 60 -> 56.

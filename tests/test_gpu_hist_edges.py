@@ -40,3 +40,25 @@ def test_every_edge(orc, lo, hi, nb, fourvel):
     h = h.double().cpu().numpy()
     assert np.array_equal(np.isfinite(h), good)
     assert np.all(np.abs(h[good] - hd[good]) <= 1e-6 * np.abs(hd[good]))
+
+
+@pytest.mark.parametrize("fourvel", [True, False])
+def test_terms_are_the_reference_s(fourvel):
+    """One particle a bin: each sum is the reference's float term (float)(1 / E), E = sqrtf(|u|^2) or
+    sqrt(1 + |u|^2), bit for bit (an FP64 reciprocal of E to about an ulp rounds to the same float except
+    within that ulp of a rounding boundary: 1e-9 of the terms)."""
+    nb = 2000
+    for lo, hi in ((0.2, 3.0), (5.0, 9.0), (-8.0, -6.0) if fourvel else (0.2, 1.0)):
+        bins = np.logspace(lo, hi, nb).astype(np.float32)
+        plan = T.HistPlan(bins, True)
+        for seed in range(10):
+            f = np.random.default_rng(seed).uniform(0.2, 0.8, nb - 1)
+            e = 10.0 ** (lo + (hi - lo) * (np.arange(nb - 1) + f) / (nb - 1))
+            x = np.sqrt(e * e - (0.0 if fourvel else 1.0)).astype(np.float32)
+            u = np.zeros((3, nb - 1), np.float32)
+            u[seed % 3] = x
+            h, c = T.energy_hist(plan, torch.from_numpy(u).cuda(), fourvel)
+            assert torch.all(c[:-1] == 1)
+            q = x * x
+            energy = np.sqrt(q).astype(np.float64) if fourvel else np.sqrt(1.0 + q.astype(np.float64))
+            assert np.array_equal(h.cpu().numpy()[:-1], (1.0 / energy).astype(np.float32))
