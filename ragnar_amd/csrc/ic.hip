@@ -5,10 +5,8 @@
 // For every output energy e_ic and every (gamma, e_soft) pair the reference adds
 //     f_g (f_s / e_s) e_ic^2 KN(Gamma, q) / g      (/ g^2 for linear gamma bins)
 // with Gamma = 4 g e_s, q = (e_ic / g) / (Gamma (1 - e_ic / g)), skipped above
-// the kinematic limit e_ic > g Gamma / (1 + Gamma).  Each term is computed here in
-// the reference's float arithmetic and operation order (KN's second part is
-// double in the reference: its 0.5 literal promotes it), and the terms of a bin
-// are summed in FP64 in a fixed order, so results are reproducible bit for bit.
+// the kinematic limit e_ic > g Gamma / (1 + Gamma).  The terms of a bin are summed
+// in FP64 in a fixed order, so results are reproducible bit for bit.
 //
 // Layout: one workgroup per (output bin, chunk of gamma bins), enough of them
 // to fill the device; its threads take the chunk's (gamma, e_soft) pairs in
@@ -22,10 +20,15 @@
 // gamma bin's, and the kinematic limit is q = 1: no divide is left in the loop.
 // Pairs where rounding could decide differently (q within 2e-6 / (1 - x) of 1:
 // the reference's limit is good to 2.4e-7 / (1 - x)) and operands outside the
-// ranges below take the reference's own operations.
-// Per call, before and after: 200^3 27.6 and 15.5 us (of it the kernel 23.4 and
+// ranges below take the reference's own operations (KN's second part is double
+// there: its 0.5 literal promotes it).
+// q, KN and the quotient by g are FP64, which issues at the rate of FP32 here and
+// takes fewer instructions than float factors with their conversions; the
+// logarithm is the hardware's float log2.  Error of a term against 64 bits (rms,
+// q < 0.5): 5.7e-8 .. 1.0e-7, of the reference's operations 6.7e-8 .. 1.2e-7.
+// Per call, before and after: 200^3 27.6 and 15.3 us (of it the kernel 23.4 and
 // 11: the loop's 125000 wave steps take 4.4, loading, staging and the reduction
-// the rest), 500^3 243 and 75, 1000^3 1596 and 452 us (71 clocks a step of 64 pairs).
+// the rest), 500^3 235 and 71, 1000^3 1589 and 439 us (69 clocks a step of 64 pairs).
 #include <algorithm>
 #include <cmath>
 
@@ -68,12 +71,11 @@ __device__ __forceinline__ double ic_rcp(double x) {
 }
 
 struct __align__(16) IcGamma {
-  float c;       // x / (4 g (1 - x)); NaN: outside the ranges, every pair by ic_term
+  double c;      // x / (4 g (1 - x)); NaN: outside the ranges, every pair by ic_term
+  double h1;     // 1 + (Gamma q)^2 / (1 + Gamma q) / 2
+  double ig;     // 1 / g, or 1 / g^2 for linear gamma bins
   float lo, hi;  // below lo (from kIcMinQ): a term; above hi: none; between: ic_term
   float f;
-  double h;  // (Gamma q)^2 / (1 + Gamma q) / 2
-  float ig;  // 1 / g, or 1 / g^2 for linear gamma bins
-  float g;
 };
 constexpr float kIcMinQ = 1e-30f;
 
@@ -81,16 +83,15 @@ __device__ __forceinline__ IcGamma ic_gamma(float g, float f, float e_ic, int g_
   IcGamma o;
   const float x = e_ic / g, one_x = 1.0f - x;
   const bool ok = g >= 1e-6f && g <= 1e12f && x >= 1e-20f && fabsf(one_x) >= 4e-6f && x < INFINITY;
-  const double gq = static_cast<double>(x) * ic_rcp(one_x);
+  const double gq = static_cast<double>(x) * ic_rcp(one_x), rg = ic_rcp(g);
   // past the limit for every e_soft where x > 1
-  o.c = !ok ? NAN : one_x > 0.0f ? static_cast<float>(0.25 * gq * ic_rcp(g)) : INFINITY;
+  o.c = !ok ? NAN : one_x > 0.0f ? 0.25 * gq * rg : INFINITY;
   const float margin = 2e-6f * __builtin_amdgcn_rcpf(fabsf(one_x));
   o.lo = 1.0f - margin;
   o.hi = 1.0f + margin;
   o.f = f;
-  o.h = 0.5 * gq * gq * ic_rcp(1.0 + gq);
-  o.ig = 1.0f / (g_log ? g : g * g);
-  o.g = g;
+  o.h1 = fma(0.5 * gq * gq, ic_rcp(1.0 + gq), 1.0);
+  o.ig = g_log ? rg : rg * rg;
   return o;
 }
 
@@ -111,25 +112,25 @@ __global__ void __launch_bounds__(kIcThreads) ic_kernel(const float* __restrict_
                                                         double* __restrict__ partial, float* __restrict__ out) {
   __shared__ double red[kIcThreads];
   __shared__ IcGamma s_g[kIcGamma];
-  __shared__ float s_r[kIcSoft], s_f[kIcSoft];  // 1 / e_soft (NaN: outside the range), f_s / e_soft
+  __shared__ double s_r[kIcSoft];  // 1 / e_soft (NaN: outside the range)
+  __shared__ float s_f[kIcSoft];   // f_s / e_soft
   const int e = blockIdx.x, neic = gridDim.x, tid = threadIdx.x;
   const float e_ic = eic[e];
   const int g0 = blockIdx.y * gper, g1 = min(ng, g0 + gper);
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   double acc = 0.0;
-  auto pair = [&](const IcGamma& G, float r, float fs_es, int si) {
-    const float q = G.c * r;
-    if (q > G.hi) return;
-    float term;
-    if (q <= G.lo && q >= kIcMinQ) {
-      const float first = 2.0f * q * (__builtin_amdgcn_logf(q) * 0.6931471805599453f);
-      const float kn = static_cast<float>(fma(static_cast<double>(1.0f - q),
-                                              static_cast<double>(1.0f + 2.0f * q) + G.h, static_cast<double>(first)));
-      term = G.f * fs_es * e_ic * e_ic * kn * G.ig;
+  // KN = 2 q ln q + (1 - q) (1 + 2 q + h)
+  auto pair = [&](const IcGamma& G, int gi, double r, float fs_es, int si) {
+    const double q = G.c * r;
+    const float qf = static_cast<float>(q);
+    if (qf > G.hi) return;
+    if (qf <= G.lo && qf >= kIcMinQ) {
+      const double lg = static_cast<double>(__builtin_amdgcn_logf(qf));
+      const double kn = fma(q * (2.0 * 0.69314718055994530942), lg, (1.0 - q) * fma(q, 2.0, G.h1));
+      acc = fma(static_cast<double>(G.f * fs_es * e_ic * e_ic), kn * G.ig, acc);
     } else {
-      term = ic_term(G.g, G.f, es[si], fs_es, e_ic, g_log);
+      acc += static_cast<double>(ic_term(g[gi], G.f, es[si], fs_es, e_ic, g_log));
     }
-    acc += static_cast<double>(term);
   };
   for (int ss = 0; ss < nes; ss += kIcSoft) {
     const int ms = min(kIcSoft, nes - ss);
@@ -154,7 +155,7 @@ __global__ void __launch_bounds__(kIcThreads) ic_kernel(const float* __restrict_
 #pragma unroll
         for (int j = 0; j < kIcSoft / kIcThreads; ++j) {
           if (tid + j * kIcThreads < ms) {
-            s_r[tid + j * kIcThreads] = soft[j] >= 1e-15f && soft[j] <= 1e15f ? 1.0f / soft[j] : NAN;
+            s_r[tid + j * kIcThreads] = soft[j] >= 1e-15f && soft[j] <= 1e15f ? ic_rcp(soft[j]) : NAN;
             s_f[tid + j * kIcThreads] = fsoft[j] / soft[j];
           }
         }
@@ -162,13 +163,14 @@ __global__ void __launch_bounds__(kIcThreads) ic_kernel(const float* __restrict_
       __syncthreads();
       if constexpr (ROWS) {
         for (int si = lane; si < ms; si += 64) {
-          const float r = s_r[si], fs_es = s_f[si];
-          for (int i = wave; i < mg; i += kIcThreads / 64) pair(s_g[i], r, fs_es, ss + si);
+          const double r = s_r[si];
+          const float fs_es = s_f[si];
+          for (int i = wave; i < mg; i += kIcThreads / 64) pair(s_g[i], gs + i, r, fs_es, ss + si);
         }
       } else {
         int i = tid / ms, si = tid % ms;
         while (i < mg) {
-          pair(s_g[i], s_r[si], s_f[si], ss + si);
+          pair(s_g[i], gs + i, s_r[si], s_f[si], ss + si);
           i += di;
           si += ds;
           if (si >= ms) {
