@@ -567,8 +567,8 @@ static_assert(kBinnedMaxNK <= 65535, "list entries keep the bucket in 16 bits");
 // the cycles).  Block clocks there: 5 us set-up, 76 us stream (5.3 TB/s), 3 us
 // window, 28 us list (18% of the sources); the call 159 -> 122 us.  At 10^6
 // particles 6 us stream, 19 us the rest; 53 us (pair by pair) -> 33 us.
-//   1  The buckets of the first kStream particles pick the window: the `rows`
-//      consecutive buckets holding most of them.
+//   1  The buckets of kStream particles spread over the block's share pick the
+//      window: the `rows` consecutive buckets holding most of them.
 //   2  Every particle's (k, W, phi) adds W and W phi to its sub-cell of the
 //      window's rows in LDS (ds_add_f64), or goes to the block's list.
 //   3  Each wave takes rows of the window: prefix sums over the sub-cells and
@@ -601,13 +601,21 @@ __global__ void __launch_bounds__(kStream) binned_stream(ParticlesDev D, unsigne
   __shared__ unsigned s_part[kWaves], s_count;
   __shared__ int s_w0;
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_uniform(tid >> 6);
-  const unsigned stride = gridDim.x * kStream;
-  unsigned p = blockIdx.x * kStream + tid;
+  // The block's share is every gridDim.x-th tile of kStream particles.  Its waves
+  // start with tiles spread evenly over the share, so that the first particles
+  // are a sample of a store in any order (species after species, sorted by
+  // energy), and then take the others in turn: step s is tile s - 1 up to the
+  // wave's first tile, s beyond it.
+  const unsigned stride = gridDim.x * kStream, p0 = blockIdx.x * kStream + tid;
+  const unsigned tiles = (n - blockIdx.x * kStream + stride - 1) / stride;
+  const unsigned first_tile = wave * tiles / kWaves;
+  unsigned p = p0 + first_tile * stride, step = 0;
+  auto at_step = [&](unsigned s) { return p0 + (s > first_tile ? s : s - 1) * stride; };  // from s = 1
   // four particles per thread in flight; past the end, the last one again
   auto load = [&](unsigned i) { return load_particle32<NT>(D, min(i, n - 1)); };
   RawParticle ring[4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) ring[i] = load(p + i * stride);
+  for (unsigned i = 0; i < 4; ++i) ring[i] = load(i ? at_step(i) : p);
   for (int i = tid; i < S.rows * pitch; i += kStream) area[i] = 0.0;
   for (int i = tid; i < NK; i += kStream) {
     hist[i] = 0u;
@@ -638,8 +646,8 @@ __global__ void __launch_bounds__(kStream) binned_stream(ParticlesDev D, unsigne
   bool in;
   auto next = [&](RawParticle& r) {
     in = stream_source<HAS_E>(r, P, l2, src) && p < n;
-    r = load(p + 4 * stride);
-    p += stride;
+    r = load(at_step(step + 4));
+    p = at_step(++step);
   };
   next(ring[0]);
   int w0 = 0;
@@ -706,7 +714,7 @@ __global__ void __launch_bounds__(kStream) binned_stream(ParticlesDev D, unsigne
   auto add_window = [&]() {
     for (int i = wave; i < rows; i += kWaves) add_bucket<Q>(L, area + i * pitch, M, P.kmin + w0 + i, node, P.T, lane);
   };
-  for (unsigned base = blockIdx.x * kStream; base < n; base += 4 * stride) {
+  for (unsigned done_tiles = 0; done_tiles < tiles; done_tiles += 4) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       if (in) {

@@ -12,7 +12,10 @@ range.  The spectrum is that of the unscaled fields times the weight.
 
 Particles that the reference's float steps drop (a momentum whose square
 overflows, a chi that overflows or vanishes as a float) add nothing, as in the
-pair-by-pair form."""
+pair-by-pair form.
+
+Ordered stores: every particle counts once, whichever tiles a block's waves
+start with (one tile to many, whole and cut)."""
 import numpy as np
 import pytest
 import torch
@@ -87,3 +90,17 @@ def test_particles_outside_the_float_range():
         plan = T.SyncPlan(T.default_table(), bins, B0=b0, g_syn=g_syn)
         for method in ("direct", "binned"):
             assert not torch.any(T.sync_spectrum(plan, u, b * field, method=method)), (field, method)
+
+
+@pytest.mark.parametrize("n", [1, 1000, 1024 * 256, 1024 * 256 + 1, 1024 * 256 * 2 - 1, 1024 * 256 * 5 + 77, 6000001])
+@pytest.mark.parametrize("order", ["ascending", "descending", "cold first"])
+def test_ordered_stores(n, order):
+    r = torch.rand(n, generator=torch.Generator(device="cuda").manual_seed(n), device="cuda", dtype=torch.float64)
+    gamma = (1.0 + (1e3 ** -1.5 - 1.0) * r) ** (-1 / 1.5)
+    key = {"ascending": gamma, "descending": -gamma, "cold first": (gamma > 1.5).double()}[order]
+    u, b = _isotropic(gamma[torch.argsort(key)])
+    table = T.default_table()
+    plan = T.SyncPlan(table, np.logspace(-2, 6, 256).astype(np.float32))
+    got = T.sync_spectrum(plan, u, b, method="binned").double()
+    ref = _reference(plan, table, u, b, None, None)
+    assert torch.linalg.norm(got - ref) <= 1e-6 * torch.linalg.norm(ref)
