@@ -621,7 +621,7 @@ void launch_combine(const SyncPlan& plan, const double* partials, int pitch, int
 
 // Automatic choice between the direct and the factorised kernels from a cost
 // model measured on MI355X (constants below).  RAGNAR_SYNC_METHOD (direct | binned) overrides the automatic choice.
-int resolve_method(const SyncPlan& plan, size_t n, int method, bool adjoint) {
+int resolve_method(const SyncPlan& plan, const ParticlesDev& D, size_t n, int method, bool adjoint) {
   // the factorised kernels address particles with 32-bit byte offsets
   const bool binned_fits = plan.binned_ok && n < kBinnedMaxParticles;
   if (method == RGN_METHOD_AUTO) {
@@ -630,13 +630,16 @@ int resolve_method(const SyncPlan& plan, size_t n, int method, bool adjoint) {
       if (std::string(m) == "binned" && binned_fits) return RGN_METHOD_BINNED;
     }
     if (!binned_fits) return RGN_METHOD_DIRECT;
-    // Seconds per call, fitted on MI355X to 2^14 .. 2^24 particles of index
-    // -2.5 and -1.7 at 32 .. 512 bins.  The pair-by-pair kernels cost per
-    // particle by NB, the number of 64-bin blocks; the factorised ones a floor
-    // of fixed work, then a cost per particle that hardly depends on the bins.
-    // Forward at 256 bins, pair by pair against factorised: 2^18 22.5 / 29, 2^19
-    // 31.5 / 31, 2^20 48 / 34 us; at 512 bins 2^19 50 / 48 us.
-    static const double c_fwd[9] = {0, 21e-12, 21e-12, 26e-12, 27e-12, 31e-12, 34e-12, 44e-12, 53e-12};
+    // Seconds per call, fitted on MI355X around the lines to populations of index
+    // -2.9, -2.2 and -1.55 at 40 .. 512 bins, with and without E.  The pair-by-pair
+    // kernels cost per particle by NB, the number of 64-bin blocks; the factorised
+    // ones a floor of fixed work, then a cost per particle that hardly depends on
+    // the bins.  Forward, pair by pair against factorised, us without E, and with:
+    //    87 bins:  4e5 23 / 25.6 .. 28.3, 23 / 28.2 .. 30.5;  8e5 34 / 26 .. 30, 34 / 30 .. 34
+    //   256 bins:  4e5 27 / 29 .. 36, 27 / 31 .. 39;  5.6e5 32 / 30 .. 38, 32 / 33 .. 41;
+    //              8e5 41 / 30 .. 39, 41 / 35 .. 43
+    //   512 bins:  2.8e5 39 .. 43 / 46, 4e5 44 .. 49 / 47, 5.6e5 56 .. 64 / 48
+    static const double c_fwd[9] = {0, 27e-12, 29e-12, 31e-12, 33e-12, 39e-12, 48e-12, 56e-12, 65e-12};
     // Adjoint: between 1.5e5 and 3.3e5 particles the pair-by-pair form is up to 4 us
     // faster since it skips blocks, but where a particle's terms nearly cancel its
     // FP32 sums are further off (a log-residual loss at 2.7e5 particles and 149
@@ -644,11 +647,12 @@ int resolve_method(const SyncPlan& plan, size_t n, int method, bool adjoint) {
     // the two once met.
     static const double c_adj[9] = {0, 27e-12, 34e-12, 43e-12, 52e-12, 63e-12, 74e-12, 84e-12, 95e-12};
     const double nd = static_cast<double>(n);
+    const bool has_e = D.e[0] || D.e[1] || D.e[2];
     const int nbk = std::min(std::max(plan.NB, 1), 8);
-    const double t_direct = adjoint ? 25e-6 + nd * c_adj[nbk] : 18e-6 + nd * c_fwd[nbk];
+    const double t_direct = adjoint ? 25e-6 + nd * c_adj[nbk] : 9e-6 + 1.3e-6 * nbk + nd * c_fwd[nbk];
     const double t_fwd = !stream_form(plan) ? std::max(47e-6, 35e-6 + nd * 8.2e-12)
-                         : plan.M <= 128    ? 22e-6 + nd * 4.1e-12
-                                            : 28e-6 + nd * 5.7e-12;
+                         : plan.M <= 128    ? (has_e ? 28.5e-6 : 25.7e-6) + nd * 4.1e-12
+                                            : (has_e ? 28.0e-6 : 25.2e-6) + plan.M * 0.024e-6 + nd * 5.5e-12;
     const double t_binned = adjoint ? std::max(33e-6, 28e-6 + nd * 13.5e-12) : t_fwd;
     return t_binned < t_direct ? RGN_METHOD_BINNED : RGN_METHOD_DIRECT;
   }
@@ -710,7 +714,7 @@ int rgn_sync_spectrum_method(const rgn_sync_plan* plan, const float* const d_u[3
     RGN_REQUIRE(d_out != nullptr, RGN_ERR_INVALID, "null output");
     const ParticlesDev D = make_particles_checked(d_u, d_e, d_b, d_w, n);
     ScratchUse order(as_stream(stream));
-    if (resolve_method(plan->p, n, method, false) == RGN_METHOD_BINNED) {
+    if (resolve_method(plan->p, D, n, method, false) == RGN_METHOD_BINNED) {
       sync_forward_binned(plan->p, D, n, d_out, as_stream(stream));
     } else {
       // 16 blocks per CU measured fastest on MI355X (2^24 x 256: 0.68 ms vs 0.74 at 4)
@@ -743,7 +747,7 @@ int rgn_sync_adjoint_method(const rgn_sync_plan* plan, const float* const d_u[3]
     RGN_REQUIRE(d_gbar != nullptr, RGN_ERR_INVALID, "null upstream gradient");
     const ParticlesDev D = make_particles_checked(d_u, d_e, d_b, d_w, n);
     ScratchUse order(as_stream(stream));
-    if (resolve_method(plan->p, n, method, true) == RGN_METHOD_BINNED) {
+    if (resolve_method(plan->p, D, n, method, true) == RGN_METHOD_BINNED) {
       sync_adjoint_binned(plan->p, D, n, d_gbar, d_gw, d_gu, d_gb, d_ge, as_stream(stream));
       return;
     }

@@ -95,7 +95,7 @@ void sync_adjoint_binned(const SyncPlan& plan, const ParticlesDev& D, size_t n, 
                          float* gw, float* const gu[3], float* const gb[3], float* const ge[3],
                          hipStream_t st);
 bool stream_form(const SyncPlan& plan);  // which factorised forward a plan takes
-int resolve_method(const SyncPlan& plan, size_t n, int method, bool adjoint);
+int resolve_method(const SyncPlan& plan, const ParticlesDev& D, size_t n, int method, bool adjoint);
 
 PlanDev device_view(const SyncPlan& plan);
 size_t forward_smem(const SyncPlan& plan);
