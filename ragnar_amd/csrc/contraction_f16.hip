@@ -654,37 +654,64 @@ struct Tile {
 // The 64 x 256 tile does the least work per product and is the one that keeps the
 // matrix cores busy, but a call with few of them leaves CUs idle through their
 // serial loop over g (3001 x 300 x 200 is 47 workgroups), and 256 columns waste
-// half of the last one where the bins end in its first half.  Measured, us per
-// call (rows given, split-BF16; generated), tiles 64 x 256, 32 x 256, 32 x 128:
-//     3001 x 300 x 200:   24.0 19.8 17.3;   34.4 25.7 21.8
-//     9000 x 512 x 512:   47.4 42.9 37.6;   50.8 43.3 49.6
-//    12000 x 512 x 512:   47.2 43.2 48.1;   51.3 46.5 57.1
-//    16384 x 512 x 512:   51.1 54.2 56.8;   55.4 59.0 72.4
-//    65536 x 512 x 512:  175.9 194.2 198.8; 188.6 200.8 255.9
-//    65536 x 512 x 128:   83.5 93.3 59.5;   89.9 96.1 73.1
-//    65536 x 300 x 300:  110.8 125.4 101.0; 138.8 140.3 133.6
-// So: 32 x 128 while five of them a CU hold the batch (one where rows are
-// generated: each column tile generates its rows again) and wherever 128 columns
-// come out odd; 32 x 256 while three a CU do.  A CU with one or two workgroups
-// waits for its K fragments in L2, so the smallest batches of given rows take
-// them four steps ahead (3001 x 512 x 512, FP16 24.7 -> 18.7 us, BF16 23.6 -> 21.2;
-// 3001 x 300 x 200, 16.8 -> 16.4); with more of them the registers cost more waves
-// (12000 x 512 x 512: 34.0 against 39.6 us), and generated rows gain nothing.
-template <bool GEN, class Launch>
+// half of the last one where the bins end in its first half.  32 x 128 is the
+// other end; where rows are generated, each column tile generates its rows again.
+// A CU with one or two workgroups waits for its K fragments in L2: the smallest
+// batches of given rows take them four steps ahead (DEEP; with more of them the
+// registers cost more waves); rows read a float at a time (LOAD 0) want few column
+// tiles, each of which reads them again.  The lines, by products (3 and 1: split FP16, 6:
+// split BF16) and by how rows are read (LOAD 2: whole 64-g blocks), lie where every
+// tile was timed at 14 batch sizes and fourteen shapes.  Us per call, 64 x 256, 32 x 256,
+// 32 x 128 (DEEP):
+//    3 products   3001 x 300 x 200:  24.4 20.5 17.4 (17.4)    6000 x 512 x 512:  27.3 25.9 26.8 (24.4)
+//                 8000 x 300 x 400:  24.5 22.8 21.5          12000 x 512 x 512:  33.0 33.3 37.5
+//                65536 x 512 x 128:  56.9      51.8          65536 x 512 x 384: 110.8 127.5 114.9
+//                65536 x 300 x 300:  91.4 84.9 78.9          20000 x 449 x 470:  75.2 64.8 85.4
+//                14000 x 255 x 500:  34.8 39.3 45.4
+//    1 product    8000 x 512 x 512:  24.0 32.0 23.0 (19.6)   12000 x 512 x 512:  24.3 34.0 28.7 (31.1)
+//                12000 x 300 x 400:  21.0 19.7 27.7          65536 x 300 x 300:  76.5 60.0 54.8
+//    6 products   3001 x 300 x 200:  24.2 19.4 18.1 (17.5)   10000 x 512 x 512:  47.3 43.7 41.3
+//                12000 x 512 x 512:  47.6 43.8 48.3          65536 x 512 x 384: 158.0 189.4 152.2
+//                 8000 x 449 x 470:  42.3 39.5 44.9          32768 x 333 x 256:  48.3 51.2 57.5
+//    generated, 3 4096 x 512 x 512:  31.4 26.4 27.9          12000 x 512 x 512:  41.5 37.5 49.4
+//                32768 x 512 x 384:  72.4 79.0 88.7          32768 x 300 x 300:  67.3 59.9 64.7
+//                14000 x 300 x 300:  37.2 39.3 38.4          65536 x 512 x 128:  70.7      61.4
+template <int NPROD, bool GEN, int LOAD, class Launch>
 void launch_tiles(size_t nd, int nb, Launch launch) {
   auto tiles = [&](int rt, int ct) { return ceil_div(nd, 32 * rt) * ceil_div(nb, 128 * ct); };
   auto with = [&](auto t) {
     launch(t, static_cast<unsigned>(tiles(t.RT, t.CT)), static_cast<int>(ceil_div(nb, 128 * t.CT)));
   };
-  const size_t cus = num_cus();
-  if (!GEN && tiles(1, 1) <= cus + cus / 2) {
-    with(Tile<1, 1, !GEN>{});
-  } else if (ceil_div(nb, 128) % 2 == 1 || tiles(1, 1) <= (GEN ? 1 : 5) * cus) {
-    with(Tile<1, 1>{});
-  } else if (tiles(1, 2) <= 3 * cus) {
-    with(Tile<1, 2>{});
+  using Small = Tile<1, 1>;
+  using Wide = Tile<1, 2>;
+  using Large = Tile<2, 2>;
+  const size_t cus = num_cus(), small = tiles(1, 1), wide = tiles(1, 2);
+  const bool one = nb <= 128, odd = ceil_div(nb, 128) % 2 == 1;  // columns of 128
+  const bool rounds = tiles(2, 2) > 2 * cus;  // the large tiles need a second round of two a CU
+  if constexpr (GEN) {
+    if (one || small <= cus) with(Small{});
+    else if (wide <= 3 * cus) with(Wide{});
+    else if (odd && LOAD != 2 && rounds) with(Small{});
+    else with(Large{});
+  } else if (2 * small <= (NPROD == 1 && LOAD > 0 ? 8 : 3) * cus) {
+    with(Tile<1, 1, true>{});
+  } else if (one) {
+    with(Small{});
+  } else if constexpr (LOAD == 0) {
+    if (wide <= 3 * cus || (NPROD != 6 && rounds)) with(Wide{});
+    else with(Large{});
+  } else if constexpr (NPROD == 6) {
+    if (odd || small <= 5 * cus) with(Small{});
+    else if (wide <= 3 * cus) with(Wide{});
+    else with(Large{});
+  } else if constexpr (NPROD == 3) {
+    if (LOAD == 1 && (odd || small <= 4 * cus)) with(Small{});
+    else if (2 * wide <= (LOAD == 2 ? 5 : 6) * cus) with(Wide{});
+    else with(Large{});
   } else {
-    with(Tile<2, 2>{});
+    if (LOAD == 1 && wide <= 3 * cus) with(Wide{});
+    else if (LOAD == 1 && odd && rounds) with(Small{});
+    else with(Large{});
   }
 }
 
@@ -712,7 +739,7 @@ void contraction_f16(const SyncPlan& plan, const float* d_gbeta, int ng, int dis
   const int nd_i = static_cast<int>(nd);
   const int load = vec ? (ng % kKB == 0 ? 2 : 1) : 0;
 #define RGN_CONTRACT(P_, L_)                                                                                        \
-  launch_tiles<false>(nd, nb, [&](auto t, unsigned grid, int ntn) {                                                      \
+  launch_tiles<P_, false, L_>(nd, nb, [&](auto t, unsigned grid, int ntn) {                                         \
     mfma_contract2<P_, L_, t.RT, t.CT, t.DEEP><<<grid, kThreads2, 0, st>>>(d_f, nd_i, ng, Bh, Bl, rB, nb, nbp, nkb, ntn, d_out); \
   })
 #define RGN_CONTRACT_P(P_)                   \
@@ -751,7 +778,7 @@ void contraction_f16_plaw(const SyncPlan& plan, const float* d_gbeta, int ng, in
   const size_t gsmem = 3 * sizeof(double) * static_cast<size_t>(ng);
   const int nd_i = static_cast<int>(nd);
 #define RGN_CONTRACT_GEN(P_, L_)                                                                            \
-  launch_tiles<true>(nd, nb, [&](auto t, unsigned grid, int ntn) {                                              \
+  launch_tiles<P_, true, L_>(nd, nb, [&](auto t, unsigned grid, int ntn) {                                 \
     mfma_contract2<P_, L_, t.RT, t.CT, t.DEEP, true><<<grid, kThreads2, gsmem, st>>>(nullptr, nd_i, ng, Bh, Bl, rB, nb, \
                                                                              nbp, nkb, ntn, d_out, gen);        \
   })
@@ -791,7 +818,7 @@ void contraction_bf16(const SyncPlan& plan, const float* d_gbeta, int ng, int di
   const bool vec = ng % 4 == 0 && reinterpret_cast<uintptr_t>(d_f) % 16 == 0;
   const size_t gsmem = 3 * sizeof(double) * static_cast<size_t>(ng);
 #define RGN_CONTRACT_BF16(L_, G_)                                                                                     \
-  launch_tiles<G_>(nd, nb, [&](auto t, unsigned grid, int ntn) {                                                     \
+  launch_tiles<6, G_, L_>(nd, nb, [&](auto t, unsigned grid, int ntn) {                                         \
     mfma_contract_bf16<L_, t.RT, t.CT, t.DEEP, G_><<<grid, kThreads2, G_ ? gsmem : 0, st>>>(                         \
       G_ ? nullptr : d_f, nd_i, ng, Bh, Bm, Bl, nb, nbp, nkb, ntn, d_out, gen);                                      \
   })
