@@ -197,11 +197,14 @@ __global__ void __launch_bounds__(kThreads) forward_kernel(SourceFn fn, size_t n
 // waves sums them over its lanes for one bin, so that the bins spread over the
 // device and nothing is combined afterwards.  Bound by latency: 200 sources x
 // 200 bins in one block of the forward kernel (each wave a share of the sources,
-// all bins) took 7.0 us, this 3.3.  Every block makes all the sources, which pays
-// up to about 5000 of them: calls on 4096 sources 13.8 (512 bins: 17.5) -> 11.0
-// us, on 8192 13.8 (17.5) -> 20, so more go to the forward kernel.
+// all bins) took 7.3 us, this 2.9.  Every block makes all the sources, 2.2 us a
+// thousand, while the forward kernel's blocks share them: the two meet at about
+// 2000 sources for 64 bins (6.4 us on the device), 2200 for 128 (6.9), 3400
+// for 256 (9.4) and beyond 4096 from 384 bins on (11.1 and 13).
 constexpr int kDistThreads = 512;
 constexpr int kDistMax = 4096;
+
+int dist_max(const SyncPlan& plan) { return std::min(kDistMax, 1500 + 450 * plan.NB); }
 
 __global__ void __launch_bounds__(kDistThreads) dist_kernel(DistSourceFn fn, int ng, PlanDev P,
                                                             float* __restrict__ out) {
@@ -824,7 +827,7 @@ int rgn_sync_fromdist(const rgn_sync_plan* plan, const float* d_gbeta, const flo
     RGN_REQUIRE(ng >= 0, RGN_ERR_INVALID, "negative distribution size");
     const SyncPlan& p = plan->p;
     hipStream_t st = as_stream(stream);
-    if (ng <= kDistMax) {  // no scratch, so no order with other calls
+    if (ng <= dist_max(p)) {  // no scratch, so no order with other calls
       const unsigned blocks = static_cast<unsigned>(ceil_div(p.nbins, kDistThreads / 64));
       const size_t smem = kDistThreads * sizeof(float4) + p.TP * sizeof(float2);
       dist_kernel<<<blocks, kDistThreads, smem, st>>>(DistSourceFn{d_gbeta, d_f, dist_log}, ng, device_view(p), d_out);
