@@ -116,6 +116,7 @@ float first_reaching(double target, bool fourvel) {
   const float inf = std::numeric_limits<float>::infinity();
   if (!(target == target)) return std::numeric_limits<float>::quiet_NaN();
   if (energy_of(0.0f, fourvel) >= target) return 0.0f;
+  if (!(energy_of(std::numeric_limits<float>::max(), fourvel) >= target)) return inf;
   // a guess within a few floats, then a step at a time
   float q = static_cast<float>(std::min(target * target - (fourvel ? 0.0 : 1.0), 3e38));
   q = std::max(q, std::numeric_limits<float>::denorm_min());
