@@ -125,7 +125,7 @@ int rgn_sync_adjoint(const rgn_sync_plan* plan, const float* const d_u[3],
  * ~independent of the bin count.  RGN_METHOD_AUTO picks the cheaper one from a
  * measured cost model (forward: binned from ~6.2e5 particles at 256 bins; env
  * RAGNAR_SYNC_METHOD=direct|binned overrides).  Binned needs fewer than 2^29
- * particles, at most 1024 distinct fractional bin offsets and a bin range of
+ * particles, at most 1024 bins of positive energy and a bin range of
  * at most 3072 table units (RGN_ERR_UNSUPPORTED otherwise; AUTO then runs
  * direct).  Same results to FP32/FP64 rounding (no reference counterpart). */
 enum { RGN_METHOD_AUTO = 0, RGN_METHOD_DIRECT = 1, RGN_METHOD_BINNED = 2 };

@@ -5,7 +5,7 @@
 // A_e = a_e + alpha_e.  Then t lies on segment m = a_e - k when phi <= alpha_e
 // and on segment m - 1 otherwise, and on segment s
 //     F = C_s(e, k) - sigma_s * phi,   C_s = y_s + (A_e - k - tau_s) sigma_s.
-// The sorted distinct alpha_e cut [0, 1) into M + 1 sub-cells; a source in
+// The sorted alpha_e, one per live bin, cut [0, 1) into M + 1 sub-cells; a source in
 // sub-cell j lies left of alpha_e exactly when j <= r_e (the rank of alpha_e).
 // So every bin needs, per k, only the prefix sums over sub-cells of
 //     m0 = sum W   and   m1 = sum W phi,
@@ -613,13 +613,12 @@ __global__ void __launch_bounds__(kStream) binned_stream(ParticlesDev D, unsigne
   // The block's share is every gridDim.x-th tile of kStream particles.  Its waves
   // start with tiles spread evenly over the share, so that the first particles
   // are a sample of a store in any order (species after species, sorted by
-  // energy), and then take the others in turn: step s is tile s - 1 up to the
-  // wave's first tile, s beyond it.
+  // energy); step s is then tile s, and tile 0 takes the place of the wave's first.
   const unsigned stride = gridDim.x * kStream, p0 = blockIdx.x * kStream + tid;
   const unsigned tiles = (n - blockIdx.x * kStream + stride - 1) / stride;
   const unsigned first_tile = wave * tiles / kWaves;
   unsigned p = p0 + first_tile * stride, step = 0;
-  auto at_step = [&](unsigned s) { return p0 + (s > first_tile ? s : s - 1) * stride; };  // from s = 1
+  auto at_step = [&](unsigned s) { return p0 + (s == first_tile ? 0 : s) * stride; };  // from s = 1
   // four particles per thread in flight; past the end, the last one again
   auto load = [&](unsigned i) { return load_particle32<NT>(D, min(i, n - 1)); };
   RawParticle ring[4];

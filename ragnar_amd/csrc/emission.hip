@@ -662,8 +662,8 @@ int resolve_method(const SyncPlan& plan, const ParticlesDev& D, size_t n, int me
   RGN_REQUIRE(method == RGN_METHOD_DIRECT || method == RGN_METHOD_BINNED, RGN_ERR_INVALID,
               "unknown method");
   RGN_REQUIRE(method != RGN_METHOD_BINNED || binned_fits, RGN_ERR_UNSUPPORTED,
-              "the binned method needs fewer than 2^29 particles, at most 1024 distinct bin "
-              "offsets and a bin range of at most 3072 table units");
+              "the binned method needs fewer than 2^29 particles, at most 1024 live bins "
+              "and a bin range of at most 3072 table units");
   return method;
 }
 

@@ -79,7 +79,7 @@ constexpr size_t kBinnedMaxParticles = size_t{1} << 29;  // 32-bit byte offsets 
 struct BinInfo {
   double A;   // A_e
   int a;      // floor(A_e)
-  int r;      // index of alpha_e in the sorted distinct list; -1 for dead bins
+  int r;      // rank of the bin's alpha_e in the sorted list (equal ones in bin order); -1 for dead bins
 };
 
 // Per table segment s (nodes s, s + 1 at their true coordinates tau):

@@ -201,10 +201,11 @@ __device__ __forceinline__ double sqrt_nr(double x) {
   return fma(g, r, g);
 }
 
-// The OmegaSync terms to about one ulp per operation, for the adjoint's
-// gradients (which need no correct rounding): reciprocal products instead of
-// divisions, refined square roots.  A particle's e_peak may differ from the
-// reference's in the last float bit; the forward kernels use omega_terms.
+// The OmegaSync terms to about one ulp per operation, for the factorised
+// adjoint's gradients and the factorised passes beyond 256 bins (which need no
+// correct rounding): reciprocal products instead of divisions, refined square
+// roots.  A particle's e_peak may differ from the reference's in the last float
+// bit; the pair-by-pair kernels use omega_terms.
 template <bool HAS_E = true>
 __device__ __forceinline__ OmegaTerms omega_terms_approx(const RawParticle& r, const EmitConst& C) {
   OmegaTerms o;
@@ -529,17 +530,6 @@ template <int CTRL, int ROW_MASK = 0xf>
 __device__ __forceinline__ float dpp_f(float v) {
   return __builtin_bit_cast(
     float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, ROW_MASK, 0xf, false));
-}
-
-// Sum over the 64 lanes of a wave; the total lands in lane 63.
-__device__ __forceinline__ float wave_sum_to_lane63(float v) {
-  v += dpp_f<kDppQuadPerm1032>(v);
-  v += dpp_f<kDppQuadPerm2301>(v);
-  v += dpp_f<kDppRowHalfMirror>(v);
-  v += dpp_f<kDppRowMirror>(v);
-  v += dpp_f<kDppRowBcast15, 0xa>(v);
-  v += dpp_f<kDppRowBcast31, 0xc>(v);
-  return v;
 }
 
 // v moved by a DPP control (lanes without a source, and rows outside ROW_MASK,
