@@ -574,8 +574,8 @@ static_assert(kBinnedMaxNK <= 65535, "list entries keep the bucket in 16 bits");
 // five, no sorted copy of the sources; bound by the loads and by vector and LDS
 // issue together (counters at 2^24 particles x 256 bins: VALU 46%, LDS 36% of
 // the cycles).  Block clocks there: 5 us set-up, 76 us stream (5.3 TB/s), 3 us
-// window, 28 us list (18% of the sources); the call 159 -> 122 us.  At 10^6
-// particles 6 us stream, 19 us the rest; 53 us (pair by pair) -> 33 us.
+// window, 28 us list (18% of the sources); the call 159 -> 124 us.  At 10^6
+// particles 6 us stream, 19 us the rest; 53 us (pair by pair) -> 34 us.
 //   1  The buckets of kStream particles spread over the block's share pick the
 //      window: the `rows` consecutive buckets holding most of them.
 //   2  Every particle's (k, W, phi) adds W and W phi to its sub-cell of the
@@ -1603,11 +1603,13 @@ static StreamShape stream_shape(const SyncPlan& plan, int Q, size_t& smem) {
 // whose lines fit in its LDS), the passes above.  A row of M + 1 sub-cells
 // takes 16 (M + 1) bytes of LDS, so with more bins the window narrows and the
 // list grows.  Call times, stream against passes, p = -2.5 and -1.6:
-//   2^24 x 256:  122 and 159 against 160 and 163 us
-//   2^22 x 256:   50 and  59 against  66 and  68
-//   2^20 x 256:   33 and  42 against  46 and  48
+//   2^24 x 256:  125 and 160 against 160 and 161 us
+//   2^22 x 256:   50 and  60 against  65 and  65
+//   2^20 x 256:   34 and  41 against  47 and  47
 //   2^24 x 512:  201 and 263 against 174 and 174
 //   2^22 x 512:   84 and 106 against  67 and  66
+// A flatter population than these (p = -1.05) fills the list: 2^24 x 256 221
+// against 162, 2^22 71 against 65, 2^20 43 against 47.
 bool stream_form(const SyncPlan& plan) { return plan.M <= 256 && plan.T <= 1023; }
 
 void sync_forward_binned(const SyncPlan& plan, const ParticlesDev& D, size_t n, float* out, hipStream_t st) {

@@ -228,9 +228,9 @@ typedef float float4u __attribute__((ext_vector_type(4), aligned(4)));
 
 // Each thread keeps two 16-byte loads per component in flight (8 particles); the
 // last n % 4 particles go one per thread.  COUNT: integer counts are kept (linear
-// bins sum ones, so their sums are the counts).  37 vector instructions a
-// particle, 14 of them FP64 (57 when the energy was formed); bound by memory latency and LDS
-// atomics (counters: VALU 40%, LDS 45% of the cycles).  2^24 particles with the
+// bins sum ones, so their sums are the counts).  43 vector instructions a
+// particle, 14 of them FP64 (57 when the energy was formed); bound by memory
+// latency and LDS atomics (counters: VALU 40%, LDS 45% of the cycles).  2^24 particles with the
 // momenta in HBM (201 MB, 39 us at the rate of a copy): 200 log bins 56.6 -> 55.5
 // us, 1000 bins 80 -> 64, linear bins 55 -> 49; 2^24 + 3 particles 60 -> 56.
 template <bool FOURVEL, bool LOGB, bool COUNT, bool NEAR>
@@ -302,7 +302,7 @@ __global__ void __launch_bounds__(kThreads) hist_kernel(const float* __restrict_
 // No global atomics.  The partials are rows of bins: as columns, 8 bytes into
 // each of nb cache lines per block, the histogram kernel took 40.3 instead of
 // 37.6 us at 2^24 particles and 200 bins, and a call at 1000 bins 54.8 instead of
-// 42.1 (4e6 particles 34.1 and 21.5; 200 bins, other momenta each call, 55.1 and
+// 42.1 (4e6 particles 34.1 and 21.5; 200 bins, three stores in turn, 55.1 and
 // 49.2).
 constexpr int kCombineThreads = 1024;
 constexpr int kCombineRows = 16;

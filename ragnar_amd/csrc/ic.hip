@@ -13,7 +13,7 @@
 // turn, both staged in LDS; a fixed-order tree per block and, with more than one
 // chunk, a second pass adding the chunks in order.  No table or plan.
 //
-// The kernel is bound by its VALU work, so what depends on one operand only is
+// The kernel is bound by its VALU work and its LDS reads, so what depends on one operand only is
 // formed once per block.  With x = e_ic / g (the reference's float value)
 //     q = [x / (4 g (1 - x))] (1 / e_s),   Gamma q = x / (1 - x),
 // so a pair's q is one product, KN's quotient (Gamma q)^2 / (1 + Gamma q) is the
