@@ -14,7 +14,7 @@
 // chunk, a second pass adding the chunks in order.  No table or plan.
 //
 // The kernel is bound by its VALU work and its LDS reads, so what depends on one operand only is
-// formed once per block.  With x = e_ic / g (the reference's float value)
+// formed once per block.  With x = e_ic / g (from x = 1/2 on the reference's float)
 //     q = [x / (4 g (1 - x))] (1 / e_s),   Gamma q = x / (1 - x),
 // so a pair's q is one product, KN's quotient (Gamma q)^2 / (1 + Gamma q) is the
 // gamma bin's, and the kinematic limit is q = 1: no divide is left in the loop.
@@ -24,11 +24,12 @@
 // there: its 0.5 literal promotes it).
 // q, KN and the quotient by g are FP64, which issues at the rate of FP32 here and
 // takes fewer instructions than float factors with their conversions; the
-// logarithm is the hardware's float log2.  Error of a term against 64 bits (rms,
-// q < 0.5): 5.7e-8 .. 1.0e-7, of the reference's operations 6.7e-8 .. 1.2e-7.
-// Per call, before and after: 200^3 27.6 and 15.3 us (of it the kernel 23.4 and
+// logarithm is the hardware's float log2.  Error of a term against 64 bits (rms):
+// 5.7e-8 at q < 1e-2, 1.2e-7 at 0.5 .. 0.9, 5.2e-7 at 0.9 .. 0.99; of the reference's
+// operations 6.7e-8, 2.2e-7 and 1.5e-6.
+// Per call, before and after: 200^3 27.6 and 15.5 us (of it the kernel 23.4 and
 // 11: the loop's 125000 wave steps take 4.4, loading, staging and the reduction
-// the rest), 500^3 235 and 71, 1000^3 1589 and 439 us (69 clocks a step of 64 pairs).
+// the rest), 500^3 235 and 72, 1000^3 1595 and 457 us (72 clocks a step of 64 pairs).
 #include <algorithm>
 #include <cmath>
 
@@ -83,7 +84,10 @@ __device__ __forceinline__ IcGamma ic_gamma(float g, float f, float e_ic, int g_
   IcGamma o;
   const float x = e_ic / g, one_x = 1.0f - x;
   const bool ok = g >= 1e-6f && g <= 1e12f && x >= 1e-20f && fabsf(one_x) >= 4e-6f && x < INFINITY;
-  const double gq = static_cast<double>(x) * ic_rcp(one_x), rg = ic_rcp(g);
+  // x unrounded, but for x near 1, where its rounding decides 1 - x: the reference's
+  const double rg = ic_rcp(g);
+  const double xd = x < 0.5f ? static_cast<double>(e_ic) * rg : static_cast<double>(x);
+  const double gq = xd * ic_rcp(1.0 - xd);
   // past the limit for every e_soft where x > 1
   o.c = !ok ? NAN : one_x > 0.0f ? 0.25 * gq * rg : INFINITY;
   const float margin = 2e-6f * __builtin_amdgcn_rcpf(fabsf(one_x));
@@ -119,14 +123,19 @@ __global__ void __launch_bounds__(kIcThreads) ic_kernel(const float* __restrict_
   const int g0 = blockIdx.y * gper, g1 = min(ng, g0 + gper);
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   double acc = 0.0;
-  // KN = 2 q ln q + (1 - q) (1 + 2 q + h)
+  // KN = 2 q ln q + (1 - q) (1 + 2 q + h), of q rounded once to float: of one q in both
+  // parts, which cancel near q = 1.  The hardware's log2 rounds down, below q = 1/4 half
+  // an ulp on average, 4e-8 of it (0 .. 2e-8 beyond): the constant takes that off (error
+  // of 200^3 against 64 bits 5.5e-8 without, 4.0e-8 with it).
+  constexpr double kTwoLn2 = 2.0 * 0.69314718055994530942 * (1.0 - 4e-8);
   auto pair = [&](const IcGamma& G, int gi, double r, float fs_es, int si) {
-    const double q = G.c * r;
-    const float qf = static_cast<float>(q);
+    const float qf = static_cast<float>(G.c * r);
     if (qf > G.hi) return;
     if (qf <= G.lo && qf >= kIcMinQ) {
       const double lg = static_cast<double>(__builtin_amdgcn_logf(qf));
-      const double kn = fma(q * (2.0 * 0.69314718055994530942), lg, (1.0 - q) * fma(q, 2.0, G.h1));
+      const double q = static_cast<double>(qf);
+      const double rest = (1.0 - q) * fma(q, 2.0, G.h1);
+      const double kn = fma(q * kTwoLn2, lg, rest);
       acc = fma(static_cast<double>(G.f * fs_es * e_ic * e_ic), kn * G.ig, acc);
     } else {
       acc += static_cast<double>(ic_term(g[gi], G.f, es[si], fs_es, e_ic, g_log));
